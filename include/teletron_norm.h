@@ -152,6 +152,27 @@ int tt_rmsnorm_backward_strided(void *dx, void *dweight, const void *dout, const
 int tt_norm_copy_rows_strided(void *dst, const void *src, int64_t n0, int64_t n1, int64_t n2, int64_t ds0,
                               int64_t ds1, int64_t ds2, int64_t cols, int dtype, void *stream);
 
+/* The QK-norm call site as one kernel per direction (teletron/models/dit/dit_attention.py:149-214): `mixed` is the
+ * fused projection [B, S, H, 3 * cols] with q, k, v of a head side by side.
+ * Forward: q, k [B, H, S, cols] contiguous = RMSNorm of their slices (v needs no kernel: it is a view of mixed).  With
+ * rope_tokens > 0 (cols 128 only) the first rope_tokens tokens of q and k are then rotated as
+ * tt_rmsnorm_rope_forward_strided does; cos, sin are fp32 [rope_tokens, cols].
+ * Backward: dmixed [B, S, H, 3 * cols] is written whole from the gradients of q, k and v ([B, H, S, cols] contiguous;
+ * NULL for an output that was not used: its slice, and its dweight, are zero).  No row statistics are kept between
+ * the two: pass the forward call's eps.
+ * Heads of at most 64 16-byte pieces (512 two-byte / 256 four-byte columns): tt_qkv_rmsnorm_supported. */
+int tt_qkv_rmsnorm_supported(int64_t cols, int dtype);
+int tt_qkv_rmsnorm_forward(void *q, void *k, const void *mixed, const void *weight_q, const void *weight_k,
+                           const float *cos, const float *sin, int64_t rope_tokens,
+                           int64_t B, int64_t S, int64_t H, int64_t cols, double eps, int dtype, void *stream);
+size_t tt_qkv_rmsnorm_backward_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t cols, int dtype);
+int tt_qkv_rmsnorm_backward(void *dmixed, void *dweight_q, void *dweight_k,
+                            const void *dq, const void *dk, const void *dv,
+                            const void *mixed, const void *weight_q, const void *weight_k,
+                            const float *cos, const float *sin, int64_t rope_tokens,
+                            int64_t B, int64_t S, int64_t H, int64_t cols, double eps, int dtype,
+                            void *workspace, size_t workspace_bytes, void *stream);
+
 /* The strided QK-norm with the rotary embedding the attention caller applies right behind it
  * (teletron/models/dit/dit_attention.py:266-273 and :435-443: apply_rotary_emb(query, (freqs_cos,
  * freqs_sin)) on the [B, H, S, D] result of q_layernorm / k_layernorm, a separate read + write pass

@@ -32,7 +32,7 @@ ARCH = "gfx950"
 # compiler narrows fp16 chains to half arithmetic and then fuses across a rounding point.
 HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",
              "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-KERNEL_SOURCES = ["norm_host.hip", "rmsnorm.hip", "adaln.hip", "anywidth.hip", "widerow.hip"]
+KERNEL_SOURCES = ["norm_host.hip", "rmsnorm.hip", "adaln.hip", "anywidth.hip", "widerow.hip", "qkv.hip"]
 EXT_MODULES = {"fused_rmsnorm": "fused_rmsnorm_ext.cpp", "fused_adaln": "fused_adaln_ext.cpp"}
 
 
@@ -69,7 +69,7 @@ def build_kernels(verbose: bool = True, out: str = None, extra_flags=()) -> str:
     obj_dir = os.path.join(LIB_DIR, "obj") if out == LIB_PATH else out + ".obj"
     os.makedirs(obj_dir, exist_ok=True)
     objs = [os.path.join(obj_dir, os.path.splitext(src)[0] + ".o") for src in KERNEL_SOURCES]
-    with ThreadPoolExecutor(max_workers=min(4, len(KERNEL_SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=min(6, len(KERNEL_SOURCES))) as pool:
         logs = list(pool.map(lambda so: _run([HIPCC, *HIP_FLAGS, *extra_flags, "-c", so[0], "-o", so[1]], cwd=CSRC),
                              zip(KERNEL_SOURCES, objs)))
     logs.append(_run([HIPCC, "--offload-arch=" + ARCH, "-fPIC", "-shared", "-o", out] + objs))

@@ -31,6 +31,8 @@ EXPORTS = (
     "tt_gated_residual_adaln_backward", "tt_adaln_backward_residual", "tt_adaln_backward_static",
     "tt_rmsnorm_rope_forward_strided", "tt_rmsnorm_rope_backward_strided",
     "tt_adaln_forward_seq_first", "tt_adaln_backward_seq_first", "tt_norm_copy_rows_strided",
+    "tt_qkv_rmsnorm_supported", "tt_qkv_rmsnorm_forward", "tt_qkv_rmsnorm_backward_workspace_bytes",
+    "tt_qkv_rmsnorm_backward",
 )
 
 
@@ -81,6 +83,11 @@ def lib() -> ctypes.CDLL:
         L.tt_gated_residual_adaln_backward.argtypes = [vp] * 13 + [i64, i64, i64, ci, vp, sz, vp]
         L.tt_adaln_backward_residual.argtypes = [vp] * 9 + [i64, i64, i64, ci, vp, sz, vp]
         L.tt_norm_copy_rows_strided.argtypes = [vp, vp] + [i64] * 7 + [ci, vp]
+        L.tt_qkv_rmsnorm_supported.argtypes = [i64, ci]
+        L.tt_qkv_rmsnorm_forward.argtypes = [vp] * 7 + [i64] * 5 + [dbl, ci, vp]
+        L.tt_qkv_rmsnorm_backward_workspace_bytes.restype = sz
+        L.tt_qkv_rmsnorm_backward_workspace_bytes.argtypes = [i64] * 4 + [ci]
+        L.tt_qkv_rmsnorm_backward.argtypes = [vp] * 11 + [i64] * 5 + [dbl, ci, vp, sz, vp]
         L.tt_norm_profile_next_row_kernel.argtypes = [vp, vp]
         _lib = L
     return _lib
@@ -240,6 +247,34 @@ def rmsnorm_rope_backward_strided(dout, x, weight, rstd, cos, sin, dx=None):
                                                   d2, cols, _dt(x), _p(ws), n, _stream(x)),
                "tt_rmsnorm_rope_backward_strided")
     return dx, dweight
+
+
+def qkv_rmsnorm_forward(mixed, weight_q, weight_k, eps: float, cos=None, sin=None):
+    """mixed [B, S, H, 3 * D] contiguous; returns q, k [B, H, S, D], rotated on tokens < cos.shape[0]."""
+    _dense_gpu(mixed, weight_q, weight_k)
+    B, S, H, D = *mixed.shape[:3], mixed.shape[-1] // 3
+    q, k = (torch.empty((B, H, S, D), dtype=mixed.dtype, device=mixed.device) for _ in range(2))
+    with torch.cuda.device(mixed.device):
+        _check(lib().tt_qkv_rmsnorm_forward(_p(q), _p(k), _p(mixed), _p(weight_q), _p(weight_k), _p(cos), _p(sin),
+                                            0 if cos is None else cos.shape[0], B, S, H, D, eps, _dt(mixed),
+                                            _stream(mixed)), "tt_qkv_rmsnorm_forward")
+    return q, k
+
+
+def qkv_rmsnorm_backward(dq, dk, dv, mixed, weight_q, weight_k, eps: float, cos=None, sin=None, dmixed=None):
+    """dq, dk, dv [B, H, S, D] contiguous, or None; returns (dmixed, dweight_q, dweight_k)."""
+    _dense_gpu(mixed, weight_q, weight_k, *(g for g in (dq, dk, dv) if g is not None))
+    B, S, H, D = *mixed.shape[:3], mixed.shape[-1] // 3
+    dmixed = torch.empty_like(mixed) if dmixed is None else dmixed
+    dwq, dwk = torch.empty_like(weight_q), torch.empty_like(weight_k)
+    with torch.cuda.device(mixed.device):
+        L = lib()
+        n = L.tt_qkv_rmsnorm_backward_workspace_bytes(B, S, H, D, _dt(mixed))
+        ws = _workspace(n, mixed)
+        _check(L.tt_qkv_rmsnorm_backward(_p(dmixed), _p(dwq), _p(dwk), _p(dq), _p(dk), _p(dv), _p(mixed), _p(weight_q),
+                                         _p(weight_k), _p(cos), _p(sin), 0 if cos is None else cos.shape[0], B, S, H, D,
+                                         eps, _dt(mixed), _p(ws), n, _stream(mixed)), "tt_qkv_rmsnorm_backward")
+    return dmixed, dwq, dwk
 
 
 def adaln_forward(x, scale, shift, eps: float, want_xnorm: bool = False, seq_first: bool = False):

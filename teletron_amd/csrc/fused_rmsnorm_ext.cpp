@@ -240,7 +240,89 @@ void torch_launch_rms_rope_backward_strided(torch::Tensor &dinp, torch::Tensor &
              "tt_rmsnorm_rope_backward_strided");
 }
 
+// ---- the whole QK-norm call site in one kernel per direction (no reference counterpart) ----
+struct QkvShape {
+    int64_t B, S, H, cols, tokens;
+    int dt;
+};
+
+static QkvShape check_qkv(const torch::Tensor &mixed, const torch::Tensor &weight_q, const torch::Tensor &weight_k,
+                          const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    const auto dev = mixed.device();
+    check_dense_on(mixed, dev, "mixed_qkv");
+    TORCH_CHECK(mixed.dim() == 4 && mixed.size(3) % 3 == 0, "mixed_qkv must be [B, S, H, 3*D]");
+    const int64_t cols = mixed.size(3) / 3;
+    for (auto *w : {&weight_q, &weight_k}) {
+        check_dense_on(*w, dev, "weight");
+        check_elems(*w, cols, mixed.scalar_type(), "weight");
+    }
+    TORCH_CHECK(cos.has_value() == sin.has_value(), "pass freqs_cos and freqs_sin together, or neither");
+    const int64_t tokens = cos.has_value() ? check_rope_tables(*cos, *sin, dev, cols, mixed.size(1)) : 0;
+    return {mixed.size(0), mixed.size(1), mixed.size(2), cols, tokens, dtype_code(mixed, "mixed_qkv")};
+}
+
+static const float *table_ptr(const c10::optional<torch::Tensor> &t) {
+    return t.has_value() ? t->data_ptr<float>() : nullptr;
+}
+
+// query, key [B, H, S, D] contiguous = RMSNorm of their slices of mixed, rotated on the tokens of the tables
+void torch_launch_qkv_rms_forward(torch::Tensor &query, torch::Tensor &key, const torch::Tensor &mixed,
+                                  const torch::Tensor &weight_q, const torch::Tensor &weight_k, double epsilon,
+                                  const c10::optional<torch::Tensor> &freqs_cos,
+                                  const c10::optional<torch::Tensor> &freqs_sin) {
+    const QkvShape s = check_qkv(mixed, weight_q, weight_k, freqs_cos, freqs_sin);
+    for (auto *t : {&query, &key}) {
+        check_dense_on(*t, mixed.device(), "query/key");
+        check_elems(*t, s.B * s.S * s.H * s.cols, mixed.scalar_type(), "query/key");
+    }
+    c10::DeviceGuard guard(mixed.device());
+    raise_on(tt_qkv_rmsnorm_forward(query.data_ptr(), key.data_ptr(), mixed.data_ptr(), weight_q.data_ptr(),
+                                    weight_k.data_ptr(), table_ptr(freqs_cos), table_ptr(freqs_sin), s.tokens, s.B, s.S,
+                                    s.H, s.cols, epsilon, s.dt, current_stream(mixed)),
+             "tt_qkv_rmsnorm_forward");
+}
+
+// dmixed is written whole; dquery / dkey / dvalue contiguous [B, H, S, D], or None for an output that was not used
+void torch_launch_qkv_rms_backward(torch::Tensor &dmixed, torch::Tensor &dweight_q, torch::Tensor &dweight_k,
+                                   const c10::optional<torch::Tensor> &dquery, const c10::optional<torch::Tensor> &dkey,
+                                   const c10::optional<torch::Tensor> &dvalue, const torch::Tensor &mixed,
+                                   const torch::Tensor &weight_q, const torch::Tensor &weight_k, double epsilon,
+                                   const c10::optional<torch::Tensor> &freqs_cos,
+                                   const c10::optional<torch::Tensor> &freqs_sin) {
+    const QkvShape s = check_qkv(mixed, weight_q, weight_k, freqs_cos, freqs_sin);
+    const auto dev = mixed.device();
+    const auto st = mixed.scalar_type();
+    const int64_t n = s.B * s.S * s.H * s.cols;
+    check_dense_on(dmixed, dev, "dmixed");
+    check_elems(dmixed, 3 * n, st, "dmixed");
+    for (auto *t : {&dweight_q, &dweight_k}) {
+        check_dense_on(*t, dev, "dweight");
+        check_elems(*t, s.cols, st, "dweight");
+    }
+    const void *g[3] = {nullptr, nullptr, nullptr};
+    const c10::optional<torch::Tensor> *grads[3] = {&dquery, &dkey, &dvalue};
+    for (int i = 0; i < 3; ++i) {
+        if (!grads[i]->has_value() || !(*grads[i])->defined()) continue;
+        check_dense_on(**grads[i], dev, "dquery/dkey/dvalue");
+        check_elems(**grads[i], n, st, "dquery/dkey/dvalue");
+        g[i] = (*grads[i])->data_ptr();
+    }
+    c10::DeviceGuard guard(dev);
+    const size_t need = tt_qkv_rmsnorm_backward_workspace_bytes(s.B, s.S, s.H, s.cols, s.dt);
+    TORCH_CHECK(need > 0 || n == 0, "unsupported head dimension ", s.cols);
+    at::Tensor ws = scratch(need, mixed);
+    raise_on(tt_qkv_rmsnorm_backward(dmixed.data_ptr(), dweight_q.data_ptr(), dweight_k.data_ptr(), g[0], g[1], g[2],
+                                     mixed.data_ptr(), weight_q.data_ptr(), weight_k.data_ptr(), table_ptr(freqs_cos),
+                                     table_ptr(freqs_sin), s.tokens, s.B, s.S, s.H, s.cols, epsilon, s.dt, ws.data_ptr(),
+                                     need, current_stream(mixed)),
+             "tt_qkv_rmsnorm_backward");
+}
+
 PYBIND11_MODULE(fused_rmsnorm, m) {
+    m.def("torch_launch_qkv_rms_forward", &torch_launch_qkv_rms_forward,
+          "RMSNorm (and rotary embedding) of the query and key slices of a fused projection");
+    m.def("torch_launch_qkv_rms_backward", &torch_launch_qkv_rms_backward,
+          "backward of torch_launch_qkv_rms_forward: the projection's whole gradient and both weight gradients");
     m.def("torch_launch_copy_rows_strided", &torch_launch_copy_rows_strided,
           "rows of a contiguous tensor into a strided view of the same shape");
     m.def("torch_launch_rms_rope_forward_strided", &torch_launch_rms_rope_forward_strided,

@@ -1,0 +1,424 @@
+// The QK-norm call site as one kernel per direction: the fused projection mixed [B, S, H, 3 * C] holds q, k and v
+// of a head side by side (teletron/models/dit/dit_attention.py:149-214); q and k leave RMS-normalised over C as
+// contiguous [B, H, S, C] tensors, optionally rotated, and backward assembles the projection's gradient in place.
+//
+//   forward   q, k read from mixed (512 contiguous bytes per head and token at C = 128 two-byte), both written
+//   backward  the gradients of q, k, v and the projection's q, k read; d mixed written whole (768 contiguous bytes);
+//             dweight of both norms as per-workgroup partial sums, one column reducer for the two
+//
+// Arithmetic and rounding points are those of rmsnorm.hip; a head's row is owned by LANES lanes (8, 16, 32 or 64),
+// 16 bytes per lane, 64 / LANES consecutive tokens of one head per wavefront.  The row statistic is formed again in
+// backward from the row it has to read anyway (the same operations, hence the same bits), so nothing but the
+// projection itself is kept between the passes.
+#include "norm_device.h"
+#include "norm_host.h"
+#include "rope_device.h"
+
+// What bounds both kernels is the memory system under a transposing mix of reads and writes: plain copies of the same
+// pattern reach 6.0 TB/s (121 us) forward and 6.0-6.2 TB/s (235-248 us) backward at [1, 29700, 24, 3 * 128] two-byte, and
+// only if what is WRITTEN at a time is contiguous: forward therefore runs its workgroups along the tokens of one head
+// at a time (one-shot), backward along the heads of one token group at a time.  Measured there, against one kernel per
+// tensor (two forward; two backward, one copy of the value gradient, two reducers): forward 122 against 150 us, with
+// tables 137 against 151; backward 256 against 297, with tables 260 against 303.
+//
+// Forward: wavefronts of a workgroup along the tokens (the others along the heads) and heads per wavefront.  Without
+// tables four consecutive token groups of one head (tokens along two / one wavefronts: 127 us; two heads: 126).  With
+// them, two heads of one token group share the 1 KiB of table per token (one head 143 us, three 136, four 149; two heads
+// with two / four wavefronts along the tokens 139 / 155).
+#ifndef TTN_QKV_FWD_TOKEN_WAVES
+#define TTN_QKV_FWD_TOKEN_WAVES (ROPE ? 1 : 4)
+#endif
+#ifndef TTN_QKV_FWD_HEADS
+#define TTN_QKV_FWD_HEADS (ROPE ? 2 : 1)
+#endif
+// Backward: persistent, for the column sums.  Two workgroups per compute unit keep 10 MB requested (three: 271, four
+// 278 us; one with the next step's rows requested ahead 263-272).  The wavefront waits for its rows, works and
+// writes; the other wavefront of its SIMD overlaps it (a second row buffer: 266-269 us).
+#ifndef TTN_QKV_BWD_BLOCKS_PER_CU
+#define TTN_QKV_BWD_BLOCKS_PER_CU 2
+#endif
+// Consecutive steps of a wavefront that are neighbouring heads: with tables the rows it has fetched then serve more than
+// one head (runs of one 271, two 260, three 261, six 267 us); without tables runs only spread the writes (two: 261).
+#ifndef TTN_QKV_BWD_RUN
+#define TTN_QKV_BWD_RUN (Rope::kOn ? 2 : 1)
+#endif
+
+namespace ttn {
+
+constexpr int kLoadNt = 2;  // cache policy of the row loads: non-temporal
+
+// FULL: the row fills its LANES lanes, so its length is known at compile time.
+template <typename T, int LANES_, bool FULL>
+struct HeadGeom {
+    static constexpr int VEC = Elem<T>::VEC;
+    static constexpr int LANES = LANES_;
+    static constexpr int CHUNKS = 1;
+    static constexpr int RPW = kWaveSize / LANES;
+    static __device__ __forceinline__ int cols(int c) { return FULL ? VEC * LANES : c; }
+};
+
+template <typename T, int LANES>
+__device__ __forceinline__ float row_rstd(const u32x4 &x, int C, float eps) {
+    float v[Elem<T>::VEC];
+    Elem<T>::unpack(x, v);
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < Elem<T>::VEC; ++j) ss = fmaf(v[j], v[j], ss);
+    ss = group_sum<LANES>(ss);
+    return 1.0f / sqrtf(ss / (float)C + eps);
+}
+
+template <typename T, int LANES, bool FULL, typename Rope>
+__global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q, T *__restrict__ k,
+                                                              const T *__restrict__ mixed, const T *__restrict__ wq,
+                                                              const T *__restrict__ wk, const Rope rope, int64_t S, int H,
+                                                              int head_blocks, int outer, int c_arg, float eps) {
+    using G = HeadGeom<T, LANES, FULL>;
+    using E = Elem<T>;
+    constexpr bool ROPE = Rope::kOn;
+    constexpr int VEC = G::VEC, RPW = G::RPW;
+    constexpr int TW = TTN_QKV_FWD_TOKEN_WAVES, HW = kRowWaves / TW, HR = TTN_QKV_FWD_HEADS;
+    const int C = G::cols(c_arg);
+    const int lane = threadIdx.x & 63;
+    const int sub = lane / LANES;
+    const int l = lane % LANES;
+    const int wave = wave_id_in_block();
+    const bool in = FULL || l * VEC < C;
+    const int64_t s0 = ((int64_t)blockIdx.x * TW + wave % TW) * RPW;
+    const bool ok = in && s0 + sub < S;
+    const uint32_t from = (uint32_t)sub * (uint32_t)(H * 3 * C * (int)sizeof(T)) + l * 16;
+    const uint32_t to = (uint32_t)(sub * C * (int)sizeof(T)) + l * 16;
+    const u32x4 zero{0, 0, 0, 0};
+
+    for (int y = blockIdx.y; y < outer; y += gridDim.y) {
+        const int64_t b = y / head_blocks;
+        const int h0 = ((y % head_blocks) * HW + wave / TW) * HR;
+        const T *src = mixed + ((b * S + s0) * H + h0) * 3 * C;
+        u32x4 xr[HR][2];
+#pragma unroll
+        for (int i = 0; i < HR; ++i) {
+            const RowReader<kLoadNt> rq(src + i * 3 * C, from), rk(src + (i * 3 + 1) * C, from);
+            const bool here = ok && h0 + i < H;
+            xr[i][0] = here ? rq.get(0) : zero;
+            xr[i][1] = here ? rk.get(0) : zero;
+        }
+        RopeRows<ROPE, 1, VEC> rot;
+        if constexpr (ROPE) rot.fetch(rope, ok, s0 + sub, C, l, LANES);
+        u32x4 w[2];
+        w[0] = in ? load16(reinterpret_cast<const u32x4 *>(wq) + l) : zero;
+        w[1] = in ? load16(reinterpret_cast<const u32x4 *>(wk) + l) : zero;
+#pragma unroll
+        for (int i = 0; i < HR; ++i) {
+            const int64_t row0 = (b * H + h0 + i) * S + s0;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float r = row_rstd<T, LANES>(xr[i][t], C, eps);
+                float v[VEC], wv[VEC];
+                E::unpack(xr[i][t], v);
+                E::unpack(w[t], wv);
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) v[j] *= r;
+                E::round(v);  // y = the normalised row in the element type
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) v[j] *= wv[j];
+                if constexpr (ROPE) {
+                    if (rot.on) {
+                        E::round(v);  // the norm's output in the element type, which the rotation reads
+                        rotate_pairs_forward<VEC>(v, rot.c[0], rot.s[0]);
+                    }
+                }
+                const RowWriter<0> out((t ? k : q) + row0 * C, to);
+                if (ok && h0 + i < H) out.put(0, E::pack(v));
+            }
+        }
+    }
+}
+
+// gq / gk / gv may be null (that output was not used): its slice of d mixed is zero, as is its dweight.
+template <typename T, int LANES, bool FULL, typename Rope>
+__global__ __launch_bounds__(kRowThreads) void qkv_bwd_kernel(
+    T *__restrict__ dmixed, float *__restrict__ partial, const T *__restrict__ gq, const T *__restrict__ gk,
+    const T *__restrict__ gv, const T *__restrict__ mixed, const T *__restrict__ wq, const T *__restrict__ wk,
+    const Rope rope, int64_t S, uint32_t H, uint32_t token_groups, uint32_t units, int c_arg, float eps) {
+    using G = HeadGeom<T, LANES, FULL>;
+    using E = Elem<T>;
+    constexpr int VEC = G::VEC, RPW = G::RPW;
+    __shared__ __align__(16) float lds[kRowWaves][2][LANES * VEC];
+    const int C = G::cols(c_arg);
+    const int lane = threadIdx.x & 63;
+    const int sub = lane / LANES;
+    const int l = lane % LANES;
+    const int wave = wave_id_in_block();
+    const bool in = FULL || l * VEC < C;
+    const uint32_t mixed_lane = (uint32_t)sub * (H * 3u * (uint32_t)C * (uint32_t)sizeof(T)) + l * 16;
+    const uint32_t dense_lane = (uint32_t)(sub * C * (int)sizeof(T)) + l * 16;
+    const u32x4 zero{0, 0, 0, 0};
+    const uint32_t one_lo = opaque_const(kOneLo<std::conditional_t<kHasDot2<T>, T, bf16_t>>);
+    const uint32_t one_hi = opaque_const(kOneHi<std::conditional_t<kHasDot2<T>, T, bf16_t>>);
+    const uint32_t waves = gridDim.x * kRowWaves, me = blockIdx.x * kRowWaves + wave;
+    const bool has[3] = {gq != nullptr, gk != nullptr, gv != nullptr};
+
+    RowParam<T, 2> wp;
+    wp.set(0, in ? load16(reinterpret_cast<const u32x4 *>(wq) + l) : zero);
+    wp.set(1, in ? load16(reinterpret_cast<const u32x4 *>(wk) + l) : zero);
+    float acc[2][VEC];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) acc[t][j] = 0.0f;
+
+    // heads fastest, so that what the wavefronts of the chip write at a time is one contiguous region of d mixed
+    constexpr uint32_t kRun = TTN_QKV_BWD_RUN;
+    [[maybe_unused]] RopeRows<Rope::kOn, 1, VEC> rot;
+    [[maybe_unused]] uint32_t rot_group = 0xffffffffu;
+    const uint32_t runs = (units + kRun - 1) / kRun;
+    const uint32_t steps = runs > me ? ((runs - me + waves - 1) / waves) * kRun : 0;
+    for (uint32_t step = 0; step < steps; ++step) {
+        const uint32_t u = (step / kRun * waves + me) * kRun + step % kRun;
+        const uint32_t h = u % H, rest = u / H;
+        const uint32_t tg = rest % token_groups;
+        const int64_t b = rest / token_groups;
+        const int64_t s0 = (int64_t)tg * RPW;
+        const bool exists = s0 + sub < S && u < units;  // this lane's token
+        const bool ok = in && exists;
+        const int64_t at = ((b * S + s0) * H + h) * 3 * C;
+        const int64_t dense = ((b * H + h) * S + s0) * C;
+        u32x4 g[3], x[2];
+        {
+            const RowReader<kLoadNt> rgq(gq + dense, dense_lane), rgk(gk + dense, dense_lane), rgv(gv + dense, dense_lane);
+            const RowReader<kLoadNt> rxq(mixed + at, mixed_lane), rxk(mixed + at + C, mixed_lane);
+            g[0] = (ok && has[0]) ? rgq.get(0) : zero;
+            g[1] = (ok && has[1]) ? rgk.get(0) : zero;
+            x[0] = ok ? rxq.get(0) : zero;
+            x[1] = ok ? rxk.get(0) : zero;
+            g[2] = (ok && has[2]) ? rgv.get(0) : zero;
+        }
+        if constexpr (Rope::kOn) {
+            if (tg != rot_group) rot.fetch(rope, in && s0 + sub < S, s0 + sub, C, l, LANES);
+            rot_group = tg;
+            // the gradients arrive rotated: back through the rotation first
+            if (rot.on) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    float gvv[VEC];
+                    E::unpack(g[t], gvv);
+                    rotate_pairs_backward<E, VEC>(gvv, rot.c[0], rot.s[0]);
+                    g[t] = E::pack(gvv);
+                }
+            }
+        }
+        u32x4 d[3] = {zero, zero, g[2]};
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if (!has[t]) continue;
+            const u32x4 gy = wp.times(t, g[t]);  // rnd(g * w)
+            float dot = 0.0f;
+            if constexpr (kHasDot2<T>) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dot = dot2<T>(gy[i], x[t][i], dot);
+            } else {
+                float gyv[VEC], xv[VEC];
+                E::unpack(gy, gyv);
+                E::unpack(x[t], xv);
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) dot = fmaf(gyv[j], xv[j], dot);
+            }
+            dot = group_sum<LANES>(dot);
+            const float rstd = row_rstd<T, LANES>(x[t], C, eps);
+            const float r = exists ? rstd : 0.0f;  // rows past the end must add nothing, whatever eps is
+            const float coef = -((dot / (float)C) * r * r * r);
+            float gyv[VEC], xv[VEC], o[VEC], y[VEC];
+            E::unpack(gy, gyv);
+            E::unpack(x[t], xv);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) {
+                o[j] = fmaf(xv[j], coef, gyv[j] * r);
+                y[j] = xv[j] * r;
+            }
+            d[t] = E::pack(o);
+            add_rounded_products<T>(acc[t], g[t], y, one_lo, one_hi);  // dw += rnd(g * rnd(y))
+        }
+        const RowWriter<0> wd[3] = {{dmixed + at, mixed_lane}, {dmixed + at + C, mixed_lane}, {dmixed + at + 2 * C, mixed_lane}};
+        if (ok) {
+#pragma unroll
+            for (int t = 0; t < 3; ++t) wd[t].put(0, d[t]);
+        }
+    }
+
+    // the workgroup's partial row: tokens of a wavefront folded, then wavefronts in order
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            const float v = fold_rows_of_wave<LANES>(acc[t][j]);
+            if (sub == 0) lds[wave][t][l * VEC + j] = v;
+        }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * C; i += kRowThreads) {
+        const int t = i >= C, c = t ? i - C : i;
+        partial[(int64_t)blockIdx.x * 2 * C + i] = ((lds[0][t][c] + lds[1][t][c]) + lds[2][t][c]) + lds[3][t][c];
+    }
+}
+
+// ------------------------------------------------------------------ host side
+
+static int head_lanes(int pieces) { return pieces <= 8 ? 8 : pieces <= 16 ? 16 : pieces <= 32 ? 32 : 64; }
+
+static int qkv_pieces(int64_t cols, int dtype) { return (int)(cols / (16 / (int64_t)elem_bytes(dtype))); }
+
+static int64_t qkv_bwd_blocks(int64_t units, int cus) {
+    const int64_t want = (units + kRowWaves - 1) / kRowWaves, most = (int64_t)cus * TTN_QKV_BWD_BLOCKS_PER_CU;
+    return want < most ? want : most;
+}
+
+struct QkvSizes {
+    int64_t B, S, H, cols;
+    int lanes;
+    int64_t token_groups() const { return (S + kWaveSize / lanes - 1) / (kWaveSize / lanes); }
+    int64_t units() const { return B * token_groups() * H; }
+};
+
+template <typename T, int LANES, bool FULL, typename Rope>
+static void launch_qkv_fwd(const QkvSizes &z, void *q, void *k, const void *mixed, const void *wq, const void *wk,
+                           const Rope &rope, float eps, hipStream_t stream) {
+    [[maybe_unused]] constexpr bool ROPE = Rope::kOn;
+    constexpr int TW = TTN_QKV_FWD_TOKEN_WAVES, heads = kRowWaves / TW * TTN_QKV_FWD_HEADS;
+    const int head_blocks = (int)((z.H + heads - 1) / heads);
+    const int64_t outer = z.B * head_blocks;
+    const dim3 grid((unsigned)((z.token_groups() + TW - 1) / TW), (unsigned)(outer < 65535 ? outer : 65535));
+    RowKernelProfile prof(stream);
+    qkv_fwd_kernel<T, LANES, FULL, Rope><<<grid, dim3(kRowThreads), 0, stream>>>(
+        (T *)q, (T *)k, (const T *)mixed, (const T *)wq, (const T *)wk, rope, z.S, (int)z.H, head_blocks, (int)outer,
+        (int)z.cols, eps);
+}
+
+template <typename T, int LANES, bool FULL, typename Rope>
+static void launch_qkv_bwd(const QkvSizes &z, int64_t blocks, void *dmixed, void *ws, const void *gq, const void *gk,
+                           const void *gv, const void *mixed, const void *wq, const void *wk, const Rope &rope, float eps,
+                           hipStream_t stream) {
+    RowKernelProfile prof(stream);
+    qkv_bwd_kernel<T, LANES, FULL, Rope><<<dim3((unsigned)blocks), dim3(kRowThreads), 0, stream>>>(
+        (T *)dmixed, (float *)ws, (const T *)gq, (const T *)gk, (const T *)gv, (const T *)mixed, (const T *)wq,
+        (const T *)wk, rope, z.S, (uint32_t)z.H, (uint32_t)z.token_groups(), (uint32_t)z.units(), (int)z.cols, eps);
+}
+
+static int check_qkv(const char *who, int64_t B, int64_t S, int64_t H, int64_t cols, int dtype, const float *cos,
+                     const float *sin, int64_t rope_tokens, QkvSizes *z) {
+    if (B < 0 || S < 0 || H < 0 || cols <= 0)
+        return fail(TT_NORM_EINVAL, "%s: B=%lld S=%lld H=%lld cols=%lld", who, (long long)B, (long long)S, (long long)H,
+                    (long long)cols);
+    if (!tt_qkv_rmsnorm_supported(cols, dtype))
+        return fail(TT_NORM_EUNSUPPORTED, "%s: cols=%lld dtype=%d (a head's row must be at most 64 whole 16-byte pieces)",
+                    who, (long long)cols, dtype);
+    if (rope_tokens < 0 || rope_tokens > S)
+        return fail(TT_NORM_EINVAL, "%s: rope_tokens=%lld outside [0, S=%lld]", who, (long long)rope_tokens, (long long)S);
+    if (rope_tokens > 0) {
+        if (cols != 128) return fail(TT_NORM_EUNSUPPORTED, "%s: the rotation is built for cols 128 (the head dimension) only", who);
+        if (!cos || !sin) return fail(TT_NORM_EINVAL, "%s: null cos/sin table", who);
+        if (!aligned16(cos) || !aligned16(sin)) return fail(TT_NORM_EALIGN, "%s: cos/sin table not 16-byte aligned", who);
+    }
+    // a wavefront's tokens are addressed with 32-bit byte offsets from the first of them
+    if (H * 3 * cols > kMaxRowStrideBytes / (int64_t)elem_bytes(dtype))
+        return fail(TT_NORM_EINVAL, "%s: a token of the projection exceeds 256 MiB", who);
+    *z = QkvSizes{B, S, H, cols, head_lanes(qkv_pieces(cols, dtype))};
+    if (z->token_groups() > 0x7fffffffLL || z->units() > 0x7fffffffLL) return fail(TT_NORM_EINVAL, "%s: grid too large", who);
+    return TT_NORM_OK;
+}
+
+static int check_qkv_ptrs(const char *who, std::initializer_list<const void *> ptrs) {
+    for (const void *p : ptrs) {
+        if (!p) return fail(TT_NORM_EINVAL, "%s: null pointer", who);
+        if (!aligned16(p)) return fail(TT_NORM_EALIGN, "%s: pointer %p not 16-byte aligned", who, p);
+    }
+    return TT_NORM_OK;
+}
+
+}  // namespace ttn
+
+using namespace ttn;
+
+// CALL(T, LANES, FULL, Rope, rope) for the run-time (dtype, lanes, full row, rotation)
+#define TTN_QKV_LANES(T, CALL)                                                                                    \
+    do {                                                                                                          \
+        constexpr int kHead = 128 / Elem<T>::VEC;                                                                 \
+        if (rope.tokens > 0) { CALL(T, kHead, true, RopeTable, rope); }                                           \
+        else if (z.lanes == 8) { if (full) { CALL(T, 8, true, NoRope, NoRope{}); } else { CALL(T, 8, false, NoRope, NoRope{}); } }    \
+        else if (z.lanes == 16) { if (full) { CALL(T, 16, true, NoRope, NoRope{}); } else { CALL(T, 16, false, NoRope, NoRope{}); } } \
+        else if (z.lanes == 32) { if (full) { CALL(T, 32, true, NoRope, NoRope{}); } else { CALL(T, 32, false, NoRope, NoRope{}); } } \
+        else { if (full) { CALL(T, 64, true, NoRope, NoRope{}); } else { CALL(T, 64, false, NoRope, NoRope{}); } } \
+    } while (0)
+#define TTN_QKV_DISPATCH(CALL)                                      \
+    do {                                                            \
+        if (dtype == TT_NORM_BF16) TTN_QKV_LANES(bf16_t, CALL);     \
+        else if (dtype == TT_NORM_F16) TTN_QKV_LANES(f16_t, CALL);  \
+        else TTN_QKV_LANES(float, CALL);                            \
+    } while (0)
+
+extern "C" {
+
+int tt_qkv_rmsnorm_supported(int64_t cols, int dtype) {
+    return (tt_norm_supported(cols, dtype) && qkv_pieces(cols, dtype) <= kWaveSize) ? 1 : 0;
+}
+
+int tt_qkv_rmsnorm_forward(void *q, void *k, const void *mixed, const void *weight_q, const void *weight_k,
+                           const float *cos, const float *sin, int64_t rope_tokens, int64_t B, int64_t S, int64_t H,
+                           int64_t cols, double eps, int dtype, void *stream) {
+    const char *who = "tt_qkv_rmsnorm_forward";
+    QkvSizes z;
+    int st = check_qkv(who, B, S, H, cols, dtype, cos, sin, rope_tokens, &z);
+    if (st != TT_NORM_OK) return st;
+    if (z.units() == 0) return TT_NORM_OK;
+    st = check_qkv_ptrs(who, {q, k, mixed, weight_q, weight_k});
+    if (st != TT_NORM_OK) return st;
+    const bool full = qkv_pieces(cols, dtype) == z.lanes;
+    const RopeTable rope{cos, sin, rope_tokens};
+#define CALL(T, L, F, R, r) launch_qkv_fwd<T, L, F, R>(z, q, k, mixed, weight_q, weight_k, r, (float)eps, (hipStream_t)stream)
+    TTN_QKV_DISPATCH(CALL);
+#undef CALL
+    return check_launch("qkv forward launch");
+}
+
+size_t tt_qkv_rmsnorm_backward_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t cols, int dtype) {
+    if (B <= 0 || S <= 0 || H <= 0 || !tt_qkv_rmsnorm_supported(cols, dtype)) return 0;
+    int st = TT_NORM_OK;
+    const int cus = current_device_cus(&st);
+    if (st != TT_NORM_OK) return 0;
+    const QkvSizes z{B, S, H, cols, head_lanes(qkv_pieces(cols, dtype))};
+    return (size_t)qkv_bwd_blocks(z.units(), cus) * 2 * cols * sizeof(float);
+}
+
+int tt_qkv_rmsnorm_backward(void *dmixed, void *dweight_q, void *dweight_k, const void *dq, const void *dk,
+                            const void *dv, const void *mixed, const void *weight_q, const void *weight_k,
+                            const float *cos, const float *sin, int64_t rope_tokens, int64_t B, int64_t S, int64_t H,
+                            int64_t cols, double eps, int dtype, void *workspace, size_t workspace_bytes, void *stream) {
+    const char *who = "tt_qkv_rmsnorm_backward";
+    QkvSizes z;
+    int st = check_qkv(who, B, S, H, cols, dtype, cos, sin, rope_tokens, &z);
+    if (st != TT_NORM_OK) return st;
+    if (!dweight_q || !dweight_k) return fail(TT_NORM_EINVAL, "%s: null dweight", who);
+    const hipStream_t s = (hipStream_t)stream;
+    // empty input: the parameter gradients are empty sums, written by the reducer over zero partial rows
+    if (z.units() == 0) return launch_colreduce(dweight_q, dweight_k, nullptr, nullptr, 1, 0, cols, 2 * cols, dtype, s);
+    st = check_qkv_ptrs(who, {dmixed, mixed, weight_q, weight_k});
+    if (st != TT_NORM_OK) return st;
+    for (const void *p : {dq, dk, dv})
+        if (!aligned16(p)) return fail(TT_NORM_EALIGN, "%s: pointer %p not 16-byte aligned", who, p);
+    const int cus = current_device_cus(&st);
+    if (st != TT_NORM_OK) return st;
+    const int64_t blocks = qkv_bwd_blocks(z.units(), cus);
+    const size_t need = (size_t)blocks * 2 * cols * sizeof(float);
+    if (!workspace || workspace_bytes < need)
+        return fail(TT_NORM_EWORKSPACE, "%s: workspace %zu B < required %zu B", who, workspace_bytes, need);
+    if (!aligned16(workspace)) return fail(TT_NORM_EALIGN, "%s: workspace %p not 16-byte aligned", who, workspace);
+    const bool full = qkv_pieces(cols, dtype) == z.lanes;
+    const RopeTable rope{cos, sin, rope_tokens};
+#define CALL(T, L, F, R, r)                                                                                        \
+    launch_qkv_bwd<T, L, F, R>(z, blocks, dmixed, workspace, dq, dk, dv, mixed, weight_q, weight_k, r, (float)eps, s)
+    TTN_QKV_DISPATCH(CALL);
+#undef CALL
+    st = check_launch("qkv backward launch");
+    if (st != TT_NORM_OK) return st;
+    return launch_colreduce(dweight_q, dweight_k, nullptr, (const float *)workspace, 1, (int)blocks, cols, 2 * cols, dtype, s);
+}
+
+}  // extern "C"

@@ -52,6 +52,7 @@ except ImportError as exc:  # pragma: no cover - exercised only on an unbuilt tr
 TUNED_COLS = (128, 3072)  # the reference's two shapes (the tuned kernels)
 _ELEM_BYTES = {torch.bfloat16: 2, torch.float16: 2, torch.float32: 4}
 _MAX_PIECES = 1024  # 16-byte pieces per row the kernels are built for
+_MAX_JOINT_HEAD_BYTES = 1024  # a head's row the joint q / k / v kernels take: 64 16-byte pieces
 
 
 def cols_supported(cols: int, dtype: torch.dtype) -> bool:
@@ -541,11 +542,11 @@ class QKVSplitNormFunction(Function):
     of one head side by side (dit_attention.py:149-190 with one query head per group).  q and k come
     back RMS-normalised over D as contiguous [B, H, S, D] tensors, v as the transposed view of its
     slice -- what torch.split, .transpose(1, 2), q_layernorm and k_layernorm produce together
-    (dit_attention.py:191-214) -- read straight out of mixed_qkv.
-    Backward writes the gradients of q and k from the kernels directly into their slices of one
-    [B, S, H, 3*D] gradient tensor and copies the gradient of v into its slice, so the concatenation
-    that torch.split's backward would run over three separate gradients never happens.
-    D: any supported row (128 runs the tuned kernels; the rotary form needs 128)."""
+    (dit_attention.py:191-214) -- read straight out of mixed_qkv, both in one kernel.
+    Backward writes the whole [B, S, H, 3*D] gradient tensor in one kernel (the norms' gradients and the
+    copy of v's), so the concatenation that torch.split's backward would run over three separate gradients
+    never happens.
+    D: any supported row (the rotary form needs 128); rows of more than 1 KiB run one strided norm per tensor."""
 
     @staticmethod
     def forward(ctx, mixed_qkv, weight_q, weight_k, epsilon, *rotary):
@@ -579,30 +580,42 @@ class QKVSplitNormFunction(Function):
         q_in, k_in, v_in = (mixed[..., i * cols:(i + 1) * cols].transpose(1, 2) for i in range(3))
         ws = [w.contiguous().to(mixed.dtype) for w in (weight_q, weight_k)]
         B, H, S, _ = q_in.shape
-        outs, stats = [], []
-        for x, w in ((q_in, ws[0]), (k_in, ws[1])):
-            out = torch.empty((B, H, S, cols), dtype=mixed.dtype, device=mixed.device)
-            invvar = torch.empty(B * H * S, device=mixed.device, dtype=torch.float32)
-            if tables is None:
-                ext.torch_launch_rms_forward_strided(out, x, w, float(epsilon), invvar)
-            else:
-                ext.torch_launch_rms_rope_forward_strided(out, x, w, float(epsilon), invvar, tables[0], tables[1])
-            outs.append(out)
-            stats.append(invvar)
-        ctx.save_for_backward(mixed, ws[0], ws[1], stats[0], stats[1], *(tables or ()))
         ctx.cols = cols
+        ctx.epsilon = float(epsilon)
         ctx.n_rotary = len(rotary)
         ctx.w_meta = [(w.shape, w.dtype) for w in (weight_q, weight_k)]
         ctx.set_materialize_grads(False)
         # v leaves as a copy-free view only when mixed_qkv itself was usable in place
         v_out = v_in if mixed is mixed_qkv else v_in.clone()
+        ctx.joint = cols * mixed.element_size() <= _MAX_JOINT_HEAD_BYTES
+        if ctx.joint:
+            q, k = (torch.empty((B, H, S, cols), dtype=mixed.dtype, device=mixed.device) for _ in range(2))
+            ext.torch_launch_qkv_rms_forward(q, k, mixed, ws[0], ws[1], ctx.epsilon, *(tables or (None, None)))
+            ctx.save_for_backward(mixed, ws[0], ws[1], *(tables or ()))
+            return q, k, v_out
+        outs, stats = [], []   # wider heads: one strided norm per tensor
+        for x, w in ((q_in, ws[0]), (k_in, ws[1])):
+            out = torch.empty((B, H, S, cols), dtype=mixed.dtype, device=mixed.device)
+            invvar = torch.empty(B * H * S, device=mixed.device, dtype=torch.float32)
+            ext.torch_launch_rms_forward_strided(out, x, w, ctx.epsilon, invvar)
+            outs.append(out)
+            stats.append(invvar)
+        ctx.save_for_backward(mixed, ws[0], ws[1], stats[0], stats[1])
         return outs[0], outs[1], v_out
 
     @staticmethod
     def backward(ctx, grad_q, grad_k, grad_v):
-        mixed, wq, wk, rstd_q, rstd_k, *tables = ctx.saved_tensors
+        d_mixed = torch.empty_like(ctx.saved_tensors[0])
+        if ctx.joint:
+            mixed, wq, wk, *tables = ctx.saved_tensors
+            grads = [None if g is None else _aligned_contiguous(g.to(mixed.dtype)) for g in (grad_q, grad_k, grad_v)]
+            grads_w = [torch.empty_like(w) for w in (wq, wk)]
+            fused_rmsnorm.torch_launch_qkv_rms_backward(d_mixed, *grads_w, *grads, mixed, wq, wk, ctx.epsilon,
+                                                        *(tables or (None, None)))
+            grads_w = [dw.reshape(shape).to(dtype) for dw, (shape, dtype) in zip(grads_w, ctx.w_meta)]
+            return (d_mixed, grads_w[0], grads_w[1], None) + (None,) * ctx.n_rotary
+        mixed, wq, wk, rstd_q, rstd_k = ctx.saved_tensors
         cols = ctx.cols
-        d_mixed = torch.empty_like(mixed)
         slices = [d_mixed[..., i * cols:(i + 1) * cols].transpose(1, 2) for i in range(3)]
         grads_w = []
         for i, (g, w, rstd) in enumerate(((grad_q, wq, rstd_q), (grad_k, wk, rstd_k))):
@@ -613,17 +626,14 @@ class QKVSplitNormFunction(Function):
             else:
                 g = _aligned_contiguous(g.to(mixed.dtype))
                 x = mixed[..., i * cols:(i + 1) * cols].transpose(1, 2)
-                if tables:
-                    fused_rmsnorm.torch_launch_rms_rope_backward_strided(slices[i], dw, g, x, w, rstd, *tables)
-                else:
-                    fused_rmsnorm.torch_launch_rms_backward_strided(slices[i], dw, g, x, w, rstd)
+                fused_rmsnorm.torch_launch_rms_backward_strided(slices[i], dw, g, x, w, rstd)
             shape, dtype = ctx.w_meta[i]
             grads_w.append(dw.reshape(shape).to(dtype))
         if grad_v is None:
             slices[2].zero_()
         else:
             fused_rmsnorm.torch_launch_copy_rows_strided(slices[2], _aligned_contiguous(grad_v.to(mixed.dtype)))
-        return (d_mixed, grads_w[0], grads_w[1], None) + (None,) * ctx.n_rotary
+        return d_mixed, grads_w[0], grads_w[1], None
 
 
 def rotate_pairs_eager(x: torch.Tensor, freqs_cos: torch.Tensor, freqs_sin: torch.Tensor) -> torch.Tensor:

@@ -1,0 +1,103 @@
+"""The joint QK-norm kernels (qkv.hip): the sizes where a row's lanes, a wavefront's tokens, a workgroup's heads or the
+persistent grid are partly empty, in every lane geometry, against the eager oracle on the CPU and, bit for bit where
+the arithmetic is the same, the strided kernels one tensor at a time."""
+import pytest
+import torch
+
+from oracle import norm_oracle as O
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-6
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.fixture(scope="module")
+def capi(gpu_device):
+    from teletron_amd import capi as c
+    c.lib()
+    return c
+
+
+# B, S, H, D, rotated tokens.  D in 16-byte pieces of two-byte rows: 1, 8, 9, 16, 32, 63, 64 -> 8, 8, 16, 16, 32, 64, 64 lanes
+CASES = [
+    (1, 1, 1, 128, 0), (2, 3, 5, 8, 0), (3, 17, 2, 64, 0), (1, 33, 7, 72, 0), (2, 15, 3, 256, 0), (1, 9, 4, 504, 0),
+    (2, 5, 3, 512, 0), (1, 1501, 24, 128, 0), (2, 61, 5, 128, 61), (1, 67, 9, 128, 40), (1, 5, 1, 128, 1),
+]
+
+
+@pytest.mark.parametrize("dtype", [BF, HF, F32])
+@pytest.mark.parametrize("B,S,H,D,rotated", CASES)
+def test_joint_kernels_match_the_oracle(capi, gpu_device, B, S, H, D, rotated, dtype):
+    if dtype == F32 and D > 256:
+        assert capi.lib().tt_qkv_rmsnorm_supported(D, capi.F32) == 0      # more than 64 pieces
+        return
+    gen = torch.Generator().manual_seed(S * 31 + D)
+    mixed = torch.randn(B, S, H, 3 * D, generator=gen).to(dtype)
+    w = [(1 + 0.02 * torch.randn(D, generator=gen)).to(dtype) for _ in range(2)]
+    grads = [torch.randn(B, H, S, D, generator=gen).to(dtype) for _ in range(3)]
+    tables = O.make_rope_tables(rotated, D, seed=5) if rotated else (None, None)
+    dev = lambda t: None if t is None else t.to(gpu_device)
+    cos, sin = dev(tables[0]), dev(tables[1])
+    m_d, w_d, g_d = dev(mixed), [dev(t) for t in w], [dev(t) for t in grads]
+
+    # outputs between margins that must stay as they are
+    def guarded(*shape):
+        buf = torch.full((2048 + torch.Size(shape).numel() + 2048,), 7.0, dtype=dtype, device=gpu_device)
+        return buf, buf[2048:-2048].view(shape)
+
+    buf, dmixed = guarded(B, S, H, 3 * D)
+    q, k = capi.qkv_rmsnorm_forward(m_d, *w_d, EPS, cos, sin)
+    _, dwq, dwk = capi.qkv_rmsnorm_backward(*g_d, m_d, *w_d, EPS, cos, sin, dmixed=dmixed)
+    assert bool((buf[:2048] == 7.0).all()) and bool((buf[-2048:] == 7.0).all())
+    assert torch.equal(dmixed[..., 2 * D:].transpose(1, 2), g_d[2])
+
+    # 16-bit bars as for the per-tensor kernels; fp32 leaves room for the order of the sums only
+    rtol, atol = (1e-4, 1e-5) if dtype == F32 else (1e-2, 1e-3)
+    for t, (out, dw) in enumerate(((q, dwq), (k, dwk))):
+        x = m_d[..., t * D:(t + 1) * D].transpose(1, 2)
+        if rotated:
+            want = capi.rmsnorm_rope_forward_strided(x, w_d[t], cos, sin, EPS)[0]
+            e_out, e_dx, e_dw = O.eager_qk_norm_rope_fwd_bwd(x.cpu(), w[t], *tables, grads[t])
+        else:
+            want = capi.rmsnorm_forward_strided(x, w_d[t], EPS)[0]
+            e_out, e_dx, e_dw = O.eager_rmsnorm_fwd_bwd(x.cpu(), w[t], grads[t])
+        assert torch.equal(out, want)
+        assert O.frac_outside(out.cpu(), e_out, 2.0 ** -6 if dtype != F32 else 1e-5, 2.0 ** -7 if dtype != F32 else 1e-6) == 0.0
+        dx = dmixed[..., t * D:(t + 1) * D].transpose(1, 2)
+        # short rows: the two terms of dx cancel, and a one-ulp disagreement has the size of the terms
+        terms = e_dx.float().abs() + x.cpu().float().abs() + grads[t].float().abs()
+        assert O.frac_outside(dx.cpu(), e_dx, rtol, atol, magnitude=terms) == 0.0
+        y = torch.nn.functional.normalize(x.cpu().float(), dim=-1) * D ** 0.5
+        assert O.colsum_outside(dw.cpu(), e_dw, (grads[t].float() * y).reshape(-1, D), dim=0, rtol=rtol,
+                                ulp=2.0 ** -6 if dtype != F32 else 1e-5) == 0
+
+
+@pytest.mark.parametrize("missing", [(0,), (1,), (2,), (0, 2)])
+def test_outputs_that_were_not_used(capi, gpu_device, missing):
+    """A missing gradient leaves zeros in its slice and its dweight and does not touch the others; a row of infinities
+    under it leaves zeros too."""
+    gen = torch.Generator(device=gpu_device).manual_seed(3)
+    mixed = torch.randn(1, 21, 3, 384, device=gpu_device, generator=gen).to(BF)
+    w = [torch.ones(128, device=gpu_device, dtype=BF) for _ in range(2)]
+    grads = [torch.randn(1, 3, 21, 128, device=gpu_device, generator=gen).to(BF) for _ in range(3)]
+    full = capi.qkv_rmsnorm_backward(*grads, mixed, *w, EPS)
+    if 0 in missing:
+        mixed[..., :128] = float("inf")
+    got = capi.qkv_rmsnorm_backward(*[None if i in missing else g for i, g in enumerate(grads)], mixed, *w, EPS)
+    for i in range(3):
+        part, whole = (t[0][..., i * 128:(i + 1) * 128] for t in (got, full))
+        assert (not part.any()) if i in missing else torch.equal(part, whole)
+        if i < 2:
+            assert (not got[1 + i].any()) if i in missing else torch.equal(got[1 + i], full[1 + i])
+
+
+def test_empty_projection_and_refusals(capi, gpu_device):
+    w = [torch.ones(64, device=gpu_device, dtype=BF) for _ in range(2)]
+    mixed = torch.empty(2, 0, 4, 192, device=gpu_device, dtype=BF)
+    none = torch.empty(2, 4, 0, 64, device=gpu_device, dtype=BF)
+    assert capi.qkv_rmsnorm_forward(mixed, *w, EPS)[0].numel() == 0
+    _, dwq, dwk = capi.qkv_rmsnorm_backward(none, none, none, mixed, *w, EPS)
+    assert not dwq.any() and not dwk.any()
+    wide = torch.empty(1, 2, 1, 3 * 520, device=gpu_device, dtype=BF)
+    with pytest.raises(capi.NormError, match="64 whole 16-byte pieces"):
+        capi.qkv_rmsnorm_forward(wide, *[torch.ones(520, device=gpu_device, dtype=BF)] * 2, EPS)
