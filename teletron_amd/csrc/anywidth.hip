@@ -16,18 +16,47 @@
 #include "norm_device.h"
 #include "norm_host.h"
 
-// Stores of dx / out: 1 = write-through at device scope (RowWriter<1>), 0 = plain streaming store.
-// Measured both ways per width: backward gains up to 7 % with write-through for rows of up to six
-// accesses per lane (512 columns 212 -> 197 us, 1024 196 -> 186 us, 1536 184 -> 182 us) and loses 3-4 %
-// at eight and twelve (4096, 6144 columns), so the wide geometries keep the plain store.
+// Rows of a full wavefront (33 pieces and more) are read and written through buffer resources that end with the row, and
+// the backward kernels request the next row between the two passes of the current one; what bounds them is the memory
+// system and, below some 50 MB per tensor, the fixed cost of a launch (ramp, last rows, flush of the column sums).
+// Measured as calls with the reducer behind them, against plain masked loads, no request ahead, two or three workgroups
+// per compute unit and one wavefront at a time in the flush: AdaLN backward 12000 x 1536 bf16 30.4 -> 25.1 us,
+// 8 x 1025 x 1536 fp16 26.4 -> 21.1, 12000 x 1024 24.5 -> 20.1, 40000 x 2560 149 -> 104 (five accesses per lane instead
+// of six, one of them empty), 30000 x 1536 fp32 105 -> 96; RMSNorm backward 12000 x 2560 51.7 -> 36.5; gated backward
+// 12000 x 2560 94 -> 71.  The packed forms of the products (RowParam, add_elements) measure the same here.
+
+// Cache policy (sc0 = 1, nt = 2, sc1 = 16) of full-wavefront rows: loads and forward stores non-temporal, backward
+// stores write-through as well (plain non-temporal: 1536 columns 184 instead of 182 us, 1024 196 / 186).
+#ifndef TTN_ANY_LOAD_POLICY
+#define TTN_ANY_LOAD_POLICY 2
+#endif
+#ifndef TTN_ANY_FWD_STORE_POLICY
+#define TTN_ANY_FWD_STORE_POLICY 2
+#endif
+#ifndef TTN_ANY_BWD_STORE_POLICY
+#define TTN_ANY_BWD_STORE_POLICY 18
+#endif
+// The same for rows of part of a wavefront: 1 = write-through (RowWriter<1>), 0 = plain streaming store.
 #ifndef TTN_ANY_FWD_STORE
 #define TTN_ANY_FWD_STORE 0
 #endif
 #ifndef TTN_ANY_BWD_STORE
 #define TTN_ANY_BWD_STORE 1
 #endif
+// AdaLN forward: rows per wavefront where that leaves enough workgroups; they share the modulation row (100000 x 1024
+// bf16: one row 73.9, two 68.4, four 71.0 us; 12000 x 1536: 18.0 / 16.7 / 16.4).
+#ifndef TTN_ANY_ADALN_FWD_ROWS
+#define TTN_ANY_ADALN_FWD_ROWS 2
+#endif
+// Backward workgroups per compute unit by accesses per lane (1 to 6).  One with the next row requested ahead beats two
+// and three without from three accesses on (12000 x 2560: 37.5 against 41.2 us), and writes fewer partial rows.
+#ifndef TTN_ANY_BWD_BLOCKS
+#define TTN_ANY_BWD_BLOCKS {6, 2, 1, 1, 1, 1}
+#endif
 
 namespace ttn {
+
+constexpr int kLoad = TTN_ANY_LOAD_POLICY, kFwdStore = TTN_ANY_FWD_STORE_POLICY, kBwdStore = TTN_ANY_BWD_STORE_POLICY;
 
 template <typename T, int LANES_, int CHUNKS_>
 struct PadGeom {
@@ -40,6 +69,34 @@ struct PadGeom {
     static_assert(LANES == 64 || CHUNKS == 1, "only full wavefronts take several accesses per lane");
 };
 
+// rnd(a * b) for the elements of one access, both packed
+template <typename T>
+__device__ __forceinline__ u32x4 packed_products(const u32x4 &a, const u32x4 &b) {
+    using E = Elem<T>;
+    if constexpr (std::is_same<T, f16_t>::value) {
+        PairFactor<f16_t> f;
+        f.set(b);
+        return rounded_products<f16_t>(a, f);
+    } else {
+        float av[E::VEC], bv[E::VEC];
+        E::unpack(a, av);
+        E::unpack(b, bv);
+#pragma unroll
+        for (int j = 0; j < E::VEC; ++j) av[j] *= bv[j];
+        return E::pack(av);
+    }
+}
+
+// acc += v per column.  Not the packed dot product against (1, 0) / (0, 1): that multiplies the pair's other element by
+// zero, and an infinity there would spread to this column's sum.
+template <typename T>
+__device__ __forceinline__ void add_columns(float (&acc)[Elem<T>::VEC], const u32x4 &v) {
+    float f[Elem<T>::VEC];
+    Elem<T>::unpack(v, f);
+#pragma unroll
+    for (int j = 0; j < Elem<T>::VEC; ++j) acc[j] += f[j];
+}
+
 // Which of this lane's accesses lie inside a row of `pieces` 16-byte pieces.
 template <typename G>
 struct LaneMask {
@@ -50,13 +107,62 @@ struct LaneMask {
     }
 };
 
+// One row of `bytes` bytes in memory, its address wave-uniform (one row per wavefront): a buffer resource that ends
+// where the row does, so accesses of the padded geometry past its end read zeros and write nothing without a branch.
+template <int POLICY>
+struct BoundedRow {
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t off;
+    __device__ __forceinline__ BoundedRow(const void *base, uint32_t bytes, int l) : off(l * 16) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0, bytes,
+                                                 RowWriter<1>::kRawDwords);
+    }
+    __device__ __forceinline__ u32x4 get(int piece) const {
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + piece * 16, 0, POLICY);
+    }
+    __device__ __forceinline__ void put(int piece, const u32x4 &v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off + piece * 16, 0, POLICY);
+    }
+};
+
+// The rows of one wavefront step: full wavefronts read their one row through a bounded resource, narrower rows
+// through per-lane addresses.  row_base is the lane's row.
 template <typename G>
 __device__ __forceinline__ void load_row(u32x4 (&dst)[G::CHUNKS], const void *row_base, int l, bool ok,
-                                         const LaneMask<G> &m) {
-    const u32x4 *p = reinterpret_cast<const u32x4 *>(row_base) + l;
+                                         const LaneMask<G> &m, uint32_t bytes) {
+    if constexpr (G::LANES == kWaveSize) {
+        const BoundedRow<kLoad> row(row_base, ok ? bytes : 0, l);
 #pragma unroll
-    for (int k = 0; k < G::CHUNKS; ++k) dst[k] = (ok && m.in[k]) ? load16_stream(p + k * G::LANES) : u32x4{0, 0, 0, 0};
+        for (int k = 0; k < G::CHUNKS; ++k) dst[k] = row.get(k * G::LANES);
+    } else {
+        const u32x4 *p = reinterpret_cast<const u32x4 *>(row_base) + l;
+#pragma unroll
+        for (int k = 0; k < G::CHUNKS; ++k) dst[k] = (ok && m.in[k]) ? load16_stream(p + k * G::LANES) : u32x4{0, 0, 0, 0};
+    }
 }
+
+// Writes of one wavefront step: `first` is the wavefront's first row, lane_bytes the distance to the lane's piece.
+template <typename G, int THROUGH, int POLICY>
+struct RowOut {
+    static constexpr bool kBounded = G::LANES == kWaveSize;
+    std::conditional_t<kBounded, BoundedRow<POLICY>, RowWriter<THROUGH>> w;
+    __device__ __forceinline__ RowOut(void *first, uint32_t lane_bytes, int l, uint32_t bytes)
+        : w([&] {
+              if constexpr (kBounded)
+                  return BoundedRow<POLICY>(first, bytes, l);
+              else
+                  return RowWriter<THROUGH>(first, lane_bytes);
+          }()) {}
+    __device__ __forceinline__ void put(int k, bool ok, const LaneMask<G> &m, const u32x4 &v) const {
+        if constexpr (kBounded)
+            w.put(k * G::LANES, v);
+        else if (ok && m.in[k])
+            w.put(k * G::LANES, v);
+    }
+};
 
 template <typename G>
 __device__ __forceinline__ void load_param(u32x4 (&dst)[G::CHUNKS], const void *base, int l, const LaneMask<G> &m) {
@@ -66,8 +172,9 @@ __device__ __forceinline__ void load_param(u32x4 (&dst)[G::CHUNKS], const void *
 }
 
 // Workgroup-level flush of per-lane column sums: rows of a wavefront folded by
-// shuffles, wavefronts added into LDS in wavefront order, one fp32 row of
-// NSETS*C partial sums written out.  lds holds NSETS*C floats.
+// shuffles; then, one set at a time, every wavefront deposits its sums in an LDS region
+// of its own and all threads add the four regions in wavefront order into the fp32 row of
+// NSETS*C partial sums.  lds holds kRowWaves*C floats.
 template <typename G, int NSETS>
 __device__ __forceinline__ void flush_partials_anywidth(float (&acc)[NSETS][G::CHUNKS][G::VEC],
                                                         float *__restrict__ partial_row, float *lds, int C,
@@ -83,21 +190,35 @@ __device__ __forceinline__ void flush_partials_anywidth(float (&acc)[NSETS][G::C
         for (int k = 0; k < CHUNKS; ++k)
 #pragma unroll
             for (int j = 0; j < VEC; ++j) acc[s][k][j] = fold_rows_of_wave<LANES>(acc[s][k][j]);
-    for (int wv = 0; wv < kRowWaves; ++wv) {
-        if (wave == wv && sub == 0) {
 #pragma unroll
-            for (int s = 0; s < NSETS; ++s)
+    for (int s = 0; s < NSETS; ++s) {
+        if (s > 0) __syncthreads();  // the set before has been read
+        if (sub == 0) {
 #pragma unroll
-                for (int k = 0; k < CHUNKS; ++k) {
-                    if (!m.in[k]) continue;
-                    float *p = lds + s * C + (k * LANES + l) * VEC;
+            for (int k = 0; k < CHUNKS; ++k) {
+                if (!m.in[k]) continue;
+                float *p = lds + wave * C + (k * LANES + l) * VEC;
 #pragma unroll
-                    for (int j = 0; j < VEC; ++j) p[j] = (wv == 0) ? acc[s][k][j] : p[j] + acc[s][k][j];
+                for (int q = 0; q < VEC / 4; ++q) {
+                    // copies the compiler cannot see through: a 16-byte store must not pin the accumulators to
+                    // groups of four consecutive registers for the whole kernel
+                    float a0 = acc[s][k][4 * q], a1 = acc[s][k][4 * q + 1], a2 = acc[s][k][4 * q + 2], a3 = acc[s][k][4 * q + 3];
+                    asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3));
+                    *reinterpret_cast<u32x4 *>(p + 4 * q) = u32x4{as_u32(a0), as_u32(a1), as_u32(a2), as_u32(a3)};
                 }
+            }
         }
         __syncthreads();
+        for (int i = threadIdx.x; i < C / 4; i += kRowThreads) {
+            u32x4 part[kRowWaves], sum;
+#pragma unroll
+            for (int w = 0; w < kRowWaves; ++w) part[w] = *reinterpret_cast<const u32x4 *>(lds + w * C + 4 * i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                sum[j] = as_u32(((as_f32(part[0][j]) + as_f32(part[1][j])) + as_f32(part[2][j])) + as_f32(part[3][j]));
+            *reinterpret_cast<u32x4 *>(partial_row + s * C + 4 * i) = sum;
+        }
     }
-    for (int i = threadIdx.x; i < NSETS * C; i += kRowThreads) partial_row[i] = lds[i];
 }
 
 // ------------------------------------------------------------------ RMSNorm
@@ -114,6 +235,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_fwd_kernel(
     const int l = lane % LANES;
     const int wave = wave_id_in_block();
     const LaneMask<G> m(l, C / VEC);
+    const uint32_t row_bytes = (uint32_t)(C * (int)sizeof(T));
 
     u32x4 wr[CHUNKS];
     load_param<G>(wr, w, l, m);
@@ -126,7 +248,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_fwd_kernel(
         const int64_t row = at.row;
         const bool ok = at.ok;
         u32x4 xr[CHUNKS];
-        load_row<G>(xr, x + at.xoff, l, ok, m);
+        load_row<G>(xr, x + at.xoff, l, ok, m, row_bytes);
 
         float ss = 0.0f;
 #pragma unroll
@@ -141,8 +263,8 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_fwd_kernel(
         if (ok && l == 0) rstd[row] = r;
 
         // the wavefront's rows are consecutive in out: base = its first row
-        const RowWriter<TTN_ANY_FWD_STORE> wo(out + map.template locate<RPW>(grp, 0, C).row * C,
-                                              (uint32_t)(sub * C * (int)sizeof(T)) + l * 16);
+        const RowOut<G, TTN_ANY_FWD_STORE, kFwdStore> wo(out + map.template locate<RPW>(grp, 0, C).row * C,
+                                              (uint32_t)(sub * C * (int)sizeof(T)) + l * 16, l, row_bytes);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
             float v[VEC], wv[VEC];
@@ -153,7 +275,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_fwd_kernel(
             E::round(v);  // y = normalised row in the element type
 #pragma unroll
             for (int j = 0; j < VEC; ++j) v[j] *= wv[j];
-            if (ok && m.in[k]) wo.put(k * LANES, E::pack(v));
+            wo.put(k, ok, m, E::pack(v));
         }
     }
 }
@@ -165,12 +287,13 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_bwd_kernel(
     using G = PadGeom<T, LANES, CHUNKS>;
     using E = Elem<T>;
     constexpr int VEC = G::VEC, RPW = G::RPW;
-    extern __shared__ float lds[];
+    extern __shared__ __align__(16) float lds[];
     const int lane = threadIdx.x & 63;
     const int sub = lane / LANES;
     const int l = lane % LANES;
     const int wave = wave_id_in_block();
     const LaneMask<G> m(l, C / VEC);
+    const uint32_t row_bytes = (uint32_t)(C * (int)sizeof(T));
 
     u32x4 wr[CHUNKS];
     load_param<G>(wr, w, l, m);
@@ -180,66 +303,69 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_bwd_kernel(
 #pragma unroll
         for (int j = 0; j < VEC; ++j) acc[0][k][j] = 0.0f;
 
+    struct Row {
+        u32x4 g[CHUNKS], x[CHUNKS];
+        float r;
+        RowAddr at;
+        int64_t doff0;
+    };
     const int64_t groups = map.template groups<RPW>();
     const int64_t stride = (int64_t)gridDim.x * kRowWaves;
-    for (int64_t grp = (int64_t)blockIdx.x * kRowWaves + wave; grp < groups; grp += stride) {
+    auto fetch = [&](Row &b, int64_t grp) {
+        b.at = map.template locate<RPW>(grp, sub, C);
+        b.doff0 = map.template locate<RPW>(grp, 0, C).doff;
+        load_row<G>(b.g, g + b.at.row * C, l, b.at.ok, m, row_bytes);
+        load_row<G>(b.x, x + b.at.xoff, l, b.at.ok, m, row_bytes);
+        b.r = b.at.ok ? rstd[b.at.row] : 0.0f;
+    };
+    auto process = [&](Row &b, auto &&between_passes) {
         keep_packed(wr);
-        const RowAddr at = map.template locate<RPW>(grp, sub, C);
-        const int64_t row = at.row;
-        const bool ok = at.ok;
-        u32x4 gr[CHUNKS], xr[CHUNKS];
-        load_row<G>(gr, g + row * C, l, ok, m);
-        load_row<G>(xr, x + at.xoff, l, ok, m);
-        const float r = ok ? rstd[row] : 0.0f;
-
+        const float r = b.r;
         // pass 1: gy = rnd(g*w) kept packed; row dot  sum_c gy * x
         u32x4 gyp[CHUNKS];
         float dot = 0.0f;
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            float gv[VEC], wv[VEC], xv[VEC];
-            E::unpack(gr[k], gv);
-            E::unpack(wr[k], wv);
+            gyp[k] = packed_products<T>(b.g[k], wr[k]);
+            if constexpr (kHasDot2<T>) {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) gv[j] *= wv[j];
-            gyp[k] = E::pack(gv);
-            E::unpack(gyp[k], gv);
-            E::unpack(xr[k], xv);
+                for (int i = 0; i < 4; ++i) dot = dot2<T>(gyp[k][i], b.x[k][i], dot);
+            } else {
+                float gy[VEC], xv[VEC];
+                E::unpack(gyp[k], gy);
+                E::unpack(b.x[k], xv);
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) dot = fmaf(gv[j], xv[j], dot);
+                for (int j = 0; j < VEC; ++j) dot = fmaf(gy[j], xv[j], dot);
+            }
         }
         dot = group_sum<LANES>(dot);
+        between_passes();
         // dx = r*(gy - xhat * mean_c(gy*xhat)) = gy*r + x*coef
         const float coef = -((dot / (float)C) * r * r * r);
         // the second pass unpacks the row again rather than holding pass 1's fp32 copies live
-        keep_packed(gr);
-        keep_packed(xr);
+        keep_packed(b.g);
+        keep_packed(b.x);
         keep_packed(gyp);
 
         // dx goes through its own strides: base = the wavefront's first row, the lane adds its row's distance
-        const int64_t doff0 = map.template locate<RPW>(grp, 0, C).doff;
-        const RowWriter<(TTN_ANY_BWD_STORE && CHUNKS <= 6)> wd(
-            dx + doff0, (uint32_t)((at.doff - doff0) * (int64_t)sizeof(T)) + l * 16);
+        const RowOut<G, (TTN_ANY_BWD_STORE && CHUNKS <= 6), kBwdStore> wd(
+            dx + b.doff0, (uint32_t)((b.at.doff - b.doff0) * (int64_t)sizeof(T)) + l * 16, l, row_bytes);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            float gv[VEC], gy[VEC], xv[VEC], o[VEC], y[VEC];
-            E::unpack(gr[k], gv);
+            float gy[VEC], xv[VEC], o[VEC], y[VEC];
             E::unpack(gyp[k], gy);
-            E::unpack(xr[k], xv);
+            E::unpack(b.x[k], xv);
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
                 o[j] = fmaf(xv[j], coef, gy[j] * r);
                 y[j] = xv[j] * r;
             }
-            if (ok && m.in[k]) wd.put(k * LANES, E::pack(o));
-            E::round(y);  // y = normalised row in the element type
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) y[j] *= gv[j];
-            E::round(y);  // g*y materialised in the element type before the column sum
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) acc[0][k][j] += y[j];
+            wd.put(k, b.at.ok, m, E::pack(o));
+            add_columns<T>(acc[0][k], packed_products<T>(b.g[k], E::pack(y)));  // dw += rnd(g * rnd(y))
         }
-    }
+    };
+    row_pipeline<CHUNKS <= 6 ? 2 : 1, true, Row>(
+        (int64_t)blockIdx.x * kRowWaves + wave, groups, stride, fetch, process);
     flush_partials_anywidth<G, 1>(acc, partial + (int64_t)blockIdx.x * C, lds, C, m);
 }
 
@@ -263,9 +389,24 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
     const int64_t b = blockIdx.x / blocks_per_sample;  // sample this workgroup serves
     const int slot = blockIdx.x % blocks_per_sample;
     const LaneMask<G> m(l, C / VEC);
+    const uint32_t row_bytes = (uint32_t)(C * (int)sizeof(T));
 
     u32x4 tr[CHUNKS], hr[CHUNKS];
     [[maybe_unused]] u32x4 qr[GATED ? CHUNKS : 1];
+
+    const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
+    const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
+    const uint32_t lane_bytes = (uint32_t)(sub * lay.row_stride * C * (int64_t)sizeof(T)) + l * 16;
+    u32x4 xr[CHUNKS];
+    [[maybe_unused]] u32x4 ar[GATED ? CHUNKS : 1];
+    auto fetch = [&](u32x4 (&dx)[CHUNKS], u32x4 (&da)[GATED ? CHUNKS : 1], int64_t i) {
+        const int64_t rs = i * RPW + sub;
+        const int64_t at = lay.row(b, rs) * C;
+        load_row<G>(dx, x + at, l, rs < rows_per_sample, m, row_bytes);
+        if constexpr (GATED) load_row<G>(da, attn + at, l, rs < rows_per_sample, m, row_bytes);
+    };
+    int64_t grp = (int64_t)slot * kRowWaves + wave;
+    if (grp < groups) fetch(xr, ar, grp);
     load_param<G>(tr, scale + b * C, l, m);
     load_param<G>(hr, shift + b * C, l, m);
     if constexpr (GATED) load_param<G>(qr, gate + b * C, l, m);
@@ -278,9 +419,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
         tr[k] = E::pack(v);
     }
 
-    const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
-    const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
-    for (int64_t grp = (int64_t)slot * kRowWaves + wave; grp < groups; grp += stride) {
+    for (; grp < groups; grp += stride) {
         keep_packed(tr);
         keep_packed(hr);
         if constexpr (GATED) keep_packed(qr);
@@ -288,13 +427,8 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
         const bool ok = rs < rows_per_sample;
         const int64_t row = lay.row(b, rs);
         const int64_t first = lay.row(b, grp * RPW) * C;  // the wavefront's first row: base of what it writes
-        const uint32_t lane_bytes = (uint32_t)(sub * lay.row_stride * C * (int64_t)sizeof(T)) + l * 16;
-        u32x4 xr[CHUNKS];
-        load_row<G>(xr, x + row * C, l, ok, m);
         if constexpr (GATED) {
-            u32x4 ar[CHUNKS];
-            load_row<G>(ar, attn + row * C, l, ok, m);
-            const RowWriter<TTN_ANY_FWD_STORE> wh(h2_out + first, lane_bytes);
+            const RowOut<G, TTN_ANY_FWD_STORE, kFwdStore> wh(h2_out + first, lane_bytes, l, row_bytes);
 #pragma unroll
             for (int k = 0; k < CHUNKS; ++k) {
                 float hv[VEC], av[VEC], gv[VEC];
@@ -307,17 +441,22 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) hv[j] += av[j];
                 xr[k] = E::pack(hv);  // h2: the new residual stream, and the row that is normalised
-                if (ok && m.in[k]) wh.put(k * LANES, xr[k]);
+                wh.put(k, ok, m, xr[k]);
             }
         }
 
         float s = 0.0f;
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            float v[VEC];
-            E::unpack(xr[k], v);
+            if constexpr (kHasDot2<T>) {  // row sum straight from the packed pairs
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) s += v[j];
+                for (int i = 0; i < 4; ++i) s = dot2<T>(xr[k][i], kOnesPair<T>, s);
+            } else {
+                float v[VEC];
+                E::unpack(xr[k], v);
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) s += v[j];
+            }
         }
         const float mu = group_sum<LANES>(s) / (float)C;
         float q = 0.0f;
@@ -339,8 +478,12 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
             rstd[row] = r;
         }
 
+        u32x4 xn[CHUNKS];  // the next row, requested before this one's output pass
+        [[maybe_unused]] u32x4 an[GATED ? CHUNKS : 1];
+        if (grp + stride < groups) fetch(xn, an, grp + stride);
+
         const float nmr = -(mu * r);
-        const RowWriter<TTN_ANY_FWD_STORE> wo(out + first, lane_bytes);
+        const RowOut<G, TTN_ANY_FWD_STORE, kFwdStore> wo(out + first, lane_bytes, l, row_bytes);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
             float v[VEC], tv[VEC], hv[VEC];
@@ -355,7 +498,13 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
             E::round(v);  // xn * (1 + scale)
 #pragma unroll
             for (int j = 0; j < VEC; ++j) v[j] += hv[j];
-            if (ok && m.in[k]) wo.put(k * LANES, E::pack(v));
+            wo.put(k, ok, m, E::pack(v));
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) xr[k] = xn[k];
+        if constexpr (GATED) {
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k) ar[k] = an[k];
         }
     }
 }
@@ -371,17 +520,12 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
     T *__restrict__ da, const T *__restrict__ e, const T *__restrict__ attn, const T *__restrict__ gate,
     int64_t rows_per_sample, const SampleLayout lay, int blocks_per_sample, int C) {
     static_assert(!(GATED && RES), "the gated form handles e itself");
-    static_assert(!(GATED || RES) || CHUNKS <= 6, "the gated and residual forms are built for rows of up to six accesses per lane");
+    static_assert(CHUNKS <= 6, "wider dense rows run on the wide-row kernels");
     constexpr int NSETS = GATED ? 3 : 2;
     using G = PadGeom<T, LANES, CHUNKS>;
     using E = Elem<T>;
     constexpr int VEC = G::VEC, RPW = G::RPW;
-    // the widest rows have no registers left for the modulation row: it is staged in LDS, in the
-    // area the final flush uses afterwards
-    constexpr bool kParamInRegs = CHUNKS <= 8;
-    // ... nor for gx = rnd(g*t) between the two passes: it is formed again (same rounding, same value)
-    constexpr bool kKeepGx = CHUNKS * VEC <= 64;
-    extern __shared__ float lds[];
+    extern __shared__ __align__(16) float lds[];
     const int lane = threadIdx.x & 63;
     const int sub = lane / LANES;
     const int l = lane % LANES;
@@ -389,26 +533,19 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
     const int64_t b = blockIdx.x / blocks_per_sample;
     const int slot = blockIdx.x % blocks_per_sample;
     const LaneMask<G> m(l, C / VEC);
+    const uint32_t row_bytes = (uint32_t)(C * (int)sizeof(T));
 
-    auto one_plus = [](const u32x4 &raw) -> u32x4 {  // t = rnd(1 + scale)
+    u32x4 tr[CHUNKS];  // t = rnd(1 + scale[sample])
+    load_param<G>(tr, scale + b * C, l, m);
+#pragma unroll
+    for (int k = 0; k < CHUNKS; ++k) {
         float v[VEC];
-        E::unpack(raw, v);
+        E::unpack(tr[k], v);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
-        return E::pack(v);
-    };
-    u32x4 tr[kParamInRegs ? CHUNKS : 1];
-    [[maybe_unused]] u32x4 qr[GATED ? CHUNKS : 1];
-    u32x4 *lds_t = reinterpret_cast<u32x4 *>(lds);  // shares the flush area: dead before the flush starts
-    if constexpr (kParamInRegs) {
-        load_param<G>(tr, scale + b * C, l, m);
-#pragma unroll
-        for (int k = 0; k < CHUNKS; ++k) tr[k] = one_plus(tr[k]);
-    } else {
-        for (int i = threadIdx.x; i < C / VEC; i += kRowThreads)
-            lds_t[i] = one_plus(load16(reinterpret_cast<const u32x4 *>(scale + b * C) + i));
-        __syncthreads();
+        tr[k] = E::pack(v);
     }
+    [[maybe_unused]] u32x4 qr[GATED ? CHUNKS : 1];
     if constexpr (GATED) load_param<G>(qr, gate + b * C, l, m);
 
     float acc[NSETS][CHUNKS][VEC];  // [0] = dscale, [1] = dshift, [2] = dgate
@@ -419,56 +556,51 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
 #pragma unroll
             for (int j = 0; j < VEC; ++j) acc[s][k][j] = 0.0f;
 
+    struct Row {
+        u32x4 g[CHUNKS], x[CHUNKS];
+        u32x4 e[(GATED || RES) ? CHUNKS : 1], a[GATED ? CHUNKS : 1];
+        float r, mu;
+        int64_t first;  // element offset of the wavefront's first row
+        bool ok;
+    };
     const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
     const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
-    for (int64_t grp = (int64_t)slot * kRowWaves + wave; grp < groups; grp += stride) {
-        if constexpr (kParamInRegs) keep_packed(tr);
-        if constexpr (GATED) keep_packed(qr);
+    const uint32_t lane_bytes = (uint32_t)(sub * lay.row_stride * C * (int64_t)sizeof(T)) + l * 16;
+    auto fetch = [&](Row &q, int64_t grp) {
         const int64_t rs = grp * RPW + sub;
-        const bool ok = rs < rows_per_sample;
+        q.ok = rs < rows_per_sample;
         const int64_t row = lay.row(b, rs);
-        const int64_t first = lay.row(b, grp * RPW) * C;
-        const uint32_t lane_bytes = (uint32_t)(sub * lay.row_stride * C * (int64_t)sizeof(T)) + l * 16;
-        u32x4 gr[CHUNKS], xr[CHUNKS];
-        [[maybe_unused]] u32x4 er[(GATED || RES) ? CHUNKS : 1], ar[GATED ? CHUNKS : 1];
-        load_row<G>(gr, g + row * C, l, ok, m);
-        load_row<G>(xr, x + row * C, l, ok, m);
-        if constexpr (GATED || RES) load_row<G>(er, e + row * C, l, ok && e != nullptr, m);
-        if constexpr (GATED) load_row<G>(ar, attn + row * C, l, ok, m);
-        const float r = ok ? rstd[row] : 0.0f;
-        const float mu = ok ? mean[row] : 0.0f;
+        q.first = lay.row(b, grp * RPW) * C;
+        load_row<G>(q.g, g + row * C, l, q.ok, m, row_bytes);
+        load_row<G>(q.x, x + row * C, l, q.ok, m, row_bytes);
+        if constexpr (GATED || RES) load_row<G>(q.e, e + row * C, l, q.ok && e != nullptr, m, row_bytes);
+        if constexpr (GATED) load_row<G>(q.a, attn + row * C, l, q.ok, m, row_bytes);
+        const int64_t srow = LANES == kWaveSize ? wave_uniform(row) : row;
+        q.r = q.ok ? rstd[srow] : 0.0f;
+        q.mu = q.ok ? mean[srow] : 0.0f;
+    };
+    auto process = [&](Row &q, auto &&between_passes) {
+        keep_packed(tr);
+        const float r = q.r, mu = q.mu;
         const float nmr = -(mu * r);  // xhat = x*r + nmr
-
-        auto gx_of = [&](int k) -> u32x4 {  // rnd(g * t) for access k, in the element type
-            float gv[VEC], tv[VEC];
-            E::unpack(gr[k], gv);
-            if constexpr (kParamInRegs)
-                E::unpack(tr[k], tv);
-            else
-                E::unpack(m.in[k] ? lds_t[k * LANES + l] : u32x4{0, 0, 0, 0}, tv);
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) gv[j] *= tv[j];
-            return E::pack(gv);
-        };
-        // pass 1: gx = rnd(g*t); s1 = sum_c gx; s2 = sum_c gx * xhat
-        u32x4 gxp[kKeepGx ? CHUNKS : 1];
+        // pass 1: gx = rnd(g*t) kept packed; s1 = sum_c gx; s2 = sum_c gx * xhat
+        // (padding: g = 0 there, so gx = 0 and neither sum sees xhat = nmr)
+        u32x4 gxp[CHUNKS];
         float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            const u32x4 gxk = gx_of(k);
-            if constexpr (kKeepGx) gxp[k] = gxk;
-            // padding: g = 0 there, so gx = 0 and neither sum sees xhat = nmr
+            gxp[k] = packed_products<T>(q.g[k], tr[k]);
             if constexpr (kHasDot2<T>) {
                 // straight from the packed pairs; s2 holds sum_c gx * x here, turned into sum_c gx * xhat below
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    s1 = dot2<T>(gxk[i], kOnesPair<T>, s1);
-                    s2 = dot2<T>(gxk[i], xr[k][i], s2);
+                    s1 = dot2<T>(gxp[k][i], kOnesPair<T>, s1);
+                    s2 = dot2<T>(gxp[k][i], q.x[k][i], s2);
                 }
             } else {
                 float gv[VEC], xv[VEC];
-                E::unpack(gxk, gv);
-                E::unpack(xr[k], xv);
+                E::unpack(gxp[k], gv);
+                E::unpack(q.x[k], xv);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) {
                     s1 += gv[j];
@@ -478,68 +610,61 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
         }
         s1 = group_sum<LANES>(s1);
         s2 = group_sum<LANES>(s2);
+        between_passes();
         if constexpr (kHasDot2<T>) s2 = r * (s2 - mu * s1);
         const float m1 = s1 / (float)C, m2 = s2 / (float)C;
         // dx = r*(gx - m1 - xhat*m2) = r*gx + x*K1 + K0
         const float k1 = -(r * m2), k0 = -(r * m1);
         const float K1 = k1 * r;
         const float K0 = fmaf(k1, nmr, k0);
-        // the second pass unpacks the row again rather than holding pass 1's fp32 copies live
-        keep_packed(gr);
-        keep_packed(xr);
-        if constexpr (kKeepGx) keep_packed(gxp);
 
-        constexpr int kDxStore = (TTN_ANY_BWD_STORE && CHUNKS <= 6 && !GATED);
-        const RowWriter<kDxStore> wd(dx + first, lane_bytes);
-        const RowWriter<0> wa(GATED ? da + first : nullptr, lane_bytes);
+        // the second pass unpacks the row again rather than holding pass 1's fp32 copies live
+        keep_packed(q.g);
+        keep_packed(q.x);
+        keep_packed(gxp);
+        const RowOut<G, (TTN_ANY_BWD_STORE && !GATED), kBwdStore> wd(dx + q.first, lane_bytes, l, row_bytes);
+        const RowOut<G, 0, kBwdStore> wa(GATED ? da + q.first : nullptr, lane_bytes, l, row_bytes);
+        if constexpr (GATED) keep_packed(qr);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            float gv[VEC], gx[VEC], xv[VEC], o[VEC], xn[VEC];
-            E::unpack(gr[k], gv);
-            if constexpr (kKeepGx)
-                E::unpack(gxp[k], gx);
-            else
-                E::unpack(gx_of(k), gx);
-            E::unpack(xr[k], xv);
+            float gx[VEC], xv[VEC], o[VEC], xn[VEC];
+            E::unpack(gxp[k], gx);
+            E::unpack(q.x[k], xv);
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
                 o[j] = fmaf(r, gx[j], fmaf(xv[j], K1, K0));
                 xn[j] = centred<T>(xv[j], mu, r, nmr);
-                acc[1][k][j] += gv[j];
             }
             if constexpr (GATED || RES) {
                 float ev[VEC];
                 E::round(o);  // the norm's dx, materialised in the element type
-                E::unpack(er[k], ev);
+                E::unpack(q.e[k], ev);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) o[j] += ev[j];
             }
             const u32x4 dxp = E::pack(o);
-            if (ok && m.in[k]) wd.put(k * LANES, dxp);
+            wd.put(k, q.ok, m, dxp);
             if constexpr (GATED) {
                 float av[VEC], qv[VEC];
                 E::unpack(dxp, o);  // dh as stored
-                E::unpack(ar[k], av);
+                E::unpack(q.a[k], av);
                 E::unpack(qr[k], qv);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) {
                     qv[j] *= o[j];
                     av[j] *= o[j];
                 }
-                if (ok && m.in[k]) wa.put(k * LANES, E::pack(qv));
+                wa.put(k, q.ok, m, E::pack(qv));
                 E::round(av);  // dh*attn materialised in the element type before the column sum
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) acc[2][k][j] += av[j];
             }
-            E::round(xn);  // the normalised row in the element type
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) xn[j] *= gv[j];
-            E::round(xn);  // g*xn materialised in the element type before the column sum
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) acc[0][k][j] += xn[j];
+            add_columns<T>(acc[1][k], q.g[k]);                                    // dshift += g (padding: g = 0)
+            add_columns<T>(acc[0][k], packed_products<T>(q.g[k], E::pack(xn)));  // dscale += rnd(g * rnd(xhat))
         }
-    }
-    if constexpr (!kParamInRegs) __syncthreads();  // every wavefront is done reading lds_t
+    };
+    row_pipeline<GATED ? 1 : 2, true, Row>((int64_t)slot * kRowWaves + wave, groups, stride, fetch,
+                                                                     process);
     flush_partials_anywidth<G, NSETS>(acc, partial + (int64_t)blockIdx.x * (NSETS * C), lds, C, m);
 }
 
@@ -562,14 +687,14 @@ static GeomChoice choose_geometry(int pieces) {
     if (pieces <= 16) return {16, 1};
     if (pieces <= 32) return {32, 1};
     const int need = (pieces + 63) / 64;
-    for (int c : {1, 2, 3, 4, 6, 8, 12, 16})
+    for (int c : {1, 2, 3, 4, 5, 6, 8, 12, 16})
         if (need <= c) return {64, c};
     return {0, 0};
 }
 
 // Calls F<T, LANES, CHUNKS>::run(args...) for the run-time (dtype, geometry).
 #define TTN_ANYWIDTH_GEOMS(X, T) \
-    X(T, 8, 1) X(T, 16, 1) X(T, 32, 1) X(T, 64, 1) X(T, 64, 2) X(T, 64, 3) X(T, 64, 4) X(T, 64, 6) X(T, 64, 8) X(T, 64, 12) X(T, 64, 16)
+    X(T, 8, 1) X(T, 16, 1) X(T, 32, 1) X(T, 64, 1) X(T, 64, 2) X(T, 64, 3) X(T, 64, 4) X(T, 64, 5) X(T, 64, 6) X(T, 64, 8) X(T, 64, 12) X(T, 64, 16)
 
 template <template <typename, int, int> class F, typename... Args>
 static int dispatch(int dtype, GeomChoice gc, Args... args) {
@@ -587,24 +712,32 @@ static int dispatch(int dtype, GeomChoice gc, Args... args) {
 }
 
 // Launch policy.  Forward: narrow rows (one access per lane) use a persistent grid of 16 workgroups
-// per compute unit, wider rows one row per wavefront.  Backward is persistent (column sums live in
-// registers); the grid shrinks as rows widen so that each compute unit keeps about the same number
-// of bytes in flight.
+// per compute unit, wider rows one row per wavefront (AdaLN: up to TTN_ANY_ADALN_FWD_ROWS).  Backward is
+// persistent (column sums live in registers); the grid shrinks as rows widen so that each compute unit
+// keeps about the same number of bytes in flight.
 constexpr int kOneShotAny = 1 << 20;
 static int fwd_blocks_per_cu(int chunks) { return chunks == 1 ? 16 : kOneShotAny; }
-static int bwd_blocks_per_cu(int chunks) { return chunks >= 6 ? 1 : (chunks >= 3 ? 2 : (chunks == 2 ? 3 : 6)); }
+static int bwd_blocks_per_cu(int chunks) {
+    constexpr int blocks[] = TTN_ANY_BWD_BLOCKS;
+    return chunks > 6 ? 1 : blocks[chunks - 1];
+}
 
 static GeomChoice geometry_for(int64_t cols, int dtype) {
     return choose_geometry((int)(cols / (16 / (int)elem_bytes(dtype))));
 }
 
 // Grid for (batch, rows_per_sample) under geometry gc; status != OK on failure.
-static int plan_for(RowPlan *plan, int64_t batch, int64_t rows_per_sample, GeomChoice gc, bool backward) {
+static int plan_for(RowPlan *plan, int64_t batch, int64_t rows_per_sample, GeomChoice gc, bool backward, int fwd_rows = 1) {
     int st = TT_NORM_OK;
     const int cus = current_device_cus(&st);
     if (st != TT_NORM_OK) return st;
     *plan = make_row_plan(batch, rows_per_sample, kWaveSize / gc.lanes,
                           backward ? bwd_blocks_per_cu(gc.chunks) : fwd_blocks_per_cu(gc.chunks), cus);
+    // below four workgroups per compute unit a second row would only lengthen the call (600 x 2048: 4.3 -> 6.1 us)
+    if (!backward && gc.chunks > 1 && plan->blocks >= (int64_t)cus * 4) {
+        plan->blocks_per_sample = (plan->blocks_per_sample + fwd_rows - 1) / fwd_rows;
+        plan->blocks = batch * plan->blocks_per_sample;
+    }
     if (plan->blocks > 0x7fffffffLL) return fail(TT_NORM_EINVAL, "grid too large");
     return TT_NORM_OK;
 }
@@ -627,7 +760,7 @@ struct RmsOn {  // the RMSNorm kernels over one kind of row map
                        const float *rstd, const Map &map, int C, hipStream_t stream) {
             RowKernelProfile prof(stream);
             anywidth_rmsnorm_bwd_kernel<T, LANES, CHUNKS, Map>
-                <<<dim3((unsigned)p.blocks), dim3(kRowThreads), (size_t)C * sizeof(float), stream>>>(
+                <<<dim3((unsigned)p.blocks), dim3(kRowThreads), (size_t)kRowWaves * C * sizeof(float), stream>>>(
                     (T *)dx, (float *)ws, (const T *)g, (const T *)x, (const T *)w, rstd, map, C);
             return TT_NORM_OK;
         }
@@ -648,8 +781,8 @@ struct AdalnOn {
         static int run(const RowPlan &p, void *out, float *mean, float *rstd, const void *x, const void *scale,
                        const void *shift, const AdalnExtra &ex, int64_t rows_per_sample, SampleLayout lay, int C,
                        double eps, hipStream_t stream) {
-            if constexpr (GATED && CHUNKS > 6) {
-                return fail(TT_NORM_EUNSUPPORTED, "gated residual + AdaLN: rows of more than six 16-byte accesses per lane");
+            if constexpr (CHUNKS > 6) {  // wider dense rows run on the wide-row kernels
+                return fail(TT_NORM_EUNSUPPORTED, "AdaLN: rows of more than six 16-byte accesses per lane");
             } else {
                 RowKernelProfile prof(stream);
                 anywidth_adaln_fwd_kernel<T, LANES, CHUNKS, GATED><<<dim3((unsigned)p.blocks), dim3(kRowThreads), 0, stream>>>(
@@ -664,13 +797,12 @@ struct AdalnOn {
         static int run(const RowPlan &p, void *dx, void *ws, const void *g, const void *x, const void *scale,
                        const float *mean, const float *rstd, const AdalnExtra &ex, int64_t rows_per_sample,
                        SampleLayout lay, int C, hipStream_t stream) {
-            if constexpr ((GATED || RES) && CHUNKS > 6) {
-                return fail(TT_NORM_EUNSUPPORTED, "gated / residual AdaLN backward: rows of more than six 16-byte accesses per lane");
+            if constexpr (CHUNKS > 6) {
+                return fail(TT_NORM_EUNSUPPORTED, "AdaLN backward: rows of more than six 16-byte accesses per lane");
             } else {
-                constexpr int NSETS = GATED ? 3 : 2;
                 RowKernelProfile prof(stream);
                 anywidth_adaln_bwd_kernel<T, LANES, CHUNKS, GATED, RES>
-                    <<<dim3((unsigned)p.blocks), dim3(kRowThreads), (size_t)NSETS * C * sizeof(float), stream>>>(
+                    <<<dim3((unsigned)p.blocks), dim3(kRowThreads), (size_t)kRowWaves * C * sizeof(float), stream>>>(
                         (T *)dx, (float *)ws, (const T *)g, (const T *)x, (const T *)scale, mean, rstd,
                         (T *)ex.h2_or_da, (const T *)ex.e, (const T *)ex.attn, (const T *)ex.gate, rows_per_sample,
                         lay, p.blocks_per_sample, C);
@@ -694,7 +826,7 @@ static int rmsnorm_forward_on(void *out, float *rstd, const void *x, const void 
 
 int anywidth_rmsnorm_forward(void *out, float *rstd, const void *x, const void *w, int64_t rows, int64_t cols,
                              double eps, int dtype, hipStream_t stream) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype)) return widerow_rmsnorm_forward(out, rstd, x, w, rows, cols, eps, dtype, stream);
+    if (widerow_takes(cols, dtype)) return widerow_rmsnorm_forward(out, rstd, x, w, rows, cols, eps, dtype, stream);
     return rmsnorm_forward_on(out, rstd, x, w, DenseRows{rows}, rows, cols, eps, dtype, stream);
 }
 
@@ -708,7 +840,7 @@ static size_t backward_scratch(int64_t batch, int64_t rows_per_sample, int64_t c
     RowPlan p;
     if (plan_for(&p, batch, rows_per_sample, geometry_for(cols, dtype), true) != TT_NORM_OK) return 0;
     size_t need = (size_t)p.blocks * nsets * cols * sizeof(float);
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype)) {  // dense rows take the other kernels, strided views these
+    if (widerow_takes(cols, dtype)) {  // dense rows take the other kernels, strided views these
         const size_t wide = widerow_backward_workspace_bytes(batch, rows_per_sample, cols, dtype, nsets);
         if (wide == 0) return 0;
         if (wide > need) need = wide;
@@ -744,7 +876,7 @@ static int rmsnorm_backward_on(void *dx, void *dw, const void *g, const void *x,
 int anywidth_rmsnorm_backward(void *dx, void *dw, const void *g, const void *x, const void *w,
                               const float *rstd, int64_t rows, int64_t cols, int dtype, void *ws,
                               size_t ws_bytes, hipStream_t stream) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype))
+    if (widerow_takes(cols, dtype))
         return widerow_rmsnorm_backward(dx, dw, g, x, w, rstd, rows, cols, dtype, ws, ws_bytes, stream);
     return rmsnorm_backward_on(dx, dw, g, x, w, rstd, DenseRows{rows}, rows, cols, dtype, ws, ws_bytes, stream);
 }
@@ -763,7 +895,7 @@ static SampleLayout layout_of(int64_t batch, int64_t rows_per_sample, bool seq_f
 bool anywidth_wide_forms_supported(int64_t cols, int dtype) {
     if (!anywidth_supported(cols, dtype)) return false;
     // rows of up to six accesses per lane here; wider dense rows on the wide-row kernels
-    return geometry_for(cols, dtype).chunks <= 6 || (TTN_WIDE_ROWS && widerow_takes(cols, dtype));
+    return geometry_for(cols, dtype).chunks <= 6 || widerow_takes(cols, dtype);
 }
 
 template <bool GATED>
@@ -773,7 +905,7 @@ static int adaln_forward_any(void *out, float *mean, float *rstd, const void *x,
     if (rows_per_sample == 0) return TT_NORM_OK;
     const GeomChoice gc = geometry_for(cols, dtype);
     RowPlan p;
-    int st = plan_for(&p, batch, rows_per_sample, gc, false);
+    int st = plan_for(&p, batch, rows_per_sample, gc, false, TTN_ANY_ADALN_FWD_ROWS);
     if (st != TT_NORM_OK) return st;
     st = dispatch<AdalnOn<GATED, false>::template Fwd>(dtype, gc, p, out, mean, rstd, x, scale, shift, ex, rows_per_sample,
                                                        layout_of(batch, rows_per_sample, seq_first), (int)cols, eps,
@@ -784,7 +916,7 @@ static int adaln_forward_any(void *out, float *mean, float *rstd, const void *x,
 int anywidth_adaln_forward(void *out, float *mean, float *rstd, const void *x, const void *scale,
                            const void *shift, int64_t batch, int64_t rows_per_sample, int64_t cols, double eps,
                            int dtype, hipStream_t stream, bool seq_first) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype))
+    if (widerow_takes(cols, dtype))
         return widerow_adaln_forward(out, mean, rstd, x, scale, shift, batch, rows_per_sample, cols, eps, dtype, seq_first,
                                      stream);
     return adaln_forward_any<false>(out, mean, rstd, x, scale, shift, AdalnExtra{nullptr, nullptr, nullptr, nullptr},
@@ -794,7 +926,7 @@ int anywidth_adaln_forward(void *out, float *mean, float *rstd, const void *x, c
 int anywidth_gated_adaln_forward(void *h2, void *out, float *mean, float *rstd, const void *h, const void *attn,
                                  const void *gate, const void *scale, const void *shift, int64_t batch,
                                  int64_t rows_per_sample, int64_t cols, double eps, int dtype, hipStream_t stream) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype))
+    if (widerow_takes(cols, dtype))
         return widerow_gated_adaln_forward(h2, out, mean, rstd, h, attn, gate, scale, shift, batch, rows_per_sample, cols,
                                            eps, dtype, stream);
     return adaln_forward_any<true>(out, mean, rstd, h, scale, shift, AdalnExtra{h2, nullptr, attn, gate}, batch,
@@ -834,7 +966,7 @@ int anywidth_adaln_backward(void *dx, void *dscale, void *dshift, const void *g,
                             const void *scale, const float *mean, const float *rstd, int64_t batch,
                             int64_t rows_per_sample, int64_t cols, int dtype, void *ws, size_t ws_bytes,
                             hipStream_t stream, bool seq_first) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype))
+    if (widerow_takes(cols, dtype))
         return widerow_adaln_backward(dx, dscale, dshift, g, x, scale, mean, rstd, batch, rows_per_sample, cols, dtype, ws,
                                       ws_bytes, seq_first, stream);
     return adaln_backward_any<false, false>(dx, dscale, dshift, nullptr, g, x, scale, mean, rstd,
@@ -846,7 +978,7 @@ int anywidth_adaln_backward_residual(void *dx, void *dscale, void *dshift, const
                                      const void *x, const void *scale, const float *mean, const float *rstd,
                                      int64_t batch, int64_t rows_per_sample, int64_t cols, int dtype, void *ws,
                                      size_t ws_bytes, hipStream_t stream) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype))
+    if (widerow_takes(cols, dtype))
         return widerow_adaln_backward_residual(dx, dscale, dshift, g, dres, x, scale, mean, rstd, batch, rows_per_sample,
                                                cols, dtype, ws, ws_bytes, stream);
     return adaln_backward_any<false, true>(dx, dscale, dshift, nullptr, g, x, scale, mean, rstd,
@@ -863,7 +995,7 @@ int anywidth_gated_adaln_backward(void *dh, void *dattn, void *dgate, void *dsca
                                   const void *scale, const float *mean, const float *rstd, int64_t batch,
                                   int64_t rows_per_sample, int64_t cols, int dtype, void *ws, size_t ws_bytes,
                                   hipStream_t stream) {
-    if (TTN_WIDE_ROWS && widerow_takes(cols, dtype))
+    if (widerow_takes(cols, dtype))
         return widerow_gated_adaln_backward(dh, dattn, dgate, dscale, dshift, g, dh2, h2, attn, gate, scale, mean, rstd,
                                             batch, rows_per_sample, cols, dtype, ws, ws_bytes, stream);
     return adaln_backward_any<true, false>(dh, dscale, dshift, dgate, g, h2, scale, mean, rstd,

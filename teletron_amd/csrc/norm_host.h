@@ -111,12 +111,6 @@ int anywidth_adaln_backward_residual(void *dx, void *dscale, void *dshift, const
                                      int64_t batch, int64_t rows_per_sample, int64_t cols, int dtype, void *ws,
                                      size_t ws_bytes, hipStream_t stream);
 
-// 1: dense rows of more than 384 pieces go to the kernels of widerow.hip (four wavefronts per row); 0: they stay
-// with the one-wavefront-per-row kernels of anywidth.hip (8, 12 or 16 accesses per lane), which strided views always use.
-#ifndef TTN_WIDE_ROWS
-#define TTN_WIDE_ROWS 1
-#endif
-
 // Measurement builds only (-DTTN_WAVE_CLOCK=1): sets the timestamp buffer of the kernels in adaln.hip.
 int adaln_set_wave_clock(void *buf);
 

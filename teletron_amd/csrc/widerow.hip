@@ -686,11 +686,11 @@ bool widerow_takes(int64_t cols, int dtype) {
 #define TTN_F32_3072_BWD_WIDE 1
 #endif
 bool gated_forward_on_wide_rows(int64_t cols, int dtype) {
-    return TTN_GATED_3072_WIDE && TTN_WIDE_ROWS && dtype != TT_NORM_F32 && cols == 3072;
+    return TTN_GATED_3072_WIDE && dtype != TT_NORM_F32 && cols == 3072;
 }
 bool dense_backward_on_wide_rows(int64_t cols, int dtype) {
-    if (TTN_16BIT_3072_BWD_WIDE && TTN_WIDE_ROWS && dtype != TT_NORM_F32 && cols == 3072) return true;
-    return TTN_F32_3072_BWD_WIDE && TTN_WIDE_ROWS && dtype == TT_NORM_F32 && cols == 3072;
+    if (TTN_16BIT_3072_BWD_WIDE && dtype != TT_NORM_F32 && cols == 3072) return true;
+    return TTN_F32_3072_BWD_WIDE && dtype == TT_NORM_F32 && cols == 3072;
 }
 
 // pieces per wavefront (a quarter of the row, rounded up) and the accesses per lane that takes

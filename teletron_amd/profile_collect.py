@@ -11,7 +11,7 @@ is the command that ran, on committed files only.
     python -m teletron_amd.profile_collect variants  --dir rocprof_out [--only base unpacked ...]
     python -m teletron_amd.profile_collect runs      --dir rocprof_out
     python -m teletron_amd.profile_collect cached    --dir rocprof_out
-    python -m teletron_amd.profile_collect wide      --dir rocprof_out [--only base onewave ...]
+    python -m teletron_amd.profile_collect wide      --dir rocprof_out [--only base bwd3 ...]
     python -m teletron_amd.profile_collect timeline  --dir rocprof_out
 
 This process never touches the GPU itself (it starts children and nothing else), every child runs under a

@@ -666,8 +666,6 @@ backward kernel.  Written by `python -m teletron_amd.profile_summary runs --dir 
 WIDE_WORKLOADS = ["w4096-bf16", "w5120-bf16", "w8192-bf16"]
 WIDE_VARIANTS = [  # name, flags, what: the choices of widerow.hip, each measured on the three wide workloads
     ("base", [], "the shipped kernels"),
-    ("onewave", ["-DTTN_WIDE_ROWS=0"],
-     "one wavefront per row (8, 12 or 16 accesses per lane): the any-width kernels, which strided views still use"),
     ("rmsfwd_persistent", ["-DTTN_WIDE_RMS_FWD_ROWS_PER_BLOCK=0"], "RMSNorm forward as a persistent grid instead of one-shot"),
     ("adalnfwd_oneshot", ["-DTTN_WIDE_ADALN_FWD_ROWS_PER_BLOCK=1"], "AdaLN forward one-shot (one row per workgroup)"),
     ("adalnfwd_persistent", ["-DTTN_WIDE_ADALN_FWD_ROWS_PER_BLOCK=0"], "AdaLN forward as a persistent grid"),
