@@ -388,7 +388,11 @@ struct RowWriter<1> {
                                                  kRawDwords);
     }
     __device__ __forceinline__ void put(int piece, const u32x4 &v) const {
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off, piece * 16, kSc1Nt);
+        // The piece goes into the vector offset, not into the scalar one: a 16-byte store must be followed by a wait
+        // state before its data registers are written again, and the compiler inserts it only for stores without a
+        // scalar offset register.  With one, rows of fp32 whose pieces are formed in the same registers had the first
+        // of a piece's four elements replaced by the next piece's, 784 of 25 million.
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off + piece * 16, 0, kSc1Nt);
     }
 };
 
