@@ -246,7 +246,78 @@ void torch_launch_gated_adaln_backward(torch::Tensor &dinp, torch::Tensor &dattn
              "tt_gated_residual_adaln_backward");
 }
 
+// ---- whole calls (see torch_glue.h) ----
+
+using Tensors = std::vector<torch::Tensor>;
+
+// Modulation rows of [B, cols] (or one row) that belong to x as it lies.
+static bool ready_modulation(const torch::Tensor &x, const torch::Tensor &scale, int64_t cols, bool seq_first) {
+    if (scale.numel() == 0 || scale.numel() % cols != 0) return false;
+    const int64_t batch = scale.numel() / cols;
+    if (seq_first) return x.dim() == 3 && x.size(1) == batch;
+    return batch == 1 || (x.dim() >= 2 && x.size(0) == batch);
+}
+
+// out, mean, inv_variance
+static c10::optional<Tensors> adaln_forward(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift,
+                                            int64_t cols, double epsilon, bool seq_first) {
+    if (!ready_rows(x, cols) || !ready(scale, x) || !ready(shift, x) || shift.numel() != scale.numel() ||
+        !ready_modulation(x, scale, cols, seq_first))
+        return c10::nullopt;
+    const int64_t rows = x.numel() / cols;
+    torch::Tensor out = at::empty_like(x), mean = row_statistics(x, rows), inv_variance = row_statistics(x, rows);
+    adaln_forward_stats_impl(out, x, scale, shift, rows, cols, epsilon, mean, inv_variance, seq_first);
+    return Tensors{out, mean, inv_variance};
+}
+
+// dinp, dscale, dshift; dres is the gradient the input receives from its other consumer, or None
+static c10::optional<Tensors> adaln_backward(const torch::Tensor &dout, const c10::optional<torch::Tensor> &dres,
+                                             const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &mean,
+                                             const torch::Tensor &inv_variance, int64_t cols, bool seq_first) {
+    const bool residual = dres.has_value() && dres->defined();
+    if (!ready(dout, x) || (residual && !ready(*dres, x))) return c10::nullopt;
+    const int64_t rows = x.numel() / cols;
+    torch::Tensor dinp = at::empty_like(x), dscale = at::empty_like(scale), dshift = at::empty_like(scale);
+    if (residual)
+        torch_launch_adaln_backward_residual(dinp, dscale, dshift, dout, *dres, x, scale, mean, inv_variance, rows, cols);
+    else
+        adaln_backward_impl(dinp, dscale, dshift, dout, x, scale, &mean, inv_variance, rows, cols, seq_first);
+    return Tensors{dinp, dscale, dshift};
+}
+
+// h2, out, mean, inv_variance
+static c10::optional<Tensors> gated_forward(const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
+                                            const torch::Tensor &scale, const torch::Tensor &shift, double epsilon) {
+    if (h.dim() < 1 || !ready_rows(h, h.size(-1)) || !ready(attn, h) || attn.sizes() != h.sizes()) return c10::nullopt;
+    const int64_t cols = h.size(-1);
+    for (auto *t : {&gate, &scale, &shift})
+        if (!ready(*t, h) || t->numel() != scale.numel()) return c10::nullopt;
+    if (!ready_modulation(h, scale, cols, false)) return c10::nullopt;
+    const int64_t rows = h.numel() / cols;
+    torch::Tensor h2 = at::empty_like(h), out = at::empty_like(h);
+    torch::Tensor mean = row_statistics(h, rows), inv_variance = row_statistics(h, rows);
+    torch_launch_gated_adaln_forward(h2, out, h, attn, gate, scale, shift, rows, cols, epsilon, mean, inv_variance);
+    return Tensors{h2, out, mean, inv_variance};
+}
+
+// dh, dattn, dgate, dscale, dshift; dh2 may be None
+static c10::optional<Tensors> gated_backward(const torch::Tensor &dout, const c10::optional<torch::Tensor> &dh2,
+                                             const torch::Tensor &h2, const torch::Tensor &attn, const torch::Tensor &gate,
+                                             const torch::Tensor &scale, const torch::Tensor &mean,
+                                             const torch::Tensor &inv_variance, int64_t cols) {
+    if (!ready(dout, h2) || (dh2.has_value() && dh2->defined() && !ready(*dh2, h2))) return c10::nullopt;
+    torch::Tensor dh = at::empty_like(h2), dattn = at::empty_like(h2);
+    torch::Tensor dgate = at::empty_like(scale), dscale = at::empty_like(scale), dshift = at::empty_like(scale);
+    torch_launch_gated_adaln_backward(dh, dattn, dgate, dscale, dshift, dout, dh2, h2, attn, gate, scale, mean, inv_variance,
+                                      h2.numel() / cols, cols);
+    return Tensors{dh, dattn, dgate, dscale, dshift};
+}
+
 PYBIND11_MODULE(fused_adaln, m) {
+    m.def("adaln_forward", &adaln_forward, "AdaLN forward: out, mean, inv_variance; None unless every operand is ready");
+    m.def("adaln_backward", &adaln_backward, "AdaLN backward: dinp, dscale, dshift; None unless every operand is ready");
+    m.def("gated_forward", &gated_forward, "gated residual update + AdaLN: h2, out, mean, inv_variance; or None");
+    m.def("gated_backward", &gated_backward, "its backward: dh, dattn, dgate, dscale, dshift; or None");
     m.def("torch_launch_adaln_backward_residual", &torch_launch_adaln_backward_residual,
           "AdaLN backward kernel with the input's other gradient added in");
     m.def("torch_launch_gated_adaln_forward", &torch_launch_gated_adaln_forward,

@@ -4,6 +4,8 @@
 // backward that works from the saved input.  Unlike the reference glue, every
 // argument is checked, the launch goes to PyTorch's current stream, and a
 // failed launch raises.
+#include <algorithm>
+
 #include "torch_glue.h"
 
 using namespace ttn_glue;
@@ -318,7 +320,83 @@ void torch_launch_qkv_rms_backward(torch::Tensor &dmixed, torch::Tensor &dweight
              "tt_qkv_rmsnorm_backward");
 }
 
+// ---- whole calls (see torch_glue.h) ----
+
+using Tensors = std::vector<torch::Tensor>;
+
+// Uninitialised tensor of x's shape laid out in x's dimension order but without its gaps.
+static torch::Tensor dense_like_layout(const torch::Tensor &x) {
+    std::vector<int64_t> order(x.dim()), sizes(x.dim()), place(x.dim());
+    for (int64_t d = 0; d < x.dim(); ++d) order[d] = d;
+    std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return x.stride(a) > x.stride(b); });
+    for (int64_t i = 0; i < x.dim(); ++i) {
+        sizes[i] = x.size(order[i]);
+        place[order[i]] = i;
+    }
+    return at::empty(sizes, x.options()).permute(place);
+}
+
+// out, inv_variance
+static c10::optional<Tensors> rms_forward(const torch::Tensor &x, const torch::Tensor &weight, int64_t cols, double epsilon) {
+    if (!ready_rows(x, cols) || !ready(weight, x) || weight.numel() != cols) return c10::nullopt;
+    const int64_t rows = x.numel() / cols;
+    torch::Tensor out = at::empty(x.sizes(), x.options()), inv_variance = row_statistics(x, rows);
+    torch_launch_rms_forward(out, x, weight, rows, cols, epsilon, inv_variance);
+    return Tensors{out, inv_variance};
+}
+
+// dinp, dweight
+static c10::optional<Tensors> rms_backward(const torch::Tensor &dout, const torch::Tensor &x, const torch::Tensor &weight,
+                                           const torch::Tensor &inv_variance, int64_t cols, bool strided) {
+    if (!ready(dout, x)) return c10::nullopt;
+    torch::Tensor dweight = at::empty_like(weight), dinp = strided ? dense_like_layout(x) : at::empty_like(x);
+    if (strided)
+        torch_launch_rms_backward_strided(dinp, dweight, dout, x, weight, inv_variance);
+    else
+        rms_backward_impl(dinp, dweight, dout, x, weight, inv_variance, x.numel() / cols, cols, false);
+    return Tensors{dinp, dweight};
+}
+
+// query, key, value: value is the transposed view of its slice of mixed
+static c10::optional<Tensors> qkv_forward(const torch::Tensor &mixed, const torch::Tensor &weight_q,
+                                          const torch::Tensor &weight_k, double epsilon,
+                                          const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    if (mixed.dim() != 4 || mixed.size(3) % 3 != 0) return c10::nullopt;
+    const int64_t cols = mixed.size(3) / 3;
+    if (!ready_rows(mixed, cols) || !tt_qkv_rmsnorm_supported(cols, dtype_code(mixed, "mixed_qkv"))) return c10::nullopt;
+    for (auto *w : {&weight_q, &weight_k})
+        if (!ready(*w, mixed) || w->numel() != cols) return c10::nullopt;
+    if (cos.has_value() != sin.has_value()) return c10::nullopt;
+    if (cos.has_value()) {
+        for (auto *t : {&*cos, &*sin})
+            if (t->scalar_type() != at::kFloat || !ready(*t, *t) || t->device() != mixed.device() || t->dim() != 2 ||
+                t->size(1) != cols || cols != 128 || t->size(0) > mixed.size(1))
+                return c10::nullopt;
+        if (cos->sizes() != sin->sizes()) return c10::nullopt;
+    }
+    const std::vector<int64_t> shape{mixed.size(0), mixed.size(2), mixed.size(1), cols};
+    torch::Tensor query = at::empty(shape, mixed.options()), key = at::empty(shape, mixed.options());
+    torch_launch_qkv_rms_forward(query, key, mixed, weight_q, weight_k, epsilon, cos, sin);
+    return Tensors{query, key, mixed.slice(3, 2 * cols, 3 * cols).transpose(1, 2)};
+}
+
+// dmixed, dweight_q, dweight_k; a gradient may be None
+static c10::optional<Tensors> qkv_backward(const c10::optional<torch::Tensor> &dquery, const c10::optional<torch::Tensor> &dkey,
+                                           const c10::optional<torch::Tensor> &dvalue, const torch::Tensor &mixed,
+                                           const torch::Tensor &weight_q, const torch::Tensor &weight_k, double epsilon,
+                                           const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    for (auto *g : {&dquery, &dkey, &dvalue})
+        if (g->has_value() && (*g)->defined() && !ready(**g, mixed)) return c10::nullopt;
+    torch::Tensor dmixed = at::empty_like(mixed), dwq = at::empty_like(weight_q), dwk = at::empty_like(weight_k);
+    torch_launch_qkv_rms_backward(dmixed, dwq, dwk, dquery, dkey, dvalue, mixed, weight_q, weight_k, epsilon, cos, sin);
+    return Tensors{dmixed, dwq, dwk};
+}
+
 PYBIND11_MODULE(fused_rmsnorm, m) {
+    m.def("rms_forward", &rms_forward, "RMSNorm forward: out, inv_variance; None unless every operand is ready");
+    m.def("rms_backward", &rms_backward, "RMSNorm backward: dinp, dweight; None unless the gradient is ready");
+    m.def("qkv_forward", &qkv_forward, "query, key, value of a fused projection; None unless every operand is ready");
+    m.def("qkv_backward", &qkv_backward, "its backward: dmixed, dweight_q, dweight_k; None unless the gradients are ready");
     m.def("torch_launch_qkv_rms_forward", &torch_launch_qkv_rms_forward,
           "RMSNorm (and rotary embedding) of the query and key slices of a fused projection");
     m.def("torch_launch_qkv_rms_backward", &torch_launch_qkv_rms_backward,

@@ -43,4 +43,22 @@ inline void raise_on(int status, const char *what) {
                 tt_norm_last_error());
 }
 
+// ---- whole calls -----------------------------------------------------------------------------
+// The autograd functions' forward and backward as one call each: checks, allocations and launch without a return to
+// Python between them.  They take only operands that need no preparation -- `ready`: an ordinary GPU tensor, contiguous,
+// 16-byte aligned, of the row tensor's dtype and device -- and return None for anything else, which the Python code then
+// prepares, or refuses with its own error.
+inline bool ready(const at::Tensor &t, const at::Tensor &like) {
+    return t.defined() && t.is_cuda() && !t.key_set().has(c10::DispatchKey::Python) && t.scalar_type() == like.scalar_type() &&
+           t.device() == like.device() && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+}
+
+inline bool ready_rows(const at::Tensor &x, int64_t cols) {
+    const auto st = x.scalar_type();
+    if (st != at::kBFloat16 && st != at::kHalf && st != at::kFloat) return false;
+    return ready(x, x) && cols > 0 && x.numel() % cols == 0 && tt_norm_supported(cols, dtype_code(x, "input"));
+}
+
+inline at::Tensor row_statistics(const at::Tensor &x, int64_t rows) { return at::empty({rows}, x.options().dtype(at::kFloat)); }
+
 }  // namespace ttn_glue

@@ -121,6 +121,14 @@ class FP32LayerNorm(nn.LayerNorm):
         return F.layer_norm(inputs.float(), self.normalized_shape, w, b, self.eps).to(inputs.dtype)
 
 
+def _like_modulation(ctx, *grads):
+    """Gradients of modulation rows in the shape and dtype the caller passed; ctx.mod_shape is None where the rows
+    were used as they came."""
+    if ctx.mod_shape is None:
+        return grads
+    return tuple(g.reshape(ctx.mod_shape).to(ctx.mod_dtype) for g in grads)
+
+
 class AdaLNModelFunction(Function):
     """out = LayerNorm(x) * (1 + scale) + shift, no LayerNorm affine.
 
@@ -137,6 +145,12 @@ class AdaLNModelFunction(Function):
         ext = _require_extension(fused_adaln, "fused_adaln")
         ctx.n_extra = len(seq_first)
         seq_first = bool(seq_first[0]) if seq_first else False
+        done = ext.adaln_forward(x, scale, shift, cols, float(epsilon), seq_first)
+        if done is not None:   # every operand was ready as it is; anything else is prepared, or refused, below
+            out, mean, invvar = done
+            ctx.save_for_backward(x, scale, mean, invvar)
+            ctx.rows, ctx.cols, ctx.seq_first, ctx.mod_shape, ctx.mod_dtype = invvar.shape[0], cols, seq_first, None, None
+            return out
         _require_gpu(x, "AdaLNModelFunction")
         x = _aligned_contiguous(x)
         scale_c = scale.contiguous()
@@ -170,6 +184,10 @@ class AdaLNModelFunction(Function):
     @staticmethod
     def backward(ctx, grad_output):
         x, scale_c, mean, invvar = ctx.saved_tensors
+        done = fused_adaln.adaln_backward(grad_output, None, x, scale_c, mean, invvar, ctx.cols, ctx.seq_first)
+        if done is not None:
+            grad_input, grad_scale, grad_shift = done
+            return (grad_input, *_like_modulation(ctx, grad_scale, grad_shift), None, None) + (None,) * ctx.n_extra
         grad_output = _aligned_contiguous(grad_output)
         if grad_output.dtype != x.dtype:
             grad_output = grad_output.to(x.dtype)
@@ -179,9 +197,7 @@ class AdaLNModelFunction(Function):
         launch = (fused_adaln.torch_launch_adaln_backward_x_seq_first if ctx.seq_first
                   else fused_adaln.torch_launch_adaln_backward_x)
         launch(grad_input, grad_scale, grad_shift, grad_output, x, scale_c, mean, invvar, ctx.rows, ctx.cols)
-        grad_scale = grad_scale.reshape(ctx.mod_shape).to(ctx.mod_dtype)
-        grad_shift = grad_shift.reshape(ctx.mod_shape).to(ctx.mod_dtype)
-        return (grad_input, grad_scale, grad_shift, None, None) + (None,) * ctx.n_extra
+        return (grad_input, *_like_modulation(ctx, grad_scale, grad_shift), None, None) + (None,) * ctx.n_extra
 
 
 class AdaLNResidualFunction(Function):
@@ -194,6 +210,13 @@ class AdaLNResidualFunction(Function):
     @staticmethod
     def forward(ctx, x, scale, shift, epsilon):
         ext = _require_extension(fused_adaln, "fused_adaln")
+        ctx.set_materialize_grads(False)
+        done = ext.adaln_forward(x, scale, shift, x.shape[-1], float(epsilon), False) if x.dim() else None
+        if done is not None:
+            out, mean, invvar = done
+            ctx.save_for_backward(x, scale, mean, invvar)
+            ctx.rows, ctx.cols, ctx.mod_shape, ctx.mod_dtype = invvar.shape[0], x.shape[-1], None, None
+            return x, out
         _require_gpu(x, "AdaLNResidualFunction")
         cols = x.shape[-1]
         if x.dtype not in _ELEM_BYTES or not wide_forms_supported(cols, x.dtype):
@@ -213,7 +236,6 @@ class AdaLNResidualFunction(Function):
         ctx.save_for_backward(x_c, scale_c, mean, invvar)
         ctx.rows, ctx.cols = rows, cols
         ctx.mod_shape, ctx.mod_dtype = scale.shape, scale.dtype
-        ctx.set_materialize_grads(False)
         return x, out
 
     @staticmethod
@@ -221,6 +243,9 @@ class AdaLNResidualFunction(Function):
         x, scale_c, mean, invvar = ctx.saved_tensors
         if grad_out is None:   # only the stream was used: the Function was an identity
             return grad_x_same, None, None, None
+        done = fused_adaln.adaln_backward(grad_out, grad_x_same, x, scale_c, mean, invvar, ctx.cols, False)
+        if done is not None:
+            return (done[0], *_like_modulation(ctx, done[1], done[2]), None)
         grad_out = _aligned_contiguous(grad_out.to(x.dtype))
         grad_input = torch.empty_like(x)
         grad_scale, grad_shift = torch.empty_like(scale_c), torch.empty_like(scale_c)
@@ -231,8 +256,7 @@ class AdaLNResidualFunction(Function):
             fused_adaln.torch_launch_adaln_backward_residual(grad_input, grad_scale, grad_shift, grad_out,
                                                              _aligned_contiguous(grad_x_same.to(x.dtype)), x, scale_c,
                                                              mean, invvar, ctx.rows, ctx.cols)
-        return (grad_input, grad_scale.reshape(ctx.mod_shape).to(ctx.mod_dtype),
-                grad_shift.reshape(ctx.mod_shape).to(ctx.mod_dtype), None)
+        return (grad_input, *_like_modulation(ctx, grad_scale, grad_shift), None)
 
 
 def modulated_layer_norm_keeping_stream(x, scale, shift, eps: float = 1e-6):
@@ -283,6 +307,14 @@ class GatedResidualAdaLNFunction(Function):
     @staticmethod
     def forward(ctx, h, attn, gate, scale, shift, epsilon):
         ext = _require_extension(fused_adaln, "fused_adaln")
+        ctx.set_materialize_grads(False)  # an unused h2 costs no zero tensor and no read
+        done = ext.gated_forward(h, attn, gate, scale, shift, float(epsilon))
+        if done is not None:
+            h2, out, mean, invvar = done
+            ctx.save_for_backward(h2, attn, gate, scale, mean, invvar)
+            ctx.rows, ctx.cols, ctx.mod_meta = invvar.shape[0], h.shape[-1], None
+            ctx.attn_dtype = attn.dtype
+            return h2, out
         _require_gpu(h, "GatedResidualAdaLNFunction")
         cols = h.shape[-1]
         if h.dtype not in _ELEM_BYTES or not wide_forms_supported(cols, h.dtype):
@@ -308,7 +340,6 @@ class GatedResidualAdaLNFunction(Function):
         ctx.rows, ctx.cols = rows, cols
         ctx.mod_meta = [(t.shape, t.dtype) for t in (gate, scale, shift)]
         ctx.attn_dtype = attn.dtype
-        ctx.set_materialize_grads(False)  # an unused h2 costs no zero tensor and no read
         return h2, out
 
     @staticmethod
@@ -316,6 +347,10 @@ class GatedResidualAdaLNFunction(Function):
         h2, attn_c, gate_c, scale_c, mean, invvar = ctx.saved_tensors
         if grad_out is None:
             grad_out = torch.zeros_like(h2)
+        if ctx.mod_meta is None:
+            done = fused_adaln.gated_backward(grad_out, grad_h2, h2, attn_c, gate_c, scale_c, mean, invvar, ctx.cols)
+            if done is not None:
+                return (*done, None)
         grad_out = _aligned_contiguous(grad_out.to(h2.dtype))
         if grad_h2 is not None:
             grad_h2 = _aligned_contiguous(grad_h2.to(h2.dtype))
@@ -324,8 +359,9 @@ class GatedResidualAdaLNFunction(Function):
         dgate, dscale, dshift = (torch.empty_like(scale_c) for _ in range(3))
         fused_adaln.torch_launch_gated_adaln_backward(dh, dattn, dgate, dscale, dshift, grad_out, grad_h2, h2,
                                                       attn_c, gate_c, scale_c, mean, invvar, ctx.rows, ctx.cols)
-        dgate, dscale, dshift = (g.reshape(shape).to(dtype)
-                                 for g, (shape, dtype) in zip((dgate, dscale, dshift), ctx.mod_meta))
+        if ctx.mod_meta is not None:
+            dgate, dscale, dshift = (g.reshape(shape).to(dtype)
+                                     for g, (shape, dtype) in zip((dgate, dscale, dshift), ctx.mod_meta))
         return dh, dattn.to(ctx.attn_dtype), dgate, dscale, dshift, None
 
 
@@ -471,6 +507,13 @@ class RMSNormModelFunction(Function):
     @staticmethod
     def forward(ctx, x, weight, epsilon, cols):
         ext = _require_extension(fused_rmsnorm, "fused_rmsnorm")
+        done = ext.rms_forward(x, weight, cols, float(epsilon))
+        if done is not None:
+            out, invvar = done
+            ctx.save_for_backward(x, weight, invvar)
+            ctx.rows, ctx.cols, ctx.strided = invvar.shape[0], cols, False
+            ctx.w_shape, ctx.w_dtype = weight.shape, weight.dtype
+            return out
         _require_gpu(x, "RMSNormModelFunction")
         if x.numel() % cols != 0:
             raise ValueError(f"Input size {x.numel()} not divisible by cols {cols}")
@@ -499,6 +542,10 @@ class RMSNormModelFunction(Function):
     @staticmethod
     def backward(ctx, grad_output):
         x, w, invvar = ctx.saved_tensors
+        done = fused_rmsnorm.rms_backward(grad_output, x, w, invvar, ctx.cols, ctx.strided)
+        if done is not None:
+            grad_input, grad_weight = done
+            return grad_input, grad_weight.reshape(ctx.w_shape).to(ctx.w_dtype), None, None
         grad_output = _aligned_contiguous(grad_output)
         if grad_output.dtype != x.dtype:
             grad_output = grad_output.to(x.dtype)
@@ -558,6 +605,13 @@ class QKVSplitNormFunction(Function):
         ext = _require_extension(fused_rmsnorm, "fused_rmsnorm")
         if len(rotary) not in (0, 2):
             raise ValueError("pass freqs_cos and freqs_sin together, or neither")
+        done = ext.qkv_forward(mixed_qkv, weight_q, weight_k, float(epsilon), *(rotary or (None, None)))
+        if done is not None:
+            ctx.epsilon, ctx.n_rotary, ctx.joint = float(epsilon), len(rotary), True
+            ctx.w_meta = [(w.shape, w.dtype) for w in (weight_q, weight_k)]
+            ctx.set_materialize_grads(False)
+            ctx.save_for_backward(mixed_qkv, weight_q, weight_k, *rotary)
+            return tuple(done)
         _require_gpu(mixed_qkv, "QKVSplitNormFunction")
         if mixed_qkv.dim() != 4 or mixed_qkv.shape[-1] % 3:
             raise ValueError(f"mixed_qkv must be [B, S, H, 3*D], got {tuple(mixed_qkv.shape)}")
@@ -605,9 +659,14 @@ class QKVSplitNormFunction(Function):
 
     @staticmethod
     def backward(ctx, grad_q, grad_k, grad_v):
-        d_mixed = torch.empty_like(ctx.saved_tensors[0])
         if ctx.joint:
             mixed, wq, wk, *tables = ctx.saved_tensors
+            done = fused_rmsnorm.qkv_backward(grad_q, grad_k, grad_v, mixed, wq, wk, ctx.epsilon, *(tables or (None, None)))
+            if done is not None:
+                d_mixed, *grads_w = done
+                grads_w = [dw.reshape(shape).to(dtype) for dw, (shape, dtype) in zip(grads_w, ctx.w_meta)]
+                return (d_mixed, grads_w[0], grads_w[1], None) + (None,) * ctx.n_rotary
+            d_mixed = torch.empty_like(mixed)
             grads = [None if g is None else _aligned_contiguous(g.to(mixed.dtype)) for g in (grad_q, grad_k, grad_v)]
             grads_w = [torch.empty_like(w) for w in (wq, wk)]
             fused_rmsnorm.torch_launch_qkv_rms_backward(d_mixed, *grads_w, *grads, mixed, wq, wk, ctx.epsilon,
@@ -615,6 +674,7 @@ class QKVSplitNormFunction(Function):
             grads_w = [dw.reshape(shape).to(dtype) for dw, (shape, dtype) in zip(grads_w, ctx.w_meta)]
             return (d_mixed, grads_w[0], grads_w[1], None) + (None,) * ctx.n_rotary
         mixed, wq, wk, rstd_q, rstd_k = ctx.saved_tensors
+        d_mixed = torch.empty_like(mixed)
         cols = ctx.cols
         slices = [d_mixed[..., i * cols:(i + 1) * cols].transpose(1, 2) for i in range(3)]
         grads_w = []
