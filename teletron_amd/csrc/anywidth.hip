@@ -69,34 +69,6 @@ struct PadGeom {
     static_assert(LANES == 64 || CHUNKS == 1, "only full wavefronts take several accesses per lane");
 };
 
-// rnd(a * b) for the elements of one access, both packed
-template <typename T>
-__device__ __forceinline__ u32x4 packed_products(const u32x4 &a, const u32x4 &b) {
-    using E = Elem<T>;
-    if constexpr (std::is_same<T, f16_t>::value) {
-        PairFactor<f16_t> f;
-        f.set(b);
-        return rounded_products<f16_t>(a, f);
-    } else {
-        float av[E::VEC], bv[E::VEC];
-        E::unpack(a, av);
-        E::unpack(b, bv);
-#pragma unroll
-        for (int j = 0; j < E::VEC; ++j) av[j] *= bv[j];
-        return E::pack(av);
-    }
-}
-
-// acc += v per column.  Not the packed dot product against (1, 0) / (0, 1): that multiplies the pair's other element by
-// zero, and an infinity there would spread to this column's sum.
-template <typename T>
-__device__ __forceinline__ void add_columns(float (&acc)[Elem<T>::VEC], const u32x4 &v) {
-    float f[Elem<T>::VEC];
-    Elem<T>::unpack(v, f);
-#pragma unroll
-    for (int j = 0; j < Elem<T>::VEC; ++j) acc[j] += f[j];
-}
-
 // Which of this lane's accesses lie inside a row of `pieces` 16-byte pieces.
 template <typename G>
 struct LaneMask {

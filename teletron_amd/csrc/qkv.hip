@@ -19,7 +19,7 @@
 // only if what is WRITTEN at a time is contiguous: forward therefore runs its workgroups along the tokens of one head
 // at a time (one-shot), backward along the heads of one token group at a time.  Measured there, against one kernel per
 // tensor (two forward; two backward, one copy of the value gradient, two reducers): forward 122 against 150 us, with
-// tables 137 against 151; backward 256 against 297, with tables 260 against 303.
+// tables 137 against 151; backward 258 against 297, with tables 262 against 303.
 //
 // Forward: wavefronts of a workgroup along the tokens (the others along the heads) and heads per wavefront.  Without
 // tables four consecutive token groups of one head (tokens along two / one wavefronts: 127 us; two heads: 126).  With
@@ -153,14 +153,11 @@ __global__ __launch_bounds__(kRowThreads) void qkv_bwd_kernel(
     const uint32_t mixed_lane = (uint32_t)sub * (H * 3u * (uint32_t)C * (uint32_t)sizeof(T)) + l * 16;
     const uint32_t dense_lane = (uint32_t)(sub * C * (int)sizeof(T)) + l * 16;
     const u32x4 zero{0, 0, 0, 0};
-    const uint32_t one_lo = opaque_const(kOneLo<std::conditional_t<kHasDot2<T>, T, bf16_t>>);
-    const uint32_t one_hi = opaque_const(kOneHi<std::conditional_t<kHasDot2<T>, T, bf16_t>>);
     const uint32_t waves = gridDim.x * kRowWaves, me = blockIdx.x * kRowWaves + wave;
     const bool has[3] = {gq != nullptr, gk != nullptr, gv != nullptr};
 
-    RowParam<T, 2> wp;
-    wp.set(0, in ? load16(reinterpret_cast<const u32x4 *>(wq) + l) : zero);
-    wp.set(1, in ? load16(reinterpret_cast<const u32x4 *>(wk) + l) : zero);
+    const u32x4 w[2] = {in ? load16(reinterpret_cast<const u32x4 *>(wq) + l) : zero,
+                        in ? load16(reinterpret_cast<const u32x4 *>(wk) + l) : zero};
     float acc[2][VEC];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -211,7 +208,7 @@ __global__ __launch_bounds__(kRowThreads) void qkv_bwd_kernel(
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             if (!has[t]) continue;
-            const u32x4 gy = wp.times(t, g[t]);  // rnd(g * w)
+            const u32x4 gy = packed_products<T>(g[t], w[t]);  // rnd(g * w)
             float dot = 0.0f;
             if constexpr (kHasDot2<T>) {
 #pragma unroll
@@ -236,7 +233,7 @@ __global__ __launch_bounds__(kRowThreads) void qkv_bwd_kernel(
                 y[j] = xv[j] * r;
             }
             d[t] = E::pack(o);
-            add_rounded_products<T>(acc[t], g[t], y, one_lo, one_hi);  // dw += rnd(g * rnd(y))
+            add_columns<T>(acc[t], packed_products<T>(g[t], E::pack(y)));  // dw += rnd(g * rnd(y))
         }
         const RowWriter<0> wd[3] = {{dmixed + at, mixed_lane}, {dmixed + at + C, mixed_lane}, {dmixed + at + 2 * C, mixed_lane}};
         if (ok) {

@@ -101,3 +101,17 @@ def test_empty_projection_and_refusals(capi, gpu_device):
     wide = torch.empty(1, 2, 1, 3 * 520, device=gpu_device, dtype=BF)
     with pytest.raises(capi.NormError, match="64 whole 16-byte pieces"):
         capi.qkv_rmsnorm_forward(wide, *[torch.ones(520, device=gpu_device, dtype=BF)] * 2, EPS)
+
+
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("dtype", [BF, HF, F32])
+def test_an_infinite_gradient_stays_in_its_column(capi, gpu_device, D, dtype):
+    gen = torch.Generator(device=gpu_device).manual_seed(D)
+    rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=gen).to(dtype)
+    mixed, w, grads = rnd(1, 19, 2, 3 * D), rnd(D), [rnd(1, 2, 19, D) for _ in range(3)]
+    bad = [g.clone() for g in grads]
+    bad[0][0, 1, 7, 20] = float("inf")
+    others = torch.arange(D, device=gpu_device) != 20
+    a, b = (capi.qkv_rmsnorm_backward(*g, mixed, w, w, EPS) for g in (grads, bad))
+    assert torch.equal(a[1][others], b[1][others]) and not bool(torch.isfinite(b[1][20]))
+    assert torch.equal(a[2], b[2])
