@@ -292,6 +292,8 @@ static c10::optional<Tensors> gated_forward(const torch::Tensor &h, const torch:
     const int64_t cols = h.size(-1);
     for (auto *t : {&gate, &scale, &shift})
         if (!ready(*t, h) || t->numel() != scale.numel()) return c10::nullopt;
+    // backward shapes the gradients after gate and scale, the rows it keeps: shift's is scale's
+    if (shift.sizes() != scale.sizes()) return c10::nullopt;
     if (!ready_modulation(h, scale, cols, false)) return c10::nullopt;
     const int64_t rows = h.numel() / cols;
     torch::Tensor h2 = at::empty_like(h), out = at::empty_like(h);
@@ -307,7 +309,7 @@ static c10::optional<Tensors> gated_backward(const torch::Tensor &dout, const c1
                                              const torch::Tensor &inv_variance, int64_t cols) {
     if (!ready(dout, h2) || (dh2.has_value() && dh2->defined() && !ready(*dh2, h2))) return c10::nullopt;
     torch::Tensor dh = at::empty_like(h2), dattn = at::empty_like(h2);
-    torch::Tensor dgate = at::empty_like(scale), dscale = at::empty_like(scale), dshift = at::empty_like(scale);
+    torch::Tensor dgate = at::empty_like(gate), dscale = at::empty_like(scale), dshift = at::empty_like(scale);
     torch_launch_gated_adaln_backward(dh, dattn, dgate, dscale, dshift, dout, dh2, h2, attn, gate, scale, mean, inv_variance,
                                       h2.numel() / cols, cols);
     return Tensors{dh, dattn, dgate, dscale, dshift};

@@ -356,7 +356,7 @@ class GatedResidualAdaLNFunction(Function):
             grad_h2 = _aligned_contiguous(grad_h2.to(h2.dtype))
         dh = torch.empty_like(h2)
         dattn = torch.empty_like(h2)
-        dgate, dscale, dshift = (torch.empty_like(scale_c) for _ in range(3))
+        dgate, dscale, dshift = (torch.empty_like(m) for m in (gate_c, scale_c, scale_c))
         fused_adaln.torch_launch_gated_adaln_backward(dh, dattn, dgate, dscale, dshift, grad_out, grad_h2, h2,
                                                       attn_c, gate_c, scale_c, mean, invvar, ctx.rows, ctx.cols)
         if ctx.mod_meta is not None:

@@ -83,3 +83,21 @@ def test_parameters_of_another_dtype_get_gradients_of_their_own(gpu_device, kind
     got = _run(kind, wide, grads)
     for a, x, y in zip(wide, got[-len(args):], want[-len(args):]):
         assert x.dtype == a.dtype and torch.equal(x, y.to(a.dtype))
+
+
+# shapes of gate, scale and shift; [B, 1, C] is gate.unsqueeze(1), as a block that broadcasts it over the tokens holds it
+@pytest.mark.parametrize("batch,gate,scale,shift", [
+    (2, (2, 1, 3072), (2, 3072), (2, 3072)), (2, (2, 3072), (2, 1, 3072), (2, 1, 3072)),
+    (2, (2, 3072), (2, 3072), (2, 1, 3072)), (1, (1, 1, 3072), (3072,), (3072,)), (1, (3072,), (1, 3072), (3072,))])
+@pytest.mark.parametrize("dense_grad", [True, False])
+def test_gated_modulation_rows_of_unlike_shapes(gpu_device, batch, gate, scale, shift, dense_grad):
+    """Every modulation row gets its gradient in its own shape, with the values that equal shapes get."""
+    args, grads = _operands("gated", torch.bfloat16, gpu_device)
+    args = [a[:batch] for a in args]
+    grads = [g[:batch] for g in grads]
+    want = _run("gated", args, grads)
+    shaped = args[:2] + [a.reshape(s) for a, s in zip(args[2:], (gate, scale, shift))]
+    got = _run("gated", shaped, grads if dense_grad else [_shifted(g) for g in grads])
+    for x, y, a in zip(got[2:], want[2:], shaped):
+        assert x.shape == a.shape and torch.equal(x, y.reshape(a.shape))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
