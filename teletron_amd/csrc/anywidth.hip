@@ -49,9 +49,12 @@
 #define TTN_ANY_ADALN_FWD_ROWS 2
 #endif
 // Backward workgroups per compute unit by accesses per lane (1 to 6).  One with the next row requested ahead beats two
-// and three without from three accesses on (12000 x 2560: 37.5 against 41.2 us), and writes fewer partial rows.
+// and three without from three accesses on (12000 x 2560: 37.5 against 41.2 us), and writes fewer partial rows.  Rows of
+// one access take four: with a second row buffer in flight six only add partial rows and contention (RMSNorm backward
+// 200000 x 256 bf16 with six 65.7 us, four 57.8, three 55.8; 100000 x 512 61.7 / 57.5 / 55.2), while three lose on strided
+// views of short rows (9000 x 16 x 96: 26.2 with four, 27.3 with three).
 #ifndef TTN_ANY_BWD_BLOCKS
-#define TTN_ANY_BWD_BLOCKS {6, 2, 1, 1, 1, 1}
+#define TTN_ANY_BWD_BLOCKS {4, 2, 1, 1, 1, 1}
 #endif
 
 namespace ttn {
