@@ -43,8 +43,11 @@
 #ifndef TTN_ANY_BWD_STORE
 #define TTN_ANY_BWD_STORE 1
 #endif
-// AdaLN forward: rows per wavefront where that leaves enough workgroups; they share the modulation row (100000 x 1024
-// bf16: one row 73.9, two 68.4, four 71.0 us; 12000 x 1536: 18.0 / 16.7 / 16.4).
+// AdaLN forward of two-byte rows whose grid of one row per wavefront is larger than what the chip holds at a time: rows
+// per wavefront, which share the modulation row (100000 x 1024 bf16 one row 79.5, two 75.3 us; 30000 x 768 23.2 / 21.6;
+// 12000 x 1024 12.2 / 11.1).  A grid that fits gets longer with a second row (64 x 64 x 1024 fp32 8.6 instead of 7.0 us,
+// 6000 x 1024 bf16 7.6 / 7.3).  The gated form and four-byte rows, with twice the bytes per row of the modulation, gain
+// nothing or lose (gated 100000 x 1024 138.3 / 141.6, 30000 x 1024 fp32 81.4 / 84.4; 20000 x 1536 fp32 42.9 / 43.9).
 #ifndef TTN_ANY_ADALN_FWD_ROWS
 #define TTN_ANY_ADALN_FWD_ROWS 2
 #endif
@@ -366,32 +369,48 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
     const LaneMask<G> m(l, C / VEC);
     const uint32_t row_bytes = (uint32_t)(C * (int)sizeof(T));
 
+    // Two orders of the requests.  Two-byte rows ask for the modulation row first and form t = rnd(1 + scale) behind the
+    // row's statistics, which then wait for neither (row first, t before the statistics: 3000 x 1536 bf16 6.5 instead of
+    // 6.0 us, 4400 x 1536 8.2 / 7.6, gated 30000 x 768 40.9 / 35.0).  Four-byte rows, with half the arithmetic per byte,
+    // ask for the row first and wait for all of it before they start, which keeps the chip's reads apart from its writes
+    // (3700 x 1024 fp32 6.3 us, the other order 7.7).  Rows of one access are walked by a persistent grid: t once per
+    // wavefront.
+    constexpr bool kRowFirst = sizeof(T) == 4 && CHUNKS > 1;
+    constexpr bool kFormLate = sizeof(T) == 2 && CHUNKS > 1;
     u32x4 tr[CHUNKS], hr[CHUNKS];
     [[maybe_unused]] u32x4 qr[GATED ? CHUNKS : 1];
+    auto one_plus = [](const u32x4 &raw) -> u32x4 {
+        float v[VEC];
+        E::unpack(raw, v);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
+        return E::pack(v);
+    };
 
     const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
     const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
     const uint32_t lane_bytes = (uint32_t)(sub * lay.row_stride * C * (int64_t)sizeof(T)) + l * 16;
     u32x4 xr[CHUNKS];
     [[maybe_unused]] u32x4 ar[GATED ? CHUNKS : 1];
-    auto fetch = [&](u32x4 (&dx)[CHUNKS], u32x4 (&da)[GATED ? CHUNKS : 1], int64_t i) {
+    auto fetch = [&](int64_t i) {
         const int64_t rs = i * RPW + sub;
         const int64_t at = lay.row(b, rs) * C;
-        load_row<G>(dx, x + at, l, rs < rows_per_sample, m, row_bytes);
-        if constexpr (GATED) load_row<G>(da, attn + at, l, rs < rows_per_sample, m, row_bytes);
+        load_row<G>(xr, x + at, l, rs < rows_per_sample, m, row_bytes);
+        if constexpr (GATED) load_row<G>(ar, attn + at, l, rs < rows_per_sample, m, row_bytes);
     };
     int64_t grp = (int64_t)slot * kRowWaves + wave;
-    if (grp < groups) fetch(xr, ar, grp);
+    if constexpr (kRowFirst) {
+        if (grp < groups) fetch(grp);
+    }
     load_param<G>(tr, scale + b * C, l, m);
     load_param<G>(hr, shift + b * C, l, m);
     if constexpr (GATED) load_param<G>(qr, gate + b * C, l, m);
+    if constexpr (!kRowFirst) {
+        if (grp < groups) fetch(grp);
+    }
+    if constexpr (!kFormLate) {
 #pragma unroll
-    for (int k = 0; k < CHUNKS; ++k) {  // t = rnd(1 + scale)
-        float v[VEC];
-        E::unpack(tr[k], v);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
-        tr[k] = E::pack(v);
+        for (int k = 0; k < CHUNKS; ++k) tr[k] = one_plus(tr[k]);
     }
 
     for (; grp < groups; grp += stride) {
@@ -453,17 +472,13 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
             rstd[row] = r;
         }
 
-        u32x4 xn[CHUNKS];  // the next row, requested before this one's output pass
-        [[maybe_unused]] u32x4 an[GATED ? CHUNKS : 1];
-        if (grp + stride < groups) fetch(xn, an, grp + stride);
-
         const float nmr = -(mu * r);
         const RowOut<G, TTN_ANY_FWD_STORE, kFwdStore> wo(out + first, lane_bytes, l, row_bytes);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
             float v[VEC], tv[VEC], hv[VEC];
             E::unpack(xr[k], v);
-            E::unpack(tr[k], tv);
+            E::unpack(kFormLate ? one_plus(tr[k]) : tr[k], tv);
             E::unpack(hr[k], hv);
 #pragma unroll
             for (int j = 0; j < VEC; ++j) v[j] = centred<T>(v[j], mu, r, nmr);
@@ -475,12 +490,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_fwd_kernel(
             for (int j = 0; j < VEC; ++j) v[j] += hv[j];
             wo.put(k, ok, m, E::pack(v));
         }
-#pragma unroll
-        for (int k = 0; k < CHUNKS; ++k) xr[k] = xn[k];
-        if constexpr (GATED) {
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k) ar[k] = an[k];
-        }
+        if (grp + stride < groups) fetch(grp + stride);
     }
 }
 
@@ -687,7 +697,7 @@ static int dispatch(int dtype, GeomChoice gc, Args... args) {
 }
 
 // Launch policy.  Forward: narrow rows (one access per lane) use a persistent grid of 16 workgroups
-// per compute unit, wider rows one row per wavefront (AdaLN: up to TTN_ANY_ADALN_FWD_ROWS).  Backward is
+// per compute unit, wider rows one row per wavefront (AdaLN: see share_modulation).  Backward is
 // persistent (column sums live in registers); the grid shrinks as rows widen so that each compute unit
 // keeps about the same number of bytes in flight.
 constexpr int kOneShotAny = 1 << 20;
@@ -702,18 +712,27 @@ static GeomChoice geometry_for(int64_t cols, int dtype) {
 }
 
 // Grid for (batch, rows_per_sample) under geometry gc; status != OK on failure.
-static int plan_for(RowPlan *plan, int64_t batch, int64_t rows_per_sample, GeomChoice gc, bool backward, int fwd_rows = 1) {
+static int plan_for(RowPlan *plan, int64_t batch, int64_t rows_per_sample, GeomChoice gc, bool backward) {
     int st = TT_NORM_OK;
     const int cus = current_device_cus(&st);
     if (st != TT_NORM_OK) return st;
     *plan = make_row_plan(batch, rows_per_sample, kWaveSize / gc.lanes,
                           backward ? bwd_blocks_per_cu(gc.chunks) : fwd_blocks_per_cu(gc.chunks), cus);
-    // below four workgroups per compute unit a second row would only lengthen the call (600 x 2048: 4.3 -> 6.1 us)
-    if (!backward && gc.chunks > 1 && plan->blocks >= (int64_t)cus * 4) {
-        plan->blocks_per_sample = (plan->blocks_per_sample + fwd_rows - 1) / fwd_rows;
+    if (plan->blocks > 0x7fffffffLL) return fail(TT_NORM_EINVAL, "grid too large");
+    return TT_NORM_OK;
+}
+
+// A grid of one row per wavefront that the chip cannot hold at once: TTN_ANY_ADALN_FWD_ROWS rows per wavefront instead.
+constexpr int kMostResident = 8;  // workgroups of four wavefronts that fill a compute unit
+static int share_modulation(RowPlan *plan, int resident) {
+    int st = TT_NORM_OK;
+    const int cus = current_device_cus(&st);
+    if (st != TT_NORM_OK) return st;
+    const int64_t batch = plan->blocks / plan->blocks_per_sample;
+    if (plan->blocks > (int64_t)cus * resident) {
+        plan->blocks_per_sample = (plan->blocks_per_sample + TTN_ANY_ADALN_FWD_ROWS - 1) / TTN_ANY_ADALN_FWD_ROWS;
         plan->blocks = batch * plan->blocks_per_sample;
     }
-    if (plan->blocks > 0x7fffffffLL) return fail(TT_NORM_EINVAL, "grid too large");
     return TT_NORM_OK;
 }
 
@@ -759,10 +778,17 @@ struct AdalnOn {
             if constexpr (CHUNKS > 6) {  // wider dense rows run on the wide-row kernels
                 return fail(TT_NORM_EUNSUPPORTED, "AdaLN: rows of more than six 16-byte accesses per lane");
             } else {
+                RowPlan q = p;
+                if constexpr (!GATED && sizeof(T) == 2 && CHUNKS > 1) {
+                    static const int resident =
+                        resident_blocks_per_cu(anywidth_adaln_fwd_kernel<T, LANES, CHUNKS, GATED>, kMostResident);
+                    const int st = share_modulation(&q, resident);
+                    if (st != TT_NORM_OK) return st;
+                }
                 RowKernelProfile prof(stream);
-                anywidth_adaln_fwd_kernel<T, LANES, CHUNKS, GATED><<<dim3((unsigned)p.blocks), dim3(kRowThreads), 0, stream>>>(
+                anywidth_adaln_fwd_kernel<T, LANES, CHUNKS, GATED><<<dim3((unsigned)q.blocks), dim3(kRowThreads), 0, stream>>>(
                     (T *)out, mean, rstd, (const T *)x, (const T *)scale, (const T *)shift, (T *)ex.h2_or_da,
-                    (const T *)ex.attn, (const T *)ex.gate, rows_per_sample, lay, p.blocks_per_sample, C, (float)eps);
+                    (const T *)ex.attn, (const T *)ex.gate, rows_per_sample, lay, q.blocks_per_sample, C, (float)eps);
                 return TT_NORM_OK;
             }
         }
@@ -880,7 +906,7 @@ static int adaln_forward_any(void *out, float *mean, float *rstd, const void *x,
     if (rows_per_sample == 0) return TT_NORM_OK;
     const GeomChoice gc = geometry_for(cols, dtype);
     RowPlan p;
-    int st = plan_for(&p, batch, rows_per_sample, gc, false, TTN_ANY_ADALN_FWD_ROWS);
+    int st = plan_for(&p, batch, rows_per_sample, gc, false);
     if (st != TT_NORM_OK) return st;
     st = dispatch<AdalnOn<GATED, false>::template Fwd>(dtype, gc, p, out, mean, rstd, x, scale, shift, ex, rows_per_sample,
                                                        layout_of(batch, rows_per_sample, seq_first), (int)cols, eps,

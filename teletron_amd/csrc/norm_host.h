@@ -61,6 +61,19 @@ struct RowPlan {
 RowPlan make_row_plan(int64_t batch, int64_t rows_per_sample, int rows_per_wave,
                       int blocks_per_cu, int cus);
 
+// Workgroups of `kernel` (of kRowThreads threads and no dynamic LDS) that one compute unit holds at a time, at most
+// `wanted`; asked of the runtime, so callers ask once per kernel.  A persistent grid must not be larger than what is
+// resident, or its surplus workgroups run as a second round.
+template <typename K>
+int resident_blocks_per_cu(K kernel, int wanted) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kRowThreads, 0) != hipSuccess || n < 1) {
+        (void)hipGetLastError();
+        return wanted;
+    }
+    return n < wanted ? n : wanted;
+}
+
 // Stage-2 reducer: partial[batch][blocks_per_sample][ncols] fp32 ->
 // out0[batch][C] (columns [0, C)), out1[batch][C] (columns [C, 2C)) when ncols >= 2C,
 // out2[batch][C] (columns [2C, 3C)) when ncols == 3C.

@@ -702,18 +702,6 @@ static int wide_chunks(int64_t cols, int dtype) {
     return (wide_pieces_per_wave(cols, dtype) + kWaveSize - 1) / kWaveSize;  // 2, 3 or 4 for 385..1024 pieces
 }
 
-// Workgroups of `kernel` that one compute unit holds at a time (asked of the runtime once per kernel): a
-// persistent grid must not be larger than what is resident, or its surplus workgroups run as a second round.
-template <typename K>
-static int resident_blocks_per_cu(K kernel, int wanted) {
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kRowThreads, 0) != hipSuccess || n < 1) {
-        (void)hipGetLastError();
-        return wanted;
-    }
-    return n < wanted ? n : wanted;
-}
-
 // One row per workgroup and step: `per_cu` workgroups per compute unit, split evenly over the samples.
 // With rows_per_block > 0 the grid is sized by the rows instead: workgroups of that many rows each, which retire
 // and are replaced as the grid drains.

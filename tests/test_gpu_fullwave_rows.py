@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 EPS = 1e-6
 BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
 # batch, rows per sample, pieces per row
-CASES = [(1, 1, 33), (2, 4101, 65), (3, 7, 129), (1, 1025, 193), (2, 515, 257), (1, 4099, 289), (1, 3, 320), (2, 67, 321),
-         (1, 130, 383)]
+CASES = [(1, 1, 33), (2, 4101, 65), (3, 7, 129), (1, 1025, 193), (2, 515, 257), (1, 4099, 289),
+         (1, 5131, 257), (1, 3, 320), (2, 67, 321), (1, 130, 383)]
 
 
 @pytest.fixture(scope="module")
