@@ -718,6 +718,10 @@ static int plan_for(RowPlan *plan, int64_t batch, int64_t rows_per_sample, GeomC
     if (st != TT_NORM_OK) return st;
     *plan = make_row_plan(batch, rows_per_sample, kWaveSize / gc.lanes,
                           backward ? bwd_blocks_per_cu(gc.chunks) : fwd_blocks_per_cu(gc.chunks), cus);
+    if (plan->blocks > kMostBlocks && batch <= kMostBlocks) {  // the kernels walk whatever the grid leaves
+        plan->blocks_per_sample = (int)(kMostBlocks / batch);
+        plan->blocks = batch * plan->blocks_per_sample;
+    }
     if (plan->blocks > 0x7fffffffLL) return fail(TT_NORM_EINVAL, "grid too large");
     return TT_NORM_OK;
 }

@@ -364,6 +364,7 @@ static c10::optional<Tensors> qkv_forward(const torch::Tensor &mixed, const torc
     if (mixed.dim() != 4 || mixed.size(3) % 3 != 0) return c10::nullopt;
     const int64_t cols = mixed.size(3) / 3;
     if (!ready_rows(mixed, cols) || !tt_qkv_rmsnorm_supported(cols, dtype_code(mixed, "mixed_qkv"))) return c10::nullopt;
+    if (!cos.has_value() && mixed.numel() / mixed.size(3) > INT32_MAX) return c10::nullopt;  // beyond the joint kernels' units
     for (auto *w : {&weight_q, &weight_k})
         if (!ready(*w, mixed) || w->numel() != cols) return c10::nullopt;
     if (cos.has_value() != sin.has_value()) return c10::nullopt;

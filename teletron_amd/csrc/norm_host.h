@@ -61,6 +61,9 @@ struct RowPlan {
 RowPlan make_row_plan(int64_t batch, int64_t rows_per_sample, int rows_per_wave,
                       int blocks_per_cu, int cus);
 
+// HIP counts the threads of one grid dimension in 32 bits: the workgroups of kRowThreads a dimension may have.
+constexpr int64_t kMostBlocks = 0xffffffffLL / kRowThreads;
+
 // Workgroups of `kernel` (of kRowThreads threads and no dynamic LDS) that one compute unit holds at a time, at most
 // `wanted`; asked of the runtime, so callers ask once per kernel.  A persistent grid must not be larger than what is
 // resident, or its surplus workgroups run as a second round.

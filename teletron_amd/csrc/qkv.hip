@@ -72,7 +72,7 @@ template <typename T, int LANES, bool FULL, typename Rope>
 __global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q, T *__restrict__ k,
                                                               const T *__restrict__ mixed, const T *__restrict__ wq,
                                                               const T *__restrict__ wk, const Rope rope, int64_t S, int H,
-                                                              int head_blocks, int outer, int c_arg, float eps) {
+                                                              uint32_t head_blocks, uint32_t outer, int c_arg, float eps) {
     using G = HeadGeom<T, LANES, FULL>;
     using E = Elem<T>;
     constexpr bool ROPE = Rope::kOn;
@@ -84,15 +84,15 @@ __global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q,
     const int l = lane % LANES;
     const int wave = wave_id_in_block();
     const bool in = FULL || l * VEC < C;
-    const int64_t s0 = ((int64_t)blockIdx.x * TW + wave % TW) * RPW;
+    const int64_t s0 = (((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * TW + wave % TW) * RPW;
     const bool ok = in && s0 + sub < S;
     const uint32_t from = (uint32_t)sub * (uint32_t)(H * 3 * C * (int)sizeof(T)) + l * 16;
     const uint32_t to = (uint32_t)(sub * C * (int)sizeof(T)) + l * 16;
     const u32x4 zero{0, 0, 0, 0};
 
-    for (int y = blockIdx.y; y < outer; y += gridDim.y) {
+    for (uint32_t y = blockIdx.y; y < outer; y += gridDim.y) {
         const int64_t b = y / head_blocks;
-        const int h0 = ((y % head_blocks) * HW + wave / TW) * HR;
+        const int h0 = ((int)(y % head_blocks) * HW + wave / TW) * HR;
         const T *src = mixed + ((b * S + s0) * H + h0) * 3 * C;
         u32x4 xr[HR][2];
 #pragma unroll
@@ -282,10 +282,11 @@ static void launch_qkv_fwd(const QkvSizes &z, void *q, void *k, const void *mixe
     constexpr int TW = TTN_QKV_FWD_TOKEN_WAVES, heads = kRowWaves / TW * TTN_QKV_FWD_HEADS;
     const int head_blocks = (int)((z.H + heads - 1) / heads);
     const int64_t outer = z.B * head_blocks;
-    const dim3 grid((unsigned)((z.token_groups() + TW - 1) / TW), (unsigned)(outer < 65535 ? outer : 65535));
+    const int64_t along = (z.token_groups() + TW - 1) / TW, layers = (along + kMostBlocks - 1) / kMostBlocks;
+    const dim3 grid((unsigned)((along + layers - 1) / layers), (unsigned)(outer < 65535 ? outer : 65535), (unsigned)layers);
     RowKernelProfile prof(stream);
     qkv_fwd_kernel<T, LANES, FULL, Rope><<<grid, dim3(kRowThreads), 0, stream>>>(
-        (T *)q, (T *)k, (const T *)mixed, (const T *)wq, (const T *)wk, rope, z.S, (int)z.H, head_blocks, (int)outer,
+        (T *)q, (T *)k, (const T *)mixed, (const T *)wq, (const T *)wk, rope, z.S, (int)z.H, (uint32_t)head_blocks, (uint32_t)outer,
         (int)z.cols, eps);
 }
 

@@ -53,6 +53,7 @@ TUNED_COLS = (128, 3072)  # the reference's two shapes (the tuned kernels)
 _ELEM_BYTES = {torch.bfloat16: 2, torch.float16: 2, torch.float32: 4}
 _MAX_PIECES = 1024  # 16-byte pieces per row the kernels are built for
 _MAX_JOINT_HEAD_BYTES = 1024  # a head's row the joint q / k / v kernels take: 64 16-byte pieces
+_MAX_JOINT_ROWS = 2 ** 31 - 1  # rows of q (or k) whose groups their 32-bit unit numbers are sure to hold
 
 
 def cols_supported(cols: int, dtype: torch.dtype) -> bool:
@@ -641,13 +642,13 @@ class QKVSplitNormFunction(Function):
         ctx.set_materialize_grads(False)
         # v leaves as a copy-free view only when mixed_qkv itself was usable in place
         v_out = v_in if mixed is mixed_qkv else v_in.clone()
-        ctx.joint = cols * mixed.element_size() <= _MAX_JOINT_HEAD_BYTES
+        ctx.joint = cols * mixed.element_size() <= _MAX_JOINT_HEAD_BYTES and (bool(rotary) or B * H * S <= _MAX_JOINT_ROWS)
         if ctx.joint:
             q, k = (torch.empty((B, H, S, cols), dtype=mixed.dtype, device=mixed.device) for _ in range(2))
             ext.torch_launch_qkv_rms_forward(q, k, mixed, ws[0], ws[1], ctx.epsilon, *(tables or (None, None)))
             ctx.save_for_backward(mixed, ws[0], ws[1], *(tables or ()))
             return q, k, v_out
-        outs, stats = [], []   # wider heads: one strided norm per tensor
+        outs, stats = [], []   # wider heads, more rows: one strided norm per tensor
         for x, w in ((q_in, ws[0]), (k_in, ws[1])):
             out = torch.empty((B, H, S, cols), dtype=mixed.dtype, device=mixed.device)
             invvar = torch.empty(B * H * S, device=mixed.device, dtype=torch.float32)

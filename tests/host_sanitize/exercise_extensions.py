@@ -51,6 +51,14 @@ def main(directory):
         for args in ((h, h, h, s, s, 8, 3072, 1e-6, st), (h,) * 3, (h, h, s, s, h, h, s, st, st, 8, 3072), ()):
             raises(fn, *args)
             n += 1
+    # the whole calls leave operands on the CPU to their caller, whatever their shapes
+    for v in views:
+        assert rms.rms_forward(v, w, 128, 1e-6) is None and rms.rms_backward(v, x, w, r, 128, False) is None
+        assert rms.qkv_forward(v, w, w, 1e-6, None, None) is None
+        assert rms.qkv_forward(torch.zeros(1, 2, 3, 384, dtype=bf), v, w, 1e-6, v, v) is None
+        assert ada.adaln_forward(v, s, s, 3072, 1e-6, False) is None and ada.adaln_forward(h, v, v, 0, 1e-6, True) is None
+        assert ada.gated_forward(v, h, s, s, s, 1e-6) is None and ada.gated_forward(h, h, v, v, v, 1e-6) is None
+        n += 8
     assert rms.supported(128, x) and rms.supported(3072, torch.zeros(1)) and not rms.supported(3071, x)
     assert not rms.supported(128, torch.zeros(1, dtype=torch.int32))
     print(f"sanitised extensions ok: {n} refused calls")

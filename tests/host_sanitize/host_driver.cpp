@@ -25,6 +25,28 @@ extern "C" void __hipRegisterFunction(void **, const void *, char *, const char 
 extern "C" void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, int) {}
 extern "C" void __hipUnregisterFatBinary(void **) {}
 
+// A launch is recorded instead of made: an error here tells the launch site that there is nothing to start.
+static struct {
+    int launches;
+    dim3 grid, block;
+} g_launch;
+extern "C" hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t) {
+    ++g_launch.launches;
+    g_launch.grid = grid;
+    g_launch.block = block;
+    return hipErrorNotReady;
+}
+// No device, or one of g_cus compute units.
+static int g_cus = 0;
+extern "C" hipError_t hipGetDevice(int *dev) {
+    *dev = 0;
+    return g_cus > 0 ? hipSuccess : hipErrorNoDevice;
+}
+extern "C" hipError_t hipDeviceGetAttribute(int *value, hipDeviceAttribute_t, int) {
+    *value = g_cus;
+    return g_cus > 0 ? hipSuccess : hipErrorNoDevice;
+}
+
 static int g_failures = 0;
 #define EXPECT(cond)                                                                  \
     do {                                                                              \
@@ -127,6 +149,33 @@ static void argument_checks(bool have_gpu) {
            TT_NORM_EINVAL);
     EXPECT(tt_rmsnorm_rope_forward_strided(a, f, b, c, f, f, 2, 1, 2, 3, 0, 0, 64, 64, 1e-6, TT_NORM_BF16, nullptr) ==
            TT_NORM_EUNSUPPORTED);
+    // the joint QK-norm: null and misaligned pointers, heads of more than 64 pieces, tables only for head dimension 128
+    EXPECT(tt_qkv_rmsnorm_supported(512, TT_NORM_BF16) == 1 && tt_qkv_rmsnorm_supported(520, TT_NORM_BF16) == 0);
+    EXPECT(tt_qkv_rmsnorm_supported(256, TT_NORM_F32) == 1 && tt_qkv_rmsnorm_supported(260, TT_NORM_F32) == 0);
+    EXPECT(tt_qkv_rmsnorm_supported(INT64_MIN, TT_NORM_F16) == 0 && tt_qkv_rmsnorm_supported(128, 7) == 0);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, nullptr, nullptr, nullptr, 0, 1, 4, 2, 128, 1e-6, TT_NORM_BF16, nullptr) ==
+           TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, odd, d, d, nullptr, nullptr, 0, 1, 4, 2, 128, 1e-6, TT_NORM_BF16, nullptr) ==
+           TT_NORM_EALIGN);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, nullptr, nullptr, 0, 1, -4, 2, 128, 1e-6, TT_NORM_BF16, nullptr) ==
+           TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, nullptr, nullptr, 0, 1, 4, 2, 520, 1e-6, TT_NORM_BF16, nullptr) ==
+           TT_NORM_EUNSUPPORTED);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, f, f, 5, 1, 4, 2, 128, 1e-6, TT_NORM_BF16, nullptr) == TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, f, f, 4, 1, 4, 2, 64, 1e-6, TT_NORM_BF16, nullptr) == TT_NORM_EUNSUPPORTED);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, f, nullptr, 4, 1, 4, 2, 128, 1e-6, TT_NORM_BF16, nullptr) == TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, nullptr, nullptr, 0, 1, 4, 1 << 20, 128, 1e-6, TT_NORM_BF16, nullptr) ==
+           TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_forward(a, b, c, d, d, nullptr, nullptr, 0, (int64_t)1 << 31, 1, 2, 128, 1e-6, TT_NORM_BF16,
+                                  nullptr) == TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_forward(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 1, 0, 2, 128, 1e-6,
+                                  TT_NORM_BF16, nullptr) == TT_NORM_OK);
+    EXPECT(tt_qkv_rmsnorm_backward(a, nullptr, b, c, c, c, d, d, d, nullptr, nullptr, 0, 1, 4, 2, 128, 1e-6, TT_NORM_BF16,
+                                   nullptr, 0, nullptr) == TT_NORM_EINVAL);
+    EXPECT(tt_qkv_rmsnorm_backward(a, b, b, c, odd, c, d, d, d, nullptr, nullptr, 0, 1, 4, 2, 128, 1e-6, TT_NORM_BF16,
+                                   nullptr, 0, nullptr) == TT_NORM_EALIGN);
+    EXPECT(tt_qkv_rmsnorm_backward_workspace_bytes(1, 4, 2, 520, TT_NORM_BF16) == 0);
+    EXPECT(tt_qkv_rmsnorm_backward_workspace_bytes(0, 4, 2, 128, TT_NORM_BF16) == 0);
     // gated / residual forms on rows that are not whole 16-byte pieces, or wider than 1024 of them
     EXPECT(tt_gated_residual_adaln_forward(a, b, f, f, a, b, c, d, a, 1, 4, 3076, 1e-6, TT_NORM_BF16, nullptr) ==
            TT_NORM_EUNSUPPORTED);
@@ -160,6 +209,38 @@ static void argument_checks(bool have_gpu) {
     }
 }
 
+// HIP counts the threads of a grid dimension in 32 bits; rows beyond that are walked, or numbered over another dimension.
+static void forward_grids() {
+    void *a = fake(0x10000), *b = fake(0x20000), *c = fake(0x30000), *d = fake(0x40000);
+    float *f = reinterpret_cast<float *>(fake(0x50000));
+    const auto fits = [] {
+        const dim3 g = g_launch.grid;
+        return g.x > 0 && (uint64_t)g.x * g_launch.block.x <= 0xffffffffu && g.y <= 65535 && g.z <= 65535;
+    };
+    const struct { int64_t S, cols; int dtype; } heads[] = {
+        {1, 128, TT_NORM_BF16}, {29700, 128, TT_NORM_BF16}, {(int64_t)1 << 30, 8, TT_NORM_BF16},
+        {((int64_t)1 << 27) + 5, 128, TT_NORM_BF16}, {((int64_t)1 << 28) - 1, 512, TT_NORM_F16}, {(int64_t)1 << 28, 64, TT_NORM_F32}};
+    for (const auto &h : heads)
+        for (int rope = 0; rope <= (h.cols == 128); ++rope) {
+            g_launch.launches = 0;
+            (void)tt_qkv_rmsnorm_forward(a, b, c, d, d, rope ? f : nullptr, rope ? f : nullptr, rope ? h.S : 0, 1, h.S, 1,
+                                         h.cols, 1e-6, h.dtype, nullptr);
+            EXPECT(g_launch.launches == 1 && fits());
+            // every token has a workgroup: a workgroup's wavefronts take at most 32 tokens, none fewer than one
+            const int64_t groups = (int64_t)g_launch.grid.x * g_launch.grid.z;
+            EXPECT(groups * 32 >= h.S && groups <= h.S + g_launch.grid.z);
+        }
+    g_cus = 256;
+    for (int64_t rows : {(int64_t)70000000, (int64_t)300000000}) {
+        g_launch.launches = 0;
+        (void)tt_adaln_forward(a, f, f, b, c, d, 1, rows, 260, 1e-6, TT_NORM_F32, nullptr);
+        EXPECT(g_launch.launches == 1 && fits());
+        (void)tt_rmsnorm_forward(a, f, b, c, rows, 520, 1e-6, TT_NORM_BF16, nullptr);
+        EXPECT(g_launch.launches == 2 && fits());
+    }
+    g_cus = 0;
+}
+
 int main() {
     int n = 0;
     const bool have_gpu = hipGetDeviceCount(&n) == hipSuccess && n > 0;
@@ -168,6 +249,7 @@ int main() {
     predicates();
     row_plans();
     argument_checks(have_gpu);
+    forward_grids();
     if (g_failures) {
         fprintf(stderr, "%d expectation(s) failed\n", g_failures);
         return 1;

@@ -101,3 +101,17 @@ def test_gated_modulation_rows_of_unlike_shapes(gpu_device, batch, gate, scale, 
     for x, y, a in zip(got[2:], want[2:], shaped):
         assert x.shape == a.shape and torch.equal(x, y.reshape(a.shape))
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_projections_of_too_many_rows_take_one_norm_per_tensor(gpu_device, monkeypatch):
+    """Past the joint kernels' row count (lowered here) the call runs one strided norm per tensor: the same values."""
+    from teletron_amd import fusedlayers as FL
+    args, grads = _operands("qkv", torch.bfloat16, gpu_device)
+    args[0] = _shifted(args[0])   # prepared in Python, where the route is chosen
+    want = _run("qkv", args, grads)
+    monkeypatch.setattr(FL, "_MAX_JOINT_ROWS", args[0].numel() // 384 - 1)
+    got = _run("qkv", args, grads)
+    assert all(torch.equal(x, y) for x, y in zip(got[:4], want[:4]))
+    # dweights: 222 terms near 1 in another order, at most 222 * 222 * 2^-24 = 3e-3 apart in fp32, then one bf16 rounding each
+    for x, y in zip(got[4:], want[4:]):
+        torch.testing.assert_close(x.float(), y.float(), rtol=2.0 ** -7, atol=3e-3)
