@@ -21,12 +21,14 @@
 // tensor (two forward; two backward, one copy of the value gradient, two reducers): forward 122 against 150 us, with
 // tables 137 against 151; backward 258 against 297, with tables 262 against 303.
 //
-// Forward: wavefronts of a workgroup along the tokens (the others along the heads) and heads per wavefront.  Without
-// tables four consecutive token groups of one head (tokens along two / one wavefronts: 127 us; two heads: 126).  With
-// them, two heads of one token group share the 1 KiB of table per token (one head 143 us, three 136, four 149; two heads
-// with two / four wavefronts along the tokens 139 / 155).
-#ifndef TTN_QKV_FWD_TOKEN_WAVES
-#define TTN_QKV_FWD_TOKEN_WAVES (ROPE ? 1 : 4)
+// Forward: wavefronts of a workgroup along the tokens (1 << LOG2 of the four; the others along heads and samples) and heads
+// per wavefront.  Without tables four consecutive token groups of one head (tokens along two / one wavefronts: 127 us; two
+// heads: 126).  With them, two heads of one token group share the 1 KiB of table per token (one head 143 us, three 136, four
+// 149; two heads with two / four wavefronts along the tokens 139 / 155).  Where there are fewer token groups, or fewer heads
+// and samples, than the split asks for, the launch moves wavefronts to the other side instead of leaving them idle
+// (4096 x 1 token x 24 heads x 128: 77 us with three of four idle, 43 now; one rotated head of 300000 tokens 216 / 106).
+#ifndef TTN_QKV_FWD_TOKEN_WAVES_LOG2
+#define TTN_QKV_FWD_TOKEN_WAVES_LOG2 (ROPE ? 0 : 2)
 #endif
 #ifndef TTN_QKV_FWD_HEADS
 #define TTN_QKV_FWD_HEADS (ROPE ? 2 : 1)
@@ -46,6 +48,8 @@
 namespace ttn {
 
 constexpr int kLoadNt = 2;  // cache policy of the row loads: non-temporal
+constexpr int kRowWavesLog2 = 2;
+static_assert(1 << kRowWavesLog2 == kRowWaves);
 
 // FULL: the row fills its LANES lanes, so its length is known at compile time.
 template <typename T, int LANES_, bool FULL>
@@ -72,27 +76,30 @@ template <typename T, int LANES, bool FULL, typename Rope>
 __global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q, T *__restrict__ k,
                                                               const T *__restrict__ mixed, const T *__restrict__ wq,
                                                               const T *__restrict__ wk, const Rope rope, int64_t S, int H,
-                                                              uint32_t head_blocks, uint32_t outer, int c_arg, float eps) {
+                                                              uint32_t head_groups, uint32_t outer, int tw_log2, int c_arg,
+                                                              float eps) {
     using G = HeadGeom<T, LANES, FULL>;
     using E = Elem<T>;
     constexpr bool ROPE = Rope::kOn;
     constexpr int VEC = G::VEC, RPW = G::RPW;
-    constexpr int TW = TTN_QKV_FWD_TOKEN_WAVES, HW = kRowWaves / TW, HR = TTN_QKV_FWD_HEADS;
+    constexpr int HR = TTN_QKV_FWD_HEADS;
     const int C = G::cols(c_arg);
     const int lane = threadIdx.x & 63;
     const int sub = lane / LANES;
     const int l = lane % LANES;
     const int wave = wave_id_in_block();
     const bool in = FULL || l * VEC < C;
-    const int64_t s0 = (((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * TW + wave % TW) * RPW;
+    // a wavefront's place among the token groups and among the (sample, group of HR heads) pairs
+    const int token_wave = wave & ((1 << tw_log2) - 1), outer_wave = wave >> tw_log2, outer_waves = kRowWaves >> tw_log2;
+    const int64_t s0 = ((((int64_t)blockIdx.z * gridDim.x + blockIdx.x) << tw_log2) + token_wave) * RPW;
     const bool ok = in && s0 + sub < S;
     const uint32_t from = (uint32_t)sub * (uint32_t)(H * 3 * C * (int)sizeof(T)) + l * 16;
     const uint32_t to = (uint32_t)(sub * C * (int)sizeof(T)) + l * 16;
     const u32x4 zero{0, 0, 0, 0};
 
-    for (uint32_t y = blockIdx.y; y < outer; y += gridDim.y) {
-        const int64_t b = y / head_blocks;
-        const int h0 = ((int)(y % head_blocks) * HW + wave / TW) * HR;
+    for (uint32_t y = blockIdx.y * outer_waves + outer_wave; y < outer; y += gridDim.y * outer_waves) {
+        const int64_t b = y / head_groups;
+        const int h0 = (int)(y % head_groups) * HR;
         const T *src = mixed + ((b * S + s0) * H + h0) * 3 * C;
         u32x4 xr[HR][2];
 #pragma unroll
@@ -279,15 +286,20 @@ template <typename T, int LANES, bool FULL, typename Rope>
 static void launch_qkv_fwd(const QkvSizes &z, void *q, void *k, const void *mixed, const void *wq, const void *wk,
                            const Rope &rope, float eps, hipStream_t stream) {
     [[maybe_unused]] constexpr bool ROPE = Rope::kOn;
-    constexpr int TW = TTN_QKV_FWD_TOKEN_WAVES, heads = kRowWaves / TW * TTN_QKV_FWD_HEADS;
-    const int head_blocks = (int)((z.H + heads - 1) / heads);
-    const int64_t outer = z.B * head_blocks;
-    const int64_t along = (z.token_groups() + TW - 1) / TW, layers = (along + kMostBlocks - 1) / kMostBlocks;
-    const dim3 grid((unsigned)((along + layers - 1) / layers), (unsigned)(outer < 65535 ? outer : 65535), (unsigned)layers);
+    constexpr int HR = TTN_QKV_FWD_HEADS;
+    const int64_t head_groups = (z.H + HR - 1) / HR, outer = z.B * head_groups;
+    int tw_log2 = TTN_QKV_FWD_TOKEN_WAVES_LOG2;  // no more wavefronts along the tokens than there are groups of them,
+    while (tw_log2 > 0 && (1 << (tw_log2 - 1)) >= z.token_groups()) --tw_log2;
+    // nor across them than there are groups of heads
+    while (tw_log2 < kRowWavesLog2 && (kRowWaves >> (tw_log2 + 1)) >= outer) ++tw_log2;
+    const int tw = 1 << tw_log2, outer_waves = kRowWaves >> tw_log2;
+    const int64_t along = (z.token_groups() + tw - 1) / tw, layers = (along + kMostBlocks - 1) / kMostBlocks;
+    const int64_t across = (outer + outer_waves - 1) / outer_waves;
+    const dim3 grid((unsigned)((along + layers - 1) / layers), (unsigned)(across < 65535 ? across : 65535), (unsigned)layers);
     RowKernelProfile prof(stream);
     qkv_fwd_kernel<T, LANES, FULL, Rope><<<grid, dim3(kRowThreads), 0, stream>>>(
-        (T *)q, (T *)k, (const T *)mixed, (const T *)wq, (const T *)wk, rope, z.S, (int)z.H, (uint32_t)head_blocks, (uint32_t)outer,
-        (int)z.cols, eps);
+        (T *)q, (T *)k, (const T *)mixed, (const T *)wq, (const T *)wk, rope, z.S, (int)z.H, (uint32_t)head_groups, (uint32_t)outer,
+        tw_log2, (int)z.cols, eps);
 }
 
 template <typename T, int LANES, bool FULL, typename Rope>

@@ -22,6 +22,10 @@ def capi(gpu_device):
 CASES = [
     (1, 1, 1, 128, 0), (2, 3, 5, 8, 0), (3, 17, 2, 64, 0), (1, 33, 7, 72, 0), (2, 15, 3, 256, 0), (1, 9, 4, 504, 0),
     (2, 5, 3, 512, 0), (1, 1501, 24, 128, 0), (2, 61, 5, 128, 61), (1, 67, 9, 128, 40), (1, 5, 1, 128, 1),
+    # few token groups or few heads: wavefronts of the forward workgroup on other samples or more tokens
+    (5, 6, 3, 128, 0), (9, 1, 1, 64, 0), (7, 1, 3, 128, 1), (1, 300, 1, 128, 290), (3, 21, 3, 128, 21),
+    # several runs of neighbouring heads per wavefront in the rotated backward, runs that straddle token groups and samples
+    (2, 1501, 24, 128, 1501), (1, 2999, 11, 128, 2950), (3, 1000, 9, 128, 990),
 ]
 
 
