@@ -262,6 +262,34 @@ def test_rotary_strided_writes_stay_inside(capi, gpu_device, B, S, H, n_rot):
     assert torch.equal(out, out2) and torch.equal(dview, dx2) and torch.equal(dw, dw2)
 
 
+@pytest.mark.parametrize("B,S,H,D,n_rot", [(1, 1001, 5, 128, 0), (2, 37, 7, 128, 20), (1, 130, 13, 72, 0), (3, 1, 1, 128, 1),
+                                           (2, 9, 3, 512, 0), (1, 2501, 9, 128, 2400)])
+def test_joint_qk_norm_writes_stay_inside(capi, gpu_device, B, S, H, D, n_rot):
+    from oracle import norm_oracle as O
+    dtype = torch.bfloat16
+    L, dt, s = capi.lib(), capi.BF16, _stream(gpu_device)
+    gen = torch.Generator(device=gpu_device).manual_seed(S)
+    mixed = torch.randn(B, S, H, 3 * D, device=gpu_device, generator=gen).to(dtype)
+    w = [(1 + 0.02 * torch.randn(D, device=gpu_device, generator=gen)).to(dtype) for _ in range(2)]
+    grads = [torch.randn(B, H, S, D, device=gpu_device, generator=gen).to(dtype) for _ in range(3)]
+    tables = [t.to(gpu_device) for t in O.make_rope_tables(n_rot, D, seed=S)] if n_rot else [None, None]
+    G = Guarded(gpu_device)
+    q, k, dmixed = G.new((B, H, S, D), dtype), G.new((B, H, S, D), dtype), G.new((B, S, H, 3 * D), dtype)
+    dws = [G.new((D,), dtype) for _ in range(2)]
+    n = L.tt_qkv_rmsnorm_backward_workspace_bytes(B, S, H, D, dt)
+    ws = G.bytes(n)
+    c, sn = (None if t is None else _p(t) for t in tables)
+    _ok(L, L.tt_qkv_rmsnorm_forward(_p(q), _p(k), _p(mixed), _p(w[0]), _p(w[1]), c, sn, n_rot, B, S, H, D, EPS, dt, s))
+    _ok(L, L.tt_qkv_rmsnorm_backward(_p(dmixed), _p(dws[0]), _p(dws[1]), *[_p(g) for g in grads], _p(mixed), _p(w[0]), _p(w[1]),
+                                     c, sn, n_rot, B, S, H, D, EPS, dt, _p(ws), n, s))
+    torch.cuda.synchronize()
+    G.check(f"joint qk norm B={B} S={S} H={H} D={D}")
+    q2, k2 = capi.qkv_rmsnorm_forward(mixed, *w, EPS, *tables)
+    dm2, *dw2 = capi.qkv_rmsnorm_backward(*grads, mixed, *w, EPS, *tables)
+    for x, y in zip((q, k, dmixed, *dws), (q2, k2, dm2, *dw2)):
+        assert torch.equal(x, y)
+
+
 def test_reference_contract_writes_stay_inside(capi, gpu_device):
     """The entry points with the reference's saved tensors (forward output / normalised rows)."""
     L, s = capi.lib(), _stream(gpu_device)

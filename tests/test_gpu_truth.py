@@ -141,6 +141,43 @@ def test_cfg2_qk_norm_with_rotary_embedding_full_shape(capi, gpu_device, n_rot):
         no_worse_than_eager(case, name, got, wnt, t)
 
 
+@pytest.mark.parametrize("n_rot", [0, 29700 - 256])
+def test_cfg2_joint_qk_norm_full_shape(capi, gpu_device, n_rot):
+    """The kernels the QK-norm call site runs, both tensors in one pass each way, at one CP=4 rank's shape."""
+    B, S, H, D = 1, 29700, 24, 128
+    gen = torch.Generator().manual_seed(22)
+    mixed = torch.randn(B, S, H, 3 * D, generator=gen).bfloat16()
+    w = [(1 + 0.02 * torch.randn(D, generator=gen)).bfloat16() for _ in range(2)]
+    grads = [torch.randn(B, H, S, D, generator=gen).bfloat16() for _ in range(3)]
+    tables = O.make_rope_tables(n_rot, D, seed=2) if n_rot else ()
+    t_g = [t.to(gpu_device) for t in tables]
+    m_g, w_g = mixed.to(gpu_device), [t.to(gpu_device) for t in w]
+    q, k = capi.qkv_rmsnorm_forward(m_g, *w_g, EPS, *t_g)
+    dmixed, *dws = capi.qkv_rmsnorm_backward(*[g.to(gpu_device) for g in grads], m_g, *w_g, EPS, *t_g)
+    assert torch.equal(dmixed[..., 2 * D:].transpose(1, 2).cpu(), grads[2])
+    for i, out in enumerate((q, k)):
+        x = mixed[..., i * D:(i + 1) * D].transpose(1, 2)
+        dx = dmixed[..., i * D:(i + 1) * D].transpose(1, 2)
+        case = f"cfg2_joint_{'qk'[i]}_{n_rot}"
+        if n_rot:
+            want = O.eager_qk_norm_rope_fwd_bwd(x, w[i], *tables, grads[i])
+            truth = O.truth_qk_norm_rope_fwd_bwd(x, w[i], *tables, grads[i])
+            excuse = O.rope_excuse(O.eager_rmsnorm(x, w[i]), want[0])
+        else:
+            want = O.eager_rmsnorm_fwd_bwd(x, w[i], grads[i])
+            truth = O.truth_rmsnorm_fwd_bwd(x, w[i], grads[i])
+            excuse = O.rmsnorm_excuse(want[0])
+        forward_bar(case, "out", out, want[0], excuse)
+        grad_bar(case, "dx", dx, want[1], allow=1e-5)
+        # a column of 712 800 terms may sum to almost nothing (-0.034 here, where eager has -0.036 and the same rounded
+        # products summed in 64 bits -0.0345): its scale is the L2 mass of its terms, about 800, of which fp32 sums in
+        # another order may differ by 2^-24 * sqrt(712 800) = 2^-14; the bar is four times that
+        terms = grads[i].float() * torch.nn.functional.normalize(x.float(), dim=-1) * D ** 0.5
+        assert O.colsum_outside(dws[i], want[2], terms.reshape(-1, D), dim=0, ulp=2.0 ** -12) == 0
+        for name, got, wnt, t in zip(("out", "dx", "dweight"), (out, dx, dws[i]), want, truth):
+            no_worse_than_eager(case, name, got, wnt, t)
+
+
 # ------------------------------------------------------------------ config 3
 
 def test_cfg3_adaln_full_shape(capi, gpu_device):
