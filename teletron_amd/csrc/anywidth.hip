@@ -85,27 +85,6 @@ struct LaneMask {
     }
 };
 
-// One row of `bytes` bytes in memory, its address wave-uniform (one row per wavefront): a buffer resource that ends
-// where the row does, so accesses of the padded geometry past its end read zeros and write nothing without a branch.
-template <int POLICY>
-struct BoundedRow {
-    __amdgpu_buffer_rsrc_t rsrc;
-    uint32_t off;
-    __device__ __forceinline__ BoundedRow(const void *base, uint32_t bytes, int l) : off(l * 16) {
-        const uint64_t a = reinterpret_cast<uint64_t>(base);
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-        rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0, bytes,
-                                                 RowWriter<1>::kRawDwords);
-    }
-    __device__ __forceinline__ u32x4 get(int piece) const {
-        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + piece * 16, 0, POLICY);
-    }
-    __device__ __forceinline__ void put(int piece, const u32x4 &v) const {
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off + piece * 16, 0, POLICY);
-    }
-};
-
 // The rows of one wavefront step: full wavefronts read their one row through a bounded resource, narrower rows
 // through per-lane addresses.  row_base is the lane's row.
 template <typename G>

@@ -416,8 +416,8 @@ struct RowWriter<1> {
                                                  kRawDwords);
     }
     __device__ __forceinline__ void put(int piece, const u32x4 &v) const {
-        // The piece goes into the vector offset, not into the scalar one: a 16-byte store must be followed by a wait
-        // state before its data registers are written again, and the compiler inserts it only for stores without a
+        // The piece goes into the vector offset, not into the scalar one: a 16-byte store must be followed by two wait
+        // states before its data registers are written again, and the compiler inserts them only for stores without a
         // scalar offset register.  With one, rows of fp32 whose pieces are formed in the same registers had the first
         // of a piece's four elements replaced by the next piece's, 784 of 25 million.
         __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off + piece * 16, 0, kSc1Nt);
@@ -440,6 +440,27 @@ struct RowReader {
     }
     __device__ __forceinline__ u32x4 get(int piece) const {
         return __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, piece * 16, POLICY);
+    }
+};
+
+// One row of `bytes` bytes in memory, its address wave-uniform (one row per wavefront): a buffer resource that ends
+// where the row does, so accesses of the padded geometry past its end read zeros and write nothing without a branch.
+template <int POLICY>
+struct BoundedRow {
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t off;
+    __device__ __forceinline__ BoundedRow(const void *base, uint32_t bytes, int l) : off(l * 16) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0, bytes,
+                                                 RowWriter<1>::kRawDwords);
+    }
+    __device__ __forceinline__ u32x4 get(int piece) const {
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + piece * 16, 0, POLICY);
+    }
+    __device__ __forceinline__ void put(int piece, const u32x4 &v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off + piece * 16, 0, POLICY);  // no scalar offset, as in RowWriter<1>
     }
 };
 

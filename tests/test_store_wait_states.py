@@ -1,6 +1,5 @@
-"""Machine code of the buffer-store row writer: the instruction after a 16-byte store must not write the registers the
-store takes its data from.  The compiler keeps that distance only for stores without a scalar offset register."""
-import os
+"""Machine code of the 16-byte buffer-store writers: the registers a store takes its data from must not be written within
+two wait states of it.  The compiler keeps that distance only for stores without a scalar offset register."""
 import re
 import subprocess
 
@@ -16,7 +15,7 @@ __global__ void rows(float *out, const float *x, const float *w) {
     const int l = threadIdx.x & 63;
     u32x4 piece = load16(reinterpret_cast<const u32x4 *>(x) + l);
     const u32x4 add = load16(reinterpret_cast<const u32x4 *>(w) + l);
-    const RowWriter<WRITER> o(out, l * 16);
+    const WRITER;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
         o.put(k * 64, piece);
@@ -25,6 +24,7 @@ __global__ void rows(float *out, const float *x, const float *w) {
     }
 }
 """
+WAIT_STATES = 2
 
 
 def _registers(operand):
@@ -35,21 +35,48 @@ def _registers(operand):
     return {int(m[1])} if m else set()
 
 
-@pytest.mark.parametrize("writer", [1])
-def test_store_data_is_not_overwritten_by_the_next_instruction(tmp_path, writer):
-    (tmp_path / "rows.hip").write_text(SOURCE)
-    asm = tmp_path / "rows.s"
-    subprocess.run([B.HIPCC, *B.HIP_FLAGS, "-w", f"-DWRITER={writer}", "-I" + B.CSRC, "--cuda-device-only", "-S",
-                    str(tmp_path / "rows.hip"), "-o", str(asm)], check=True, capture_output=True)
-    lines = [t for t in (l.split(";")[0].strip() for l in asm.read_text().splitlines()) if t and not t.startswith(".")]
-    stores = 0
-    for this, after in zip(lines, lines[1:]):
-        op, _, args = this.partition("\t") if "\t" in this else this.partition(" ")
+def _split(line):
+    op, _, args = line.replace("\t", " ").partition(" ")
+    return op, [a.strip() for a in args.split(",")]
+
+
+def overwritten(lines):
+    """(number of 16-byte buffer stores, those whose data an instruction within the wait states overwrites)."""
+    stores, bad = 0, []
+    for i, line in enumerate(lines):
+        op, args = _split(line)
         if op != "buffer_store_dwordx4":
             continue
         stores += 1
-        data = _registers(args.split(",")[0].strip())
-        next_op, _, next_args = after.partition("\t") if "\t" in after else after.partition(" ")
-        if next_op.startswith("v_"):
-            assert not data & _registers(next_args.split(",")[0].strip()), (this, after)
-    assert stores == 12
+        data, passed = _registers(args[0]), 0
+        for after in lines[i + 1:]:
+            if passed >= WAIT_STATES or after.endswith(":"):
+                break
+            next_op, next_args = _split(after)
+            if next_op.startswith("v_") and data & _registers(next_args[0]):
+                bad.append((line, after))
+            passed += int(next_args[0]) + 1 if next_op == "s_nop" else 1
+    return stores, bad
+
+
+def _assembly(tmp_path, writer):
+    (tmp_path / "rows.hip").write_text(SOURCE.replace("WRITER", writer))
+    asm = tmp_path / "rows.s"
+    subprocess.run([B.HIPCC, *B.HIP_FLAGS, "-w", "-I" + B.CSRC, "--cuda-device-only", "-S",
+                    str(tmp_path / "rows.hip"), "-o", str(asm)], check=True, capture_output=True)
+    lines = (l.split(";")[0].strip() for l in asm.read_text().splitlines())
+    return [t for t in lines if t and not t.startswith(".")]
+
+
+@pytest.mark.parametrize("writer", ["RowWriter<1> o(out, l * 16)", "BoundedRow<18> o(out, 12 * 1024, l)",
+                                    "BoundedRow<2> o(out, 12 * 1024, l)"])
+def test_store_data_is_not_overwritten_within_the_wait_states(tmp_path, writer):
+    stores, bad = overwritten(_assembly(tmp_path, writer))
+    assert stores == 12 and not bad
+
+
+@pytest.mark.parametrize("between,clean", [([], False), (["s_nop 0"], False), (["s_nop 1"], True), (["v_mov_b32 v9, v8"], False),
+                                           (["s_waitcnt vmcnt(0)", "s_nop 0"], True)])
+def test_the_check_sees_an_early_overwrite(between, clean):
+    lines = ["buffer_store_dwordx4 v[0:3], v4, s[0:3], 0 offen"] + between + ["v_mul_f32 v2, v2, v6", "s_endpgm"]
+    assert overwritten(lines) == (1, [] if clean else [(lines[0], "v_mul_f32 v2, v2, v6")])
