@@ -746,10 +746,14 @@ size_t tt_adaln_backward_workspace_bytes(int64_t batch, int64_t rows_per_sample,
     int st = TT_NORM_OK;
     const int cus = current_device_cus(&st);
     if (st != TT_NORM_OK) return 0;
-#define CALL(T, C) \
-    return (size_t)adaln_backward_plan<T, C>(batch, rows_per_sample, cus).blocks * 2 * C * sizeof(float)
+    size_t need = 0;
+#define CALL(T, C) need = (size_t)adaln_backward_plan<T, C>(batch, rows_per_sample, cus).blocks * 2 * C * sizeof(float)
     TTN_DISPATCH(dtype, cols, CALL);
 #undef CALL
+    if (cols == 3072) return need;
+    // the residual and gated forms of the other tuned width run on the any-width kernels, whose grid is another
+    const size_t any = anywidth_adaln_backward_workspace_bytes(batch, rows_per_sample, cols, dtype);
+    return any > need ? any : need;
 }
 
 int tt_adaln_backward(void *dx, void *dscale, void *dshift, const void *dout, const void *x,

@@ -241,6 +241,35 @@ static void forward_grids() {
     g_cus = 0;
 }
 
+// A backward call takes the workspace that its query asks for, in every form and at every width.
+static void workspace_queries() {
+    void *a = fake(0x10000), *b = fake(0x20000), *c = fake(0x30000), *d = fake(0x40000), *ws = fake(0x60000);
+    float *f = reinterpret_cast<float *>(fake(0x50000));
+    g_cus = 256;
+    for (int dt : {TT_NORM_BF16, TT_NORM_F32, TT_NORM_F16})
+        for (int64_t cols : {8, 64, 128, 256, 512, 520, 1536, 2048, 2560, 3072, 3328, 4096, 6400, 8192})
+            for (int64_t rows : {1, 5, 700, 4100, 29700, 1000000})
+                for (int64_t batch : {1, 2, 7, 300}) {
+                    if (!tt_norm_supported(cols, dt)) continue;
+                    const size_t n2 = tt_adaln_backward_workspace_bytes(batch, rows, cols, dt);
+                    const size_t n3 = tt_gated_residual_adaln_backward_workspace_bytes(batch, rows, cols, dt);
+                    const size_t n1 = tt_rmsnorm_backward_workspace_bytes(batch * rows, cols, dt);
+                    const size_t nq = tt_qkv_rmsnorm_backward_workspace_bytes(batch, rows, 3, cols, dt);
+                    const auto took = [&](int st) { return st != TT_NORM_EWORKSPACE; };
+                    EXPECT(took(tt_adaln_backward(a, b, c, d, a, b, f, f, batch, rows, cols, dt, ws, n2, nullptr)));
+                    EXPECT(took(tt_adaln_backward_seq_first(a, b, c, d, a, b, f, f, batch, rows, cols, dt, ws, n2, nullptr)));
+                    EXPECT(took(tt_adaln_backward_residual(a, b, c, d, a, b, c, f, f, batch, rows, cols, dt, ws, n2, nullptr)));
+                    EXPECT(took(tt_gated_residual_adaln_backward(a, b, c, c, c, d, a, b, a, d, d, f, f, batch, rows, cols, dt, ws,
+                                                                 n3, nullptr)));
+                    EXPECT(took(tt_rmsnorm_backward(a, b, c, d, a, f, batch * rows, cols, dt, ws, n1, nullptr)));
+                    EXPECT(took(tt_rmsnorm_backward_strided(a, b, c, d, a, f, batch, 1, rows, 0, 0, 2 * cols, 0, 0, cols, cols, dt,
+                                                            ws, n1, nullptr)));
+                    if (nq) EXPECT(took(tt_qkv_rmsnorm_backward(a, b, b, c, c, c, d, d, d, nullptr, nullptr, 0, batch, rows, 3, cols,
+                                                                1e-6, dt, ws, nq, nullptr)));
+                }
+    g_cus = 0;
+}
+
 int main() {
     int n = 0;
     const bool have_gpu = hipGetDeviceCount(&n) == hipSuccess && n > 0;
@@ -250,6 +279,7 @@ int main() {
     row_plans();
     argument_checks(have_gpu);
     forward_grids();
+    workspace_queries();
     if (g_failures) {
         fprintf(stderr, "%d expectation(s) failed\n", g_failures);
         return 1;

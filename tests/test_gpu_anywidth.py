@@ -330,6 +330,30 @@ def test_adaln_backward_residual_at_other_widths(capi, gpu_device, C, dtype):
     assert torch.equal(dxr, dx + other.to(gpu_device)) and torch.equal(dsr, ds) and torch.equal(dhr, dh)
 
 
+@pytest.mark.parametrize("dtype", [BF, F32])
+def test_residual_and_gated_forms_at_128_columns_past_the_tuned_grid(capi, gpu_device, dtype):
+    """The plain backward at 128 columns and the any-width kernels that have the other forms run different grids, hence
+    different partial rows: the one workspace query covers both."""
+    B, S, C = 2, 20001, 128
+    h, a, q, sc, sh, go, g2 = (t.to(gpu_device) for t in O.make_gated_inputs(B, S, C, dtype, seed=4))
+    _, mean, rstd = capi.adaln_forward(h, sc, sh, EPS)
+    dx, *sums = capi.adaln_backward(go, h, sc, mean, rstd)
+    dxr, *sums_r = capi.adaln_backward_residual(go, g2, h, sc, mean, rstd)
+    # fp32: s1 and s2 of a row are added in other lanes' order, and so is everything behind them
+    close = torch.equal if dtype == BF else lambda x, y: torch.allclose(x, y, rtol=1e-4, atol=1e-5)
+    assert close(dxr, dx + g2)
+    for got, want, terms in zip(sums_r, sums, (3 * go, go)):
+        colsum_ok(got, want.cpu(), terms.float().cpu(), 1, "residual sums")
+    h2, _, mean, rstd = capi.gated_residual_adaln_forward(h, a, q, sc, sh, EPS)
+    dh, da, dq, *sums_g = capi.gated_residual_adaln_backward(go, g2, h2, a, q, sc, mean, rstd)
+    dx, *sums = capi.adaln_backward(go, h2, sc, mean, rstd)
+    assert close(dh, dx + g2) and close(da, dh * q[:, None])
+    want = (dh.double() * a.double()).sum(1)
+    assert O.colsum_outside(dq.cpu(), want.cpu(), (dh.float() * a.float()).cpu(), dim=1) == 0
+    for got, want, terms in zip(sums_g, sums, (3 * go, go)):
+        colsum_ok(got, want.cpu(), terms.float().cpu(), 1, "gated sums")
+
+
 @pytest.mark.parametrize("C,dtype,B,S", [(3072, BF, 3, 129), (3072, F32, 2, 33), (1536, HF, 4, 65), (128, BF, 3, 1001),
                                          (64, BF, 5, 77), (3072, BF, 1, 100), (4096, BF, 2, 40)])
 def test_adaln_on_sequence_first_rows(capi, gpu_device, C, dtype, B, S):
