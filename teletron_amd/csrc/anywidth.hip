@@ -17,16 +17,18 @@
 #include "norm_host.h"
 
 // Rows of a full wavefront (33 pieces and more) are read and written through buffer resources that end with the row, and
-// the backward kernels request the next row between the two passes of the current one; what bounds them is the memory
-// system and, below some 50 MB per tensor, the fixed cost of a launch (ramp, last rows, flush of the column sums).
+// the backward kernels with registers for a second row (rows of up to six accesses, not the gated form) request it between
+// the two passes of the current one; what bounds them is the memory system and, below some 50 MB per tensor, the fixed
+// cost of a launch (ramp, last rows, flush of the column sums).
 // Measured as calls with the reducer behind them, against plain masked loads, no request ahead, two or three workgroups
 // per compute unit and one wavefront at a time in the flush: AdaLN backward 12000 x 1536 bf16 30.4 -> 25.1 us,
 // 8 x 1025 x 1536 fp16 26.4 -> 21.1, 12000 x 1024 24.5 -> 20.1, 40000 x 2560 149 -> 104 (five accesses per lane instead
 // of six, one of them empty), 30000 x 1536 fp32 105 -> 96; RMSNorm backward 12000 x 2560 51.7 -> 36.5; gated backward
-// 12000 x 2560 94 -> 71.  The packed forms of the products (RowParam, add_elements) measure the same here.
+// 12000 x 2560 94 -> 71.  The packed forms of the products (widerow.hip) measure the same here.
 
 // Cache policy (sc0 = 1, nt = 2, sc1 = 16) of full-wavefront rows: loads and forward stores non-temporal, backward
-// stores write-through as well (plain non-temporal: 1536 columns 184 instead of 182 us, 1024 196 / 186).
+// stores write-through as well (plain non-temporal: 1536 columns 184 instead of 182 us, 1024 196 / 186; strided views of
+// 6144 columns 140.6 / 137.4, of 4096 82.7 / 82.9, of 8192 and of 4096 fp32 the same).
 #ifndef TTN_ANY_LOAD_POLICY
 #define TTN_ANY_LOAD_POLICY 2
 #endif
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_bwd_kernel(
         keep_packed(gyp);
 
         // dx goes through its own strides: base = the wavefront's first row, the lane adds its row's distance
-        const RowOut<G, (TTN_ANY_BWD_STORE && CHUNKS <= 6), kBwdStore> wd(
+        const RowOut<G, TTN_ANY_BWD_STORE, kBwdStore> wd(
             dx + b.doff0, (uint32_t)((b.at.doff - b.doff0) * (int64_t)sizeof(T)) + l * 16, l, row_bytes);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
@@ -725,21 +727,29 @@ struct RmsOn {  // the RMSNorm kernels over one kind of row map
     struct Fwd {
         static int run(const RowPlan &p, void *out, float *rstd, const void *x, const void *w, const Map &map, int C,
                        double eps, hipStream_t stream) {
-            RowKernelProfile prof(stream);
-            anywidth_rmsnorm_fwd_kernel<T, LANES, CHUNKS, Map><<<dim3((unsigned)p.blocks), dim3(kRowThreads), 0, stream>>>(
-                (T *)out, rstd, (const T *)x, (const T *)w, map, C, (float)eps);
-            return TT_NORM_OK;
+            if constexpr (CHUNKS > 6 && std::is_same<Map, DenseRows>::value) {  // run on the wide-row kernels
+                return fail(TT_NORM_EUNSUPPORTED, "RMSNorm: dense rows of more than six 16-byte accesses per lane");
+            } else {
+                RowKernelProfile prof(stream);
+                anywidth_rmsnorm_fwd_kernel<T, LANES, CHUNKS, Map><<<dim3((unsigned)p.blocks), dim3(kRowThreads), 0, stream>>>(
+                    (T *)out, rstd, (const T *)x, (const T *)w, map, C, (float)eps);
+                return TT_NORM_OK;
+            }
         }
     };
     template <typename T, int LANES, int CHUNKS>
     struct Bwd {
         static int run(const RowPlan &p, void *dx, void *ws, const void *g, const void *x, const void *w,
                        const float *rstd, const Map &map, int C, hipStream_t stream) {
-            RowKernelProfile prof(stream);
-            anywidth_rmsnorm_bwd_kernel<T, LANES, CHUNKS, Map>
-                <<<dim3((unsigned)p.blocks), dim3(kRowThreads), (size_t)kRowWaves * C * sizeof(float), stream>>>(
-                    (T *)dx, (float *)ws, (const T *)g, (const T *)x, (const T *)w, rstd, map, C);
-            return TT_NORM_OK;
+            if constexpr (CHUNKS > 6 && std::is_same<Map, DenseRows>::value) {
+                return fail(TT_NORM_EUNSUPPORTED, "RMSNorm backward: dense rows of more than six 16-byte accesses per lane");
+            } else {
+                RowKernelProfile prof(stream);
+                anywidth_rmsnorm_bwd_kernel<T, LANES, CHUNKS, Map>
+                    <<<dim3((unsigned)p.blocks), dim3(kRowThreads), (size_t)kRowWaves * C * sizeof(float), stream>>>(
+                        (T *)dx, (float *)ws, (const T *)g, (const T *)x, (const T *)w, rstd, map, C);
+                return TT_NORM_OK;
+            }
         }
     };
 };

@@ -263,78 +263,6 @@ __device__ __forceinline__ u32x4 rounded_products<bf16_t>(const u32x4 &a, const 
     return u32x4{r0, r1, r2, r3};
 }
 
-// The resident second factor of gy = rnd(g * w) / gx = rnd(g * t): masked pairs (or packed halves) for
-// 2-byte rows, fp32 values for 4-byte rows.
-template <typename T, int CH>
-struct RowParam {
-    using E = Elem<T>;
-    using Factor = PairFactor<std::conditional_t<kHasDot2<T>, T, bf16_t>>;
-    Factor f[kHasDot2<T> ? CH : 1];
-    float v[kHasDot2<T> ? 1 : CH][E::VEC];
-    __device__ __forceinline__ void set(int k, const u32x4 &packed) {
-        if constexpr (kHasDot2<T>)
-            f[k].set(packed);
-        else
-            E::unpack(packed, v[k]);
-    }
-    // rnd(g * param) for access k, in the element type
-    __device__ __forceinline__ u32x4 times(int k, const u32x4 &g) const {
-        if constexpr (kHasDot2<T>) {
-            return rounded_products<T>(g, f[k]);
-        } else {
-            float gv[E::VEC];
-            E::unpack(g, gv);
-#pragma unroll
-            for (int j = 0; j < E::VEC; ++j) gv[j] *= v[k][j];
-            return E::pack(gv);
-        }
-    }
-};
-
-// acc += rnd(g * rnd(n)) per column, n the eight (four) fp32 values of the normalised row for this access
-template <typename T>
-__device__ __forceinline__ void add_rounded_products(float (&acc)[Elem<T>::VEC], const u32x4 &g,
-                                                     float (&n)[Elem<T>::VEC], uint32_t one_lo, uint32_t one_hi) {
-    using E = Elem<T>;
-    if constexpr (kHasDot2<T>) {
-        PairFactor<T> nf;
-        nf.set_rounded(n);
-        const u32x4 pp = rounded_products<T>(g, nf);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[2 * i] = dot2<T>(pp[i], one_lo, acc[2 * i]);
-            acc[2 * i + 1] = dot2<T>(pp[i], one_hi, acc[2 * i + 1]);
-        }
-    } else {
-        float gv[E::VEC];
-        E::unpack(g, gv);
-        E::round(n);
-#pragma unroll
-        for (int j = 0; j < E::VEC; ++j) n[j] *= gv[j];
-        E::round(n);
-#pragma unroll
-        for (int j = 0; j < E::VEC; ++j) acc[j] += n[j];
-    }
-}
-
-// acc += g per column
-template <typename T>
-__device__ __forceinline__ void add_elements(float (&acc)[Elem<T>::VEC], const u32x4 &g, uint32_t one_lo, uint32_t one_hi) {
-    using E = Elem<T>;
-    if constexpr (kHasDot2<T>) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[2 * i] = dot2<T>(g[i], one_lo, acc[2 * i]);
-            acc[2 * i + 1] = dot2<T>(g[i], one_hi, acc[2 * i + 1]);
-        }
-    } else {
-        float gv[E::VEC];
-        E::unpack(g, gv);
-#pragma unroll
-        for (int j = 0; j < E::VEC; ++j) acc[j] += gv[j];
-    }
-}
-
 // rnd(a * b) for the elements of one access, both packed
 template <typename T>
 __device__ __forceinline__ u32x4 packed_products(const u32x4 &a, const u32x4 &b) {
