@@ -45,7 +45,9 @@ extern "C" {
  *    up to 384 16-byte pieces (they took 3072 columns only); the measurement kernels tt_norm_stream_copy
  *    and tt_norm_stream_probe left this library for libteletron_probe.so (include/teletron_probe.h).
  * 3: the gated residual and residual entry points take every supported row (up to 1024 pieces); scratch passed
- *    to a backward entry point must be 16-byte aligned; TT_NORM_STATIC_SCRATCH_BYTES is 32 MiB. */
+ *    to a backward entry point must be 16-byte aligned; TT_NORM_STATIC_SCRATCH_BYTES is 32 MiB.
+ *    Added since, with nothing that was there changed: the joint QK-norm, tt_qkv_rmsnorm_supported / _forward /
+ *    _backward_workspace_bytes / _backward. */
 #define TT_NORM_ABI_VERSION 3
 
 enum tt_norm_status {
