@@ -79,8 +79,8 @@ WORKLOADS = {
                       "and PyTorch's copies (no normalization arithmetic: the bandwidth envelope the kernels live in)",
     "qkv-site-rope": "the QK-norm call site including the rotary embedding the attention forward applies to q and k "
                      "behind the norms (fp32 cos/sin tables [29700, 128]): QKVSplitNormFunction with the tables, "
-                     "forward + backward; traffic counted as 12 slice-sized tensors plus the two tables once per "
-                     "kernel launch (4 launches)",
+                     "forward + backward, one kernel each; traffic counted as 12 slice-sized tensors plus the two "
+                     "tables once per kernel",
     "qkv-site-rope-reference": "the same call site the reference's way with these kernels: torch.split, transpose, "
                                "contiguous copy, dense RMSNorm Function per tensor, then the rotary embedding as "
                                "PyTorch ops (the published apply_rotary_emb formula), torch.split's backward; same "
@@ -257,7 +257,7 @@ def build_workload(name, torch, capi, dev):
 
         fn = fused if name == "qkv-site-rope" else reference_way
         slice_bytes = B * H * S * D * 2
-        tensors = 12 + 4 * (2 * S * D * 4) / slice_bytes
+        tensors = 12 + 2 * (2 * S * D * 4) / slice_bytes
         return [(name.replace("-", "_") + "_fwd_bwd", fn, tensors)], slice_bytes, S, "bf16", gq
     if name in ("qkv-site", "qkv-site-reference"):
         from teletron_amd import fusedlayers as FL

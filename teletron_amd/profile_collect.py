@@ -26,8 +26,8 @@ import sys
 import time
 
 from teletron_amd.build import ROOT
-from teletron_amd.profile_summary import (CACHED_VARIANTS, CFG4_PASSES, PASS_COUNTERS, RUN_LENGTHS, VARIANTS, WIDE_VARIANTS,
-                                          WIDE_WORKLOADS, WORKLOAD_INFO)
+from teletron_amd.profile_summary import (CACHED_VARIANTS, CFG4_PASSES, PASS_COUNTERS, RUN_LENGTHS, TRAFFIC_WORKLOADS, VARIANTS,
+                                          WIDE_VARIANTS, WIDE_WORKLOADS, WORKLOAD_INFO)
 
 BENCH = ["python3", "bench.py"]
 QUICK = ["--steps", "3", "--warmup", "1", "--no-cpu-baseline"]
@@ -73,6 +73,9 @@ def workloads(directory, only):
         args = ["--steps", "30", "--warmup", "5", "--no-cpu-baseline", "--workload", w]
         run([*BENCH, *args], out=os.path.join(directory, f"bench_{w}.json"))
         trace(directory, f"trace_{w}", args)
+        if w in TRAFFIC_WORKLOADS:
+            pmc(directory, f"fetch_{w}", "FETCH_SIZE", [*QUICK, "--workload", w])
+            pmc(directory, f"write_{w}", "WRITE_SIZE", [*QUICK, "--workload", w])
 
 
 def stream(directory, only):

@@ -30,7 +30,7 @@ from teletron_amd.build import ROOT, kernel_source_digest
 
 PROFILES = os.path.join(ROOT, "profiles")
 DIR_SHOWN = "rocprof_out"   # the --dir argument as typed: what the summaries print in their commands
-OURS = ("rmsnorm_", "adaln_", "stream_copy", "stream_probe", "colreduce", "copy_rows")
+OURS = ("rmsnorm_", "adaln_", "qkv_", "stream_copy", "stream_probe", "colreduce", "copy_rows")
 BOX = "MI355X (gfx950, 256 CUs), ROCm 7.2, one GPU"
 
 
@@ -284,12 +284,29 @@ WORKLOAD_INFO = {
     "w5120-bf16": "wide-row kernels: RMSNorm + AdaLN fwd+bwd, 71 280 x 5120 bf16",
     "w8192-bf16": "wide-row kernels: RMSNorm + AdaLN fwd+bwd, 44 550 x 8192 bf16",
     "w4096-bf16-gated": "wide-row kernels: gated residual + AdaLN fwd (2R 2W) + bwd (4R 2W), 89 100 x 4096 bf16",
-    "qkv-site": "QK-norm call site through the autograd Function: q and k normalised on the strided views of the "
-                "fused QKV projection, gradients written straight into the projection's gradient",
+    "qkv-site": "QK-norm call site through the autograd Function: one kernel normalises q and k out of the fused QKV "
+                "projection, one writes the projection's whole gradient",
     "qkv-site-rope": "QK-norm call site with the rotary embedding fused behind the norm",
     "qkv-site-rope-reference": "the same call site the reference's way: split, transposing copy, dense RMSNorm, rotary "
                                "embedding as PyTorch ops",
 }
+TRAFFIC_WORKLOADS = ("qkv-site", "qkv-site-rope", "w1536-f16")   # with HBM bytes per launch besides the trace
+
+
+def _traffic_lines(directory, workload, tensor_bytes):
+    """Markdown lines: bytes each kernel of the workload reads and writes per launch, from its FETCH_SIZE and WRITE_SIZE
+    passes, scaled by what they counted for the copy of one tensor in the same run."""
+    found = [counters(os.path.join(directory, f"{kind}_{workload}")) for kind in ("fetch", "write")]
+    scale = [tensor_bytes / _find(c, "stream_copy_kernel")[n] for c, n in zip(found, ("FETCH_SIZE", "WRITE_SIZE"))]
+    lines = [f"HBM bytes per launch (`rocprofv3 --pmc FETCH_SIZE` and `--pmc WRITE_SIZE` over the same workload at 3 steps, scaled "
+             f"by the copy of one {tensor_bytes / 1e6:.1f} MB tensor):", "", "| kernel | read MB | in tensors | written MB | in tensors |",
+             "|---|---|---|---|---|"]
+    for k in sorted(set(found[0]) & set(found[1])):
+        if k.startswith(("stream_copy", "colreduce")):
+            continue
+        read, written = found[0][k]["FETCH_SIZE"] * scale[0], found[1][k]["WRITE_SIZE"] * scale[1]
+        lines.append(f"| `{k}` | {read / 1e6:.1f} | {read / tensor_bytes:.3f} | {written / 1e6:.1f} | {written / tensor_bytes:.3f} |")
+    return "\n".join(lines) + "\n"
 
 
 def workloads(directory):
@@ -315,6 +332,8 @@ bench.py's own (back-to-back) result for the same command without a profiler, wh
                               for k, v in b["per_call_untimed"].items())
             md.append(f"bench.py: {b['ms_per_step']:.4f} ms per step, {b['value']:.0f} GB/s "
                       f"({100 * b['frac_of_hbm_peak']:.1f} % of 8 TB/s); per call (HIP-event medians): {calls}.\n")
+            if os.path.isdir(os.path.join(directory, f"fetch_{w}")):
+                md.append(_traffic_lines(directory, w, b["config"]["tensor_bytes"]))
     with open(os.path.join(PROFILES, "bench_other_workloads_kernels.md"), "w") as f:
         f.write("\n".join(md))
     print("wrote profiles/bench_other_workloads_kernels.md")
