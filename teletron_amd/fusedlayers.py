@@ -17,7 +17,7 @@ What differs from the reference, on purpose:
   * both operators accept any row of whole 16-byte pieces (up to 8192 two-byte or
     4096 four-byte columns) in bf16, fp16 or fp32; 128 and 3072 columns
     run the tuned kernels; strided views are read in place at every width, the
-    gated and residual forms exist for rows of up to 384 pieces, the rotary form
+    gated and residual forms exist for every supported row, the rotary form
     for 128 columns;
   * gated_residual_layer_norm fuses the residual update in front of a modulated
     LayerNorm (dit_layerspec.py:152-163) into the norm, forward and backward;
@@ -303,7 +303,7 @@ class GatedResidualAdaLNFunction(Function):
     (dit_layerspec.py:152-167, :351-352), which the reference runs as separate
     elementwise kernels around the norm.  h, attn [B, S, C]; gate, scale, shift [B, C].
     h2 is the new residual stream; its gradient from later uses is folded into the
-    same backward pass.  C: 3072, or any supported row of up to 3072 two-byte / 1536 four-byte columns."""
+    same backward pass.  C: any supported row."""
 
     @staticmethod
     def forward(ctx, h, attn, gate, scale, shift, epsilon):
