@@ -25,14 +25,6 @@
 #ifndef TTN_ADALN_BWD_ROW_BUFFERS
 #define TTN_ADALN_BWD_ROW_BUFFERS 2
 #endif
-// Gated backward, 2-byte rows: when attn and e (the gradient arriving at h2) are fetched.
-//   0: with g and x, one row at a time
-//   1: at the start of a row's processing (they are needed in its second pass only), while g and x of
-//      the NEXT row are requested between the two passes (two g/x buffers)
-//   2: in the second pass, where they are used
-#ifndef TTN_GATED_OPERANDS
-#define TTN_GATED_OPERANDS 1
-#endif
 #ifndef TTN_ADALN_BWD_PREFETCH_MID
 #define TTN_ADALN_BWD_PREFETCH_MID 1
 #endif
@@ -95,22 +87,6 @@
 #endif
 
 namespace ttn {
-
-// Loads this sample's modulation row and returns t = rnd(1 + scale) packed in
-// the element type.
-template <typename T, int C>
-__device__ __forceinline__ void load_one_plus_scale(u32x4 *tr, const T *__restrict__ scale_row, int l) {
-    using G = RowGeom<T, C>;
-    using E = Elem<T>;
-#pragma unroll
-    for (int k = 0; k < G::CHUNKS; ++k) {
-        float v[G::VEC];
-        E::unpack(load16(reinterpret_cast<const u32x4 *>(scale_row) + k * G::LANES + l), v);
-#pragma unroll
-        for (int j = 0; j < G::VEC; ++j) v[j] = 1.0f + v[j];
-        tr[k] = E::pack(v);
-    }
-}
 
 // GATED = true: the normalised tensor is first formed as h2 = rnd(x + rnd(attn * gate[b])) (the
 // gated residual update that precedes the norm in the transformer blocks) and written out too.
@@ -295,7 +271,7 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
     constexpr int kRowBuffers = (sizeof(T) == 4 && C >= 1024) ? 1 : TTN_ADALN_BWD_ROW_BUFFERS;
     // A row's first pass starts only when the stores of the row before it have left the wavefront
     // (see the RMSNorm backward): 359 us with this wait, 366 us without, at 118 800 rows.
-    constexpr bool kDrainStores = TTN_BWD_DRAIN_STORES && TTN_ADALN_BWD_STORE && !GATED && kRowBuffers == 2 && C >= 1024;
+    constexpr bool kDrainStores = TTN_BWD_DRAIN_STORES && TTN_ADALN_BWD_STORE && kRowBuffers == 2 && C >= 1024;
     __shared__ __align__(16) float lds[kFlushLdsFloats<NSETS, C>];
     const int lane = threadIdx.x & 63;
     const int sub = lane / LANES;
@@ -313,29 +289,60 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
     [[maybe_unused]] const uint32_t one_lo = opaque_const(kOneLo<T>), one_hi = opaque_const(kOneHi<T>);
     [[maybe_unused]] float tv[kPackedProducts ? 1 : CHUNKS][VEC];
     [[maybe_unused]] Factor tf[kPackedProducts ? CHUNKS : 1];
-    {
-        u32x4 tr[CHUNKS];
-        load_one_plus_scale<T, C>(tr, scale + smp * C, l);
+    u32x4 tr[CHUNKS];
 #pragma unroll
-        for (int k = 0; k < CHUNKS; ++k) {
-            if constexpr (kPackedProducts)
-                tf[k].set(tr[k]);
-            else
-                E::unpack(tr[k], tv[k]);
-        }
-    }
+    for (int k = 0; k < CHUNKS; ++k) tr[k] = load16(reinterpret_cast<const u32x4 *>(scale + smp * C) + k * LANES + l);
 
     // gate[sample]: unpacked once for 2-byte elements; 4-byte rows have no registers to spare and
     // re-read it (cache hits) where it is used
     constexpr bool kGateResident = GATED && sizeof(T) == 2;
-    constexpr bool kEarlyOperands = kGateResident && TTN_GATED_OPERANDS == 0;    // attn, e fetched with g, x
-    constexpr bool kStartOperands = kGateResident && TTN_GATED_OPERANDS == 1;    // ... when processing starts
     [[maybe_unused]] float gatev[kGateResident ? CHUNKS : 1][VEC];
+    [[maybe_unused]] u32x4 gr[kGateResident ? CHUNKS : 1];
     if constexpr (kGateResident) {
 #pragma unroll
-        for (int k = 0; k < CHUNKS; ++k)
-            E::unpack(load16(reinterpret_cast<const u32x4 *>(gate + smp * C) + k * LANES + l), gatev[k]);
+        for (int k = 0; k < CHUNKS; ++k) gr[k] = load16(reinterpret_cast<const u32x4 *>(gate + smp * C) + k * LANES + l);
     }
+
+    // What bounds the gated (4 reads, 2 writes) and residual (3 reads, 1 write) forms is the memory system and, with one
+    // wavefront per SIMD, what of a row's latency nothing overlaps.  Their second-pass operands (attn and e, or e alone)
+    // have one register buffer, which is asked to hold the next row's piece as soon as the current row's has been used:
+    // those loads then have a row's time to arrive instead of the length of a first pass (gated, requested when a row's
+    // processing starts), or one buffer less is carried (residual, requested with g and x).  With it the gated form
+    // gains from waiting for the stores of the row before (kDrainStores), as the others do.  Calls with the reducer:
+    // gated 14 850 rows 110.5 -> 104.5 us, 29 700 205 -> 196, 256 14.7 -> 13.2; residual 29 700 133 -> 127, 118 800
+    // 522 -> 495.  Nothing of a row that does not exist is read (an empty resource).
+    constexpr bool kAheadOperands = (GATED || RES) && sizeof(T) == 2 && kRowBuffers == 2 && TTN_ADALN_BWD_PREFETCH_MID;
+    static_assert(!kAheadOperands || LANES == kWaveSize, "a wavefront's row has a wave-uniform address");
+    [[maybe_unused]] u32x4 an[kAheadOperands && GATED ? CHUNKS : 1], en[kAheadOperands ? CHUNKS : 1];
+    [[maybe_unused]] int64_t next_row = 0;
+    [[maybe_unused]] bool next_ok = false;
+    [[maybe_unused]] auto request_operands = [&](int k) {
+        // the loads stay here, spread over the second pass: scheduled together they measure 3 % slower (gated, 60 000 rows)
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int kPolicy = TTN_BWD_LOAD_POLICY >= 0 ? TTN_BWD_LOAD_POLICY : 2;
+        const uint32_t bytes = next_ok ? C * (uint32_t)sizeof(T) : 0;
+        if constexpr (GATED) an[k] = BoundedRow<kPolicy>(attn + next_row * C, bytes, l).get(k * LANES);
+        en[k] = BoundedRow<kPolicy>(e + next_row * C, e != nullptr ? bytes : 0, l).get(k * LANES);
+    };
+    auto prepare = [&] {
+        if constexpr (kAheadOperands) {
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k) request_operands(k);
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) {
+            float v[VEC];
+            E::unpack(tr[k], v);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
+            const u32x4 t = E::pack(v);
+            if constexpr (kPackedProducts)
+                tf[k].set(t);
+            else
+                E::unpack(t, tv[k]);
+            if constexpr (kGateResident) E::unpack(gr[k], gatev[k]);
+        }
+    };
 
     float acc[NSETS][CHUNKS][VEC];  // [0] = dscale, [1] = dshift, [2] = dgate
 #pragma unroll
@@ -347,7 +354,7 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
 
     struct RowRegs {
         u32x4 g[CHUNKS], x[CHUNKS];
-        u32x4 a[kEarlyOperands ? CHUNKS : 1], e[(kEarlyOperands || RES) ? CHUNKS : 1];
+        u32x4 e[(RES && !kAheadOperands) ? CHUNKS : 1];
         float r, mu;
         int64_t row;
         int64_t first;  // element offset of the wavefront's first row (wave-uniform)
@@ -388,19 +395,14 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
             b.x[k] = b.ok ? load16_stream(px + k * LANES) : u32x4{0, 0, 0, 0};
         }
 #endif
-        if constexpr (RES) {
+        if constexpr (RES && !kAheadOperands) {
             const u32x4 *pe = reinterpret_cast<const u32x4 *>(e + b.row * C) + l;
 #pragma unroll
             for (int k = 0; k < CHUNKS; ++k) b.e[k] = b.ok ? load16_stream(pe + k * LANES) : u32x4{0, 0, 0, 0};
         }
-        if constexpr (kEarlyOperands) {  // otherwise these two are fetched where they are used
-            const u32x4 *pa = reinterpret_cast<const u32x4 *>(attn + b.row * C) + l;
-            const u32x4 *pe = reinterpret_cast<const u32x4 *>(e + b.row * C) + l;
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k) b.a[k] = b.ok ? load16_stream(pa + k * LANES) : u32x4{0, 0, 0, 0};
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k)
-                b.e[k] = (b.ok && e != nullptr) ? load16_stream(pe + k * LANES) : u32x4{0, 0, 0, 0};
+        if constexpr (kAheadOperands) {
+            next_row = b.row;
+            next_ok = b.ok;
         }
         // one row per wavefront: its statistics come through the scalar cache
         const int64_t srow = LANES == kWaveSize ? wave_uniform(b.row) : b.row;
@@ -410,16 +412,6 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
     auto process = [&](const RowRegs &b, auto &&between_passes) {
         const float r = b.r, mu = b.mu;
         const float nmr = -(mu * r);  // xhat = x*r + nmr
-        [[maybe_unused]] u32x4 ar[kStartOperands ? CHUNKS : 1], er[kStartOperands ? CHUNKS : 1];
-        if constexpr (kStartOperands) {
-            const u32x4 *pa = reinterpret_cast<const u32x4 *>(attn + b.row * C) + l;
-            const u32x4 *pe = reinterpret_cast<const u32x4 *>(e + b.row * C) + l;
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k) ar[k] = b.ok ? load16_stream(pa + k * LANES) : u32x4{0, 0, 0, 0};
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k)
-                er[k] = (b.ok && e != nullptr) ? load16_stream(pe + k * LANES) : u32x4{0, 0, 0, 0};
-        }
         // pass 1: gx = rnd(g*t) kept packed; s1 = sum_c gx; s2 = sum_c gx * xhat
         u32x4 gxp[CHUNKS];
         float s1 = 0.0f, s2 = 0.0f;
@@ -455,6 +447,7 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
         }
         s1 = group_sum<LANES>(s1);
         s2 = group_sum<LANES>(s2);
+        if constexpr (kAheadOperands) next_ok = false;  // until the next row is asked for
         between_passes();
         if constexpr (kHasDot2<T> && !FROM_XNORM) s2 = r * (s2 - mu * s1);
         const float m1 = s1 / (float)C, m2 = s2 / (float)C;
@@ -483,12 +476,9 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
             if constexpr (GATED) {
                 float ev[VEC], av[VEC], dav[VEC];
                 E::round(o);  // the norm's dx, materialised in the element type
-                if constexpr (kEarlyOperands) {
-                    E::unpack(b.e[k], ev);
-                    E::unpack(b.a[k], av);
-                } else if constexpr (kStartOperands) {
-                    E::unpack(er[k], ev);
-                    E::unpack(ar[k], av);
+                if constexpr (kAheadOperands) {
+                    E::unpack(en[k], ev);
+                    E::unpack(an[k], av);
                 } else {
                     const int64_t at = b.row * (C / VEC) + l + k * LANES;
                     const u32x4 zero{0, 0, 0, 0};
@@ -518,12 +508,13 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
                 if constexpr (RES) {
                     float ev[VEC];
                     E::round(o);  // the norm's dx, materialised in the element type
-                    E::unpack(b.e[k], ev);
+                    E::unpack(kAheadOperands ? en[k] : b.e[k], ev);
 #pragma unroll
                     for (int j = 0; j < VEC; ++j) o[j] += ev[j];
                 }
                 if (b.ok) wd.put(k * LANES, E::pack(o));
             }
+            if constexpr (kAheadOperands) request_operands(k);
             if constexpr (kPackedColumnSums) {
                 Factor nf;  // the normalised row in the element type
                 if constexpr (FROM_XNORM)
@@ -552,10 +543,7 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
     const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
     const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
     int64_t grp = (int64_t)slot * kRowWaves + wave;
-    if constexpr (kStartOperands)
-        row_pipeline<2, true, RowRegs>(grp, groups, stride, fetch, process);
-    else
-        row_pipeline<kRowBuffers, TTN_ADALN_BWD_PREFETCH_MID != 0, RowRegs>(grp, groups, stride, fetch, process);
+    row_pipeline<kRowBuffers, TTN_ADALN_BWD_PREFETCH_MID != 0, RowRegs>(grp, groups, stride, fetch, process, prepare);
     wave_clock_mark(kClockAdalnBwd, 2);  // rows done; what follows is the workgroup's partial row
     flush_column_partials<G, NSETS>(acc, partial + (int64_t)blockIdx.x * (NSETS * C), lds);
     wave_clock_mark(kClockAdalnBwd, 1);

@@ -17,7 +17,7 @@
 #include "norm_host.h"
 
 // Rows of a full wavefront (33 pieces and more) are read and written through buffer resources that end with the row, and
-// the backward kernels with registers for a second row (rows of up to six accesses, not the gated form) request it between
+// the backward kernels with registers for a second row (rows of up to six accesses; gated from three on) request it between
 // the two passes of the current one; what bounds them is the memory system and, below some 50 MB per tensor, the fixed
 // cost of a launch (ramp, last rows, flush of the column sums).
 // Measured as calls with the reducer behind them, against plain masked loads, no request ahead, two or three workgroups
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_bwd_kernel(
         }
     };
     row_pipeline<CHUNKS <= 6 ? 2 : 1, true, Row>(
-        (int64_t)blockIdx.x * kRowWaves + wave, groups, stride, fetch, process);
+        (int64_t)blockIdx.x * kRowWaves + wave, groups, stride, fetch, process, [] {});
     flush_partials_anywidth<G, 1>(acc, partial + (int64_t)blockIdx.x * C, lds, C, m);
 }
 
@@ -501,18 +501,40 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
     const LaneMask<G> m(l, C / VEC);
     const uint32_t row_bytes = (uint32_t)(C * (int)sizeof(T));
 
-    u32x4 tr[CHUNKS];  // t = rnd(1 + scale[sample])
+    u32x4 tr[CHUNKS];  // t = rnd(1 + scale[sample]), formed behind the first row's requests
     load_param<G>(tr, scale + b * C, l, m);
-#pragma unroll
-    for (int k = 0; k < CHUNKS; ++k) {
-        float v[VEC];
-        E::unpack(tr[k], v);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
-        tr[k] = E::pack(v);
-    }
     [[maybe_unused]] u32x4 qr[GATED ? CHUNKS : 1];
     if constexpr (GATED) load_param<G>(qr, gate + b * C, l, m);
+
+    // Gated, rows of three accesses and more: attn and e have one register buffer, which is asked to hold the next row's piece as
+    // soon as the current row's has been used, as in adaln.hip (with g and x, one row at a time: 43402 x 1152 bf16 115.6 us,
+    // now 106.0; 3906 x 1536 22.4 / 20.5; 24414 x 2048 111.6 / 110.0; 8 x 1025 x 1536 fp16 38.5 / 37.1).  Narrower rows
+    // take them with g and x, one row at a time (ahead: 48828 x 1024 112.6 / 115.2, 50000 x 512 62.8 / 64.4), and so does
+    // the residual form, which has registers for two rows (ahead it gains 2-4 % at most widths and loses 8 % at 1152).
+    constexpr bool kAhead = GATED && CHUNKS >= 3;
+    [[maybe_unused]] u32x4 an[kAhead ? CHUNKS : 1], en[kAhead ? CHUNKS : 1];
+    [[maybe_unused]] int64_t next_row = 0;
+    [[maybe_unused]] bool next_ok = false;
+    [[maybe_unused]] auto request_operands = [&](int k) {
+        __builtin_amdgcn_sched_barrier(0);  // spread over the second pass
+        const uint32_t bytes = next_ok ? row_bytes : 0;
+        an[k] = BoundedRow<kLoad>(attn + next_row * C, bytes, l).get(k * LANES);
+        en[k] = BoundedRow<kLoad>(e + next_row * C, e != nullptr ? bytes : 0, l).get(k * LANES);
+    };
+    auto prepare = [&] {
+        if constexpr (kAhead) {
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k) request_operands(k);
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) {
+            float v[VEC];
+            E::unpack(tr[k], v);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
+            tr[k] = E::pack(v);
+        }
+    };
 
     float acc[NSETS][CHUNKS][VEC];  // [0] = dscale, [1] = dshift, [2] = dgate
 #pragma unroll
@@ -524,7 +546,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
 
     struct Row {
         u32x4 g[CHUNKS], x[CHUNKS];
-        u32x4 e[(GATED || RES) ? CHUNKS : 1], a[GATED ? CHUNKS : 1];
+        u32x4 e[(GATED || RES) && !kAhead ? CHUNKS : 1], a[GATED && !kAhead ? CHUNKS : 1];
         float r, mu;
         int64_t first;  // element offset of the wavefront's first row
         bool ok;
@@ -539,8 +561,12 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
         q.first = lay.row(b, grp * RPW) * C;
         load_row<G>(q.g, g + row * C, l, q.ok, m, row_bytes);
         load_row<G>(q.x, x + row * C, l, q.ok, m, row_bytes);
-        if constexpr (GATED || RES) load_row<G>(q.e, e + row * C, l, q.ok && e != nullptr, m, row_bytes);
-        if constexpr (GATED) load_row<G>(q.a, attn + row * C, l, q.ok, m, row_bytes);
+        if constexpr ((GATED || RES) && !kAhead) load_row<G>(q.e, e + row * C, l, q.ok && e != nullptr, m, row_bytes);
+        if constexpr (GATED && !kAhead) load_row<G>(q.a, attn + row * C, l, q.ok, m, row_bytes);
+        if constexpr (kAhead) {
+            next_row = wave_uniform(row);
+            next_ok = q.ok;
+        }
         const int64_t srow = LANES == kWaveSize ? wave_uniform(row) : row;
         q.r = q.ok ? rstd[srow] : 0.0f;
         q.mu = q.ok ? mean[srow] : 0.0f;
@@ -576,6 +602,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
         }
         s1 = group_sum<LANES>(s1);
         s2 = group_sum<LANES>(s2);
+        if constexpr (kAhead) next_ok = false;  // until the next row is asked for
         between_passes();
         if constexpr (kHasDot2<T>) s2 = r * (s2 - mu * s1);
         const float m1 = s1 / (float)C, m2 = s2 / (float)C;
@@ -604,7 +631,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
             if constexpr (GATED || RES) {
                 float ev[VEC];
                 E::round(o);  // the norm's dx, materialised in the element type
-                E::unpack(q.e[k], ev);
+                E::unpack(kAhead ? en[k] : q.e[k], ev);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) o[j] += ev[j];
             }
@@ -613,7 +640,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
             if constexpr (GATED) {
                 float av[VEC], qv[VEC];
                 E::unpack(dxp, o);  // dh as stored
-                E::unpack(q.a[k], av);
+                E::unpack(kAhead ? an[k] : q.a[k], av);
                 E::unpack(qr[k], qv);
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) {
@@ -625,12 +652,13 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) acc[2][k][j] += av[j];
             }
+            if constexpr (kAhead) request_operands(k);
             add_columns<T>(acc[1][k], q.g[k]);                                    // dshift += g (padding: g = 0)
             add_columns<T>(acc[0][k], packed_products<T>(q.g[k], E::pack(xn)));  // dscale += rnd(g * rnd(xhat))
         }
     };
-    row_pipeline<GATED ? 1 : 2, true, Row>((int64_t)slot * kRowWaves + wave, groups, stride, fetch,
-                                                                     process);
+    row_pipeline<GATED && !kAhead ? 1 : 2, true, Row>((int64_t)slot * kRowWaves + wave, groups, stride, fetch, process,
+                                          prepare);
     flush_partials_anywidth<G, NSETS>(acc, partial + (int64_t)blockIdx.x * (NSETS * C), lds, C, m);
 }
 

@@ -525,24 +525,31 @@ __device__ __forceinline__ void wave_clock_mark(int, int) {}
 // loads of a row, `process(buf, mid)` consumes them and calls `mid()` once
 // between its two register passes.  grp advances by `stride` and is
 // wave-uniform, so every branch here is too.
-//   NBUF = 1 : plain loop (load, process, store; nothing else in flight).
+// `prepare()` runs once, behind the requests of the first row: what a kernel forms from its parameters (which it has
+// requested before) then costs that row no time of its own.  A wavefront without rows never calls it.
+//   NBUF = 1 : one row at a time, the next one requested when the current one is done.
 //   NBUF = 2, MID = false : the next row is requested before the current one is processed.
 //   NBUF = 2, MID = true  : the next row is requested half-way through the current one.
-template <int NBUF, bool MID, typename RowRegs, typename Fetch, typename Process>
+template <int NBUF, bool MID, typename RowRegs, typename Fetch, typename Process, typename Prepare>
 __device__ __forceinline__ void row_pipeline(int64_t grp, int64_t groups, int64_t stride, Fetch &&fetch,
-                                             Process &&process) {
+                                             Process &&process, Prepare &&prepare) {
     static_assert(NBUF == 1 || NBUF == 2, "one or two row buffers");
     auto nothing = [] {};
+    if (grp >= groups) return;
     if constexpr (NBUF == 1) {
-        for (; grp < groups; grp += stride) {
-            RowRegs a;
-            fetch(a, grp);
+        RowRegs a;
+        fetch(a, grp);
+        prepare();
+        for (;;) {
             process(a, nothing);
+            grp += stride;
+            if (grp >= groups) return;
+            fetch(a, grp);
         }
     } else {
-        if (grp >= groups) return;
         RowRegs buf0, buf1;
         fetch(buf0, grp);
+        prepare();
         // one row: process `cur`, requesting the row after it into `nxt`; false when it was the last
         auto step = [&](RowRegs &cur, RowRegs &nxt) -> bool {
             const int64_t ahead = grp + stride;

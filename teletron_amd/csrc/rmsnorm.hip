@@ -221,16 +221,20 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
     [[maybe_unused]] float wv[(kPackedProducts && !FROM_OUT) ? 1 : CHUNKS][VEC];
     [[maybe_unused]] Factor wf[kPackedProducts ? CHUNKS : 1];
     [[maybe_unused]] float winv[FROM_OUT ? CHUNKS : 1][VEC];  // 1/weight for the saved-output variant
+    u32x4 wr[CHUNKS];
 #pragma unroll
-    for (int k = 0; k < CHUNKS; ++k) {
-        const u32x4 wr = load16(reinterpret_cast<const u32x4 *>(w) + k * LANES + l);
-        if constexpr (kPackedProducts) wf[k].set(wr);
-        if constexpr (!kPackedProducts || FROM_OUT) E::unpack(wr, wv[k]);
-        if constexpr (FROM_OUT) {
+    for (int k = 0; k < CHUNKS; ++k) wr[k] = load16(reinterpret_cast<const u32x4 *>(w) + k * LANES + l);
+    auto prepare = [&] {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) winv[k][j] = __builtin_amdgcn_rcpf(wv[k][j]);
+        for (int k = 0; k < CHUNKS; ++k) {
+            if constexpr (kPackedProducts) wf[k].set(wr[k]);
+            if constexpr (!kPackedProducts || FROM_OUT) E::unpack(wr[k], wv[k]);
+            if constexpr (FROM_OUT) {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) winv[k][j] = __builtin_amdgcn_rcpf(wv[k][j]);
+            }
         }
-    }
+    };
 
     float acc[1][CHUNKS][VEC];
 #pragma unroll
@@ -402,12 +406,12 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(C >= 1024 ? TTN
     };
 
     if constexpr (kRun == 1) {
-        row_pipeline<kRowBuffers, TTN_RMS_BWD_PREFETCH_MID != 0, RowRegs>(me, groups, waves, fetch, process);
+        row_pipeline<kRowBuffers, TTN_RMS_BWD_PREFETCH_MID != 0, RowRegs>(me, groups, waves, fetch, process, prepare);
     } else {
         // runs this wavefront starts: m = 0, 1, ... with (m * waves + me) * kRun < groups
         const int64_t all_runs = (groups + kRun - 1) / kRun;
         const int64_t my_runs = all_runs > me ? (all_runs - me + waves - 1) / waves : 0;
-        row_pipeline<kRowBuffers, TTN_RMS_BWD_PREFETCH_MID != 0, RowRegs>(0, my_runs * kRun, 1, fetch, process);
+        row_pipeline<kRowBuffers, TTN_RMS_BWD_PREFETCH_MID != 0, RowRegs>(0, my_runs * kRun, 1, fetch, process, prepare);
     }
     flush_column_partials<G, 1>(acc, partial + (int64_t)blockIdx.x * C, lds);
 }
