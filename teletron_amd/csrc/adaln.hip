@@ -39,15 +39,20 @@
 #endif
 // Dynamic LDS requested by the forward launch (0: none).  Only a throttle on how many
 // one-shot workgroups a compute unit holds at once; the kernel does not touch it.
-// AdaLN forward spends longer in the ALU per row than RMSNorm forward and wants all the
-// wavefronts its registers and its staged parameters allow (six workgroups per compute unit for
-// 2-byte rows: 236 us at 118 800 rows against 238 with four and 280 with three).  The gated form
-// moves twice the bytes per row (2 reads + 2 writes) and streams best with three workgroups per
-// compute unit (12 KiB on top of its 30 KiB: 482 vs 509 us between backward launches).  4-byte rows
-// carry twice the bytes per wavefront: 40 KiB on top of the staged modulation rows leaves two
-// workgroups per compute unit (232 vs 244 us at 59 400 rows).
+// With its row requested before the parameters are staged, a two-byte workgroup streams best four to a compute unit
+// while the grid is short (16 KiB on top of its 24 KiB: 14 850 rows 34.0 us against 34.3 with six and 34.5 with three,
+// 4000 rows 10.0 / 10.1 / 11.9) and three once it refills every compute unit many times (24 KiB: 118 800 rows 240.5 us
+// against 244.6 with four and 250.7 with six; 80 000 rows 165 either way).  The gated form runs unthrottled, five by its
+// registers and LDS (118 800 rows 489 us, 493 with three; 4000 rows 20.9 / 22.2).  4-byte rows carry twice the bytes per
+// wavefront: 40 KiB on top of the staged modulation rows leaves two workgroups per compute unit (59 400 rows 243 us, 260
+// with three); gated, 16 KiB leave three (8192 rows 70.2 us, 72.9 with two).
 #ifndef TTN_ADALN_FWD_DYN_LDS
-#define TTN_ADALN_FWD_DYN_LDS (C >= 1024 ? (sizeof(T) == 4 ? 40960 : (GATED ? 12288 : 0)) : 0)
+#define TTN_ADALN_FWD_DYN_LDS                                                                        \
+    (C < 1024           ? 0                                                                          \
+     : GATED            ? (sizeof(T) == 4 ? 16384 : 0)                                               \
+     : sizeof(T) == 4   ? 40960                                                                      \
+     : p.blocks < 64 * (int64_t)cus ? 16384                                                          \
+                        : 24576)
 #endif
 // Backward row fetch: all of g's accesses, then all of x's (two contiguous 6 KiB runs per
 // wavefront at 3072 columns) rather than alternating 1 KiB pieces; worth ~0.7 %.
@@ -118,41 +123,69 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(sizeof(T) == 2 
     constexpr int kPieces = C / VEC;  // 16-byte pieces per parameter row
     constexpr int kPlanes = VEC / 4;
     __shared__ u32x4 lds_t[kPlanes][kPieces], lds_h[kPlanes][kPieces], lds_g[GATED ? kPieces : 1];
-    for (int i = threadIdx.x; i < kPieces; i += kRowThreads) {
-        float v[VEC], h[VEC];
-        E::unpack(load16(reinterpret_cast<const u32x4 *>(scale + b * C) + i), v);
+    // The modulation row is requested first and the wavefront's row right behind it, before the staging waits for the
+    // former: a workgroup of the one-shot grid then spends one memory latency less (4000 x 3072 bf16 11.1 -> 10.7 us, 29 700 64.9 -> 63.4,
+    // 118 800 245 -> 241; gated fp32 8192 rows 74.4 -> 70.2, bf16 4000 rows 22.0 -> 20.9; 1500 rows 6.4 -> 6.5).
+    constexpr int kShare = (kPieces + kRowThreads - 1) / kRowThreads;  // pieces of a parameter row per thread
+    u32x4 ps[kShare], ph[kShare];
+    [[maybe_unused]] u32x4 pg[GATED ? kShare : 1];
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
-        E::round(v);  // t = 1 + scale in the element type
-        E::unpack(load16(reinterpret_cast<const u32x4 *>(shift + b * C) + i), h);
-#pragma unroll
-        for (int p = 0; p < kPlanes; ++p) {
-            lds_t[p][i] = u32x4{as_u32(v[4 * p]), as_u32(v[4 * p + 1]), as_u32(v[4 * p + 2]), as_u32(v[4 * p + 3])};
-            lds_h[p][i] = u32x4{as_u32(h[4 * p]), as_u32(h[4 * p + 1]), as_u32(h[4 * p + 2]), as_u32(h[4 * p + 3])};
+    for (int n = 0; n < kShare; ++n) {
+        const int i = threadIdx.x + n * kRowThreads;
+        if (i < kPieces) {
+            ps[n] = load16(reinterpret_cast<const u32x4 *>(scale + b * C) + i);
+            ph[n] = load16(reinterpret_cast<const u32x4 *>(shift + b * C) + i);
+            if constexpr (GATED) pg[n] = load16(reinterpret_cast<const u32x4 *>(gate + b * C) + i);
         }
-        if constexpr (GATED) lds_g[i] = load16(reinterpret_cast<const u32x4 *>(gate + b * C) + i);
+    }
+    const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
+    const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
+    u32x4 xr[CHUNKS];
+    [[maybe_unused]] u32x4 ar[GATED ? CHUNKS : 1];
+    auto fetch = [&](int64_t grp) {
+        const int64_t rs = grp * RPW + sub;  // row inside the sample
+        const bool ok = rs < rows_per_sample;
+        const int64_t row = lay.row(b, rs);
+        const u32x4 *px = reinterpret_cast<const u32x4 *>(x + row * C) + l;
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) xr[k] = ok ? load16_stream(px + k * LANES) : u32x4{0, 0, 0, 0};
+        if constexpr (GATED) {
+            const u32x4 *pa = reinterpret_cast<const u32x4 *>(attn + row * C) + l;
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k) ar[k] = ok ? load16_stream(pa + k * LANES) : u32x4{0, 0, 0, 0};
+        }
+    };
+    int64_t grp = (int64_t)slot * kRowWaves + wave;
+    fetch(grp);  // a row past the end reads nothing
+#pragma unroll
+    for (int n = 0; n < kShare; ++n) {
+        const int i = threadIdx.x + n * kRowThreads;
+        if (i < kPieces) {
+            float v[VEC], h[VEC];
+            E::unpack(ps[n], v);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
+            E::round(v);  // t = 1 + scale in the element type
+            E::unpack(ph[n], h);
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) {
+                lds_t[p][i] = u32x4{as_u32(v[4 * p]), as_u32(v[4 * p + 1]), as_u32(v[4 * p + 2]), as_u32(v[4 * p + 3])};
+                lds_h[p][i] = u32x4{as_u32(h[4 * p]), as_u32(h[4 * p + 1]), as_u32(h[4 * p + 2]), as_u32(h[4 * p + 3])};
+            }
+            if constexpr (GATED) lds_g[i] = pg[n];
+        }
     }
     __syncthreads();
 
-    const int64_t groups = (rows_per_sample + RPW - 1) / RPW;
-    const int64_t stride = (int64_t)blocks_per_sample * kRowWaves;
-    for (int64_t grp = (int64_t)slot * kRowWaves + wave; grp < groups; grp += stride) {
-        const int64_t rs = grp * RPW + sub;  // row inside the sample
+    for (; grp < groups; grp += stride) {
+        const int64_t rs = grp * RPW + sub;
         const bool ok = rs < rows_per_sample;
         const int64_t row = lay.row(b, rs);
         // where the wavefront writes starts at its first row; the lane adds the distance to its own row
         const int64_t first = lay.row(b, grp * RPW) * C;
         const uint32_t lane_bytes = (uint32_t)(sub * lay.row_stride * C * sizeof(T)) + l * 16;
-        const u32x4 *px = reinterpret_cast<const u32x4 *>(x + row * C) + l;
-        u32x4 xr[CHUNKS];
-#pragma unroll
-        for (int k = 0; k < CHUNKS; ++k) xr[k] = ok ? load16_stream(px + k * LANES) : u32x4{0, 0, 0, 0};
         if constexpr (GATED) {
-            const u32x4 *pa = reinterpret_cast<const u32x4 *>(attn + row * C) + l;
             const RowWriter<TTN_ADALN_FWD_STORE> wh(h2_out + first, lane_bytes);
-            u32x4 ar[CHUNKS];
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k) ar[k] = ok ? load16_stream(pa + k * LANES) : u32x4{0, 0, 0, 0};
 #pragma unroll
             for (int k = 0; k < CHUNKS; ++k) {
                 float hv[VEC], av[VEC], gv[VEC];
@@ -234,6 +267,7 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(sizeof(T) == 2 
             for (int j = 0; j < VEC; ++j) v[j] += hv[j];
             if (ok) wo.put(k * LANES, E::pack(v));
         }
+        if (grp + stride < groups) fetch(grp + stride);
     }
     wave_clock_mark(kClockAdalnFwd, 1);
 }
