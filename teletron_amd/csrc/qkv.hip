@@ -22,16 +22,41 @@
 // us, with tables 137 against 151; backward 258 against 297, with tables 262 against 303.
 //
 // Forward: wavefronts of a workgroup along the tokens (1 << LOG2 of the four; the others along heads and samples) and heads
-// per wavefront.  Without tables four consecutive token groups of one head (tokens along two / one wavefronts: 127 us; two
-// heads: 126).  With them, two heads of one token group share the 1 KiB of table per token (one head 143 us, three 136, four
-// 149; two heads with two / four wavefronts along the tokens 139 / 155).  Where there are fewer token groups, or fewer heads
-// and samples, than the split asks for, the launch moves wavefronts to the other side instead of leaving them idle
-// (4096 x 1 token x 24 heads x 128: 77 us with three of four idle, 43 now; one rotated head of 300000 tokens 216 / 106).
+// per wavefront (HR).  With tables, two heads of one token group share the 1 KiB of table per token (one head 143 us, three
+// 136, four 149; two heads with two / four wavefronts along the tokens 139 / 155).  Without tables four consecutive token
+// groups of one head (tokens along two / one wavefronts: 127 us) or of two, whichever keeps the chip busier: two heads per
+// wavefront double what a wavefront has in flight, which wins once every compute unit has four workgroups of one head to
+// choose from (1500 x 24 x 128 bf16 10.0 -> 9.3 us, 3000 x 16 x 64 6.9 -> 6.2; below, half the wavefronts is what counts:
+// 256 x 24 x 128 3.4 / 3.6) and loses on long streams of whole rows (6000 x 24 x 128 29.1 either way, 29700 128 / 131).
+// Rows that leave lanes empty keep gaining (5208 x 12 x 80 12.1 -> 10.9, 30000 53.3 -> 50.3, 52083 90.8 -> 90.1).
+// Where there are fewer token groups, or fewer heads and samples, than the split asks for, the launch moves wavefronts to
+// the other side instead of leaving them idle (4096 x 1 token x 24 heads x 128: 77 us with three of four idle, 43 now; one
+// rotated head of 300000 tokens 216 / 106).
 #ifndef TTN_QKV_FWD_TOKEN_WAVES_LOG2
 #define TTN_QKV_FWD_TOKEN_WAVES_LOG2 (ROPE ? 0 : 2)
 #endif
-#ifndef TTN_QKV_FWD_HEADS
-#define TTN_QKV_FWD_HEADS (ROPE ? 2 : 1)
+#ifndef TTN_QKV_FWD_TWO_HEADS_FROM
+#define TTN_QKV_FWD_TWO_HEADS_FROM 4  // workgroups of one head per compute unit
+#endif
+#ifndef TTN_QKV_FWD_TWO_HEADS_BELOW
+#define TTN_QKV_FWD_TWO_HEADS_BELOW (FULL ? 32 : 1 << 20)
+#endif
+// Forward, tokens a multiple of 4 KiB apart in the projection: the pieces of one head then lie at one offset of the
+// memory's 4 KiB interleave, and a launch that walks all tokens of one head before the next reads from a part of the
+// channels only.  There it takes the heads of 2048 tokens before the next 2048 (bf16, 16 x 128: 24414 tokens 85.9 -> 74.1 us,
+// 8000 27.7 -> 25.9; 32 x 64 86.2 -> 76.7; fp32 16 x 64 84.0 -> 75.1; 1024 or 4096 tokens at a time within 3 %).  Other strides
+// are better off with the longest contiguous writes (24 x 128 128 us, 133 in pieces), and so are fewer than three such
+// pieces (4000 tokens 15.2 / 15.6) and rotated four-byte rows, whose two heads are 2.5 KiB in one run (91.9 / 94.3).
+constexpr int64_t kInterleave = 4096, kTileTokens = 2048;
+// Forward with tables: dynamic LDS the kernel does not touch, as a throttle on a long grid whose workgroups are all busy:
+// five to a compute unit stream better than eight (24 heads, 29700 tokens 142.5 -> 135.7 us, 7681 39.2 -> 38.1, 4000 22.3 ->
+// 21.8; four the same, six 138).  A short grid wants every wavefront (2500 tokens 15.5 / 15.9), and so does one whose heads leave
+// wavefronts of a workgroup idle (12 heads, 30000 tokens 74.7 / 77.9).
+#ifndef TTN_QKV_FWD_ROPE_LDS
+#define TTN_QKV_FWD_ROPE_LDS 32768
+#endif
+#ifndef TTN_QKV_FWD_ROPE_LDS_FROM
+#define TTN_QKV_FWD_ROPE_LDS_FROM 10  // workgroups per compute unit
 #endif
 // Backward: persistent, for the column sums.  Two workgroups per compute unit keep 10 MB requested (three: 271, four
 // 278 us; one with the next step's rows requested ahead 263-272).  The wavefront waits for its rows, works and
@@ -72,7 +97,7 @@ __device__ __forceinline__ float row_rstd(const u32x4 &x, int C, float eps) {
     return 1.0f / sqrtf(ss / (float)C + eps);
 }
 
-template <typename T, int LANES, bool FULL, typename Rope>
+template <typename T, int LANES, bool FULL, typename Rope, int HR>
 __global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q, T *__restrict__ k,
                                                               const T *__restrict__ mixed, const T *__restrict__ wq,
                                                               const T *__restrict__ wk, const Rope rope, int64_t S, int H,
@@ -82,7 +107,6 @@ __global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q,
     using E = Elem<T>;
     constexpr bool ROPE = Rope::kOn;
     constexpr int VEC = G::VEC, RPW = G::RPW;
-    constexpr int HR = TTN_QKV_FWD_HEADS;
     const int C = G::cols(c_arg);
     const int lane = threadIdx.x & 63;
     const int sub = lane / LANES;
@@ -286,24 +310,39 @@ struct QkvSizes {
     int64_t units() const { return B * token_groups() * H; }
 };
 
-template <typename T, int LANES, bool FULL, typename Rope>
-static void launch_qkv_fwd(const QkvSizes &z, void *q, void *k, const void *mixed, const void *wq, const void *wk,
-                           const Rope &rope, float eps, hipStream_t stream) {
-    [[maybe_unused]] constexpr bool ROPE = Rope::kOn;
-    constexpr int HR = TTN_QKV_FWD_HEADS;
+template <typename T, int LANES, bool FULL, typename Rope, int HR>
+static void launch_qkv_fwd_heads(const QkvSizes &z, int cus, void *q, void *k, const void *mixed, const void *wq, const void *wk,
+                                 const Rope &rope, float eps, hipStream_t stream) {
+    constexpr bool ROPE = Rope::kOn;
     const int64_t head_groups = (z.H + HR - 1) / HR, outer = z.B * head_groups;
     int tw_log2 = TTN_QKV_FWD_TOKEN_WAVES_LOG2;  // no more wavefronts along the tokens than there are groups of them,
     while (tw_log2 > 0 && (1 << (tw_log2 - 1)) >= z.token_groups()) --tw_log2;
     // nor across them than there are groups of heads
     while (tw_log2 < kRowWavesLog2 && (kRowWaves >> (tw_log2 + 1)) >= outer) ++tw_log2;
     const int tw = 1 << tw_log2, outer_waves = kRowWaves >> tw_log2;
-    const int64_t along = (z.token_groups() + tw - 1) / tw, layers = (along + kMostBlocks - 1) / kMostBlocks;
-    const int64_t across = (outer + outer_waves - 1) / outer_waves;
+    const int64_t along = (z.token_groups() + tw - 1) / tw, across = (outer + outer_waves - 1) / outer_waves;
+    // the grid is walked along the tokens of a layer, then across, then layer by layer
+    int64_t layers = (along + kMostBlocks - 1) / kMostBlocks;
+    const int64_t tiles = z.S / kTileTokens < 65535 ? z.S / kTileTokens : 65535;
+    if (z.H * 3 * z.cols * (int64_t)sizeof(T) % kInterleave == 0 && !(ROPE && sizeof(T) == 4) && tiles >= 3 && tiles > layers)
+        layers = tiles;
     const dim3 grid((unsigned)((along + layers - 1) / layers), (unsigned)(across < 65535 ? across : 65535), (unsigned)layers);
+    const bool throttle = ROPE && outer % outer_waves == 0 && along * across >= (int64_t)cus * TTN_QKV_FWD_ROPE_LDS_FROM;
     RowKernelProfile prof(stream);
-    qkv_fwd_kernel<T, LANES, FULL, Rope><<<grid, dim3(kRowThreads), 0, stream>>>(
+    qkv_fwd_kernel<T, LANES, FULL, Rope, HR><<<grid, dim3(kRowThreads), throttle ? TTN_QKV_FWD_ROPE_LDS : 0, stream>>>(
         (T *)q, (T *)k, (const T *)mixed, (const T *)wq, (const T *)wk, rope, z.S, (int)z.H, (uint32_t)head_groups, (uint32_t)outer,
         tw_log2, (int)z.cols, eps);
+}
+
+template <typename T, int LANES, bool FULL, typename Rope>
+static void launch_qkv_fwd(const QkvSizes &z, int cus, void *q, void *k, const void *mixed, const void *wq, const void *wk,
+                           const Rope &rope, float eps, hipStream_t stream) {
+    const int64_t blocks = z.units() / kRowWaves;  // of one head per wavefront
+    if (Rope::kOn || (z.H > 1 && blocks >= (int64_t)cus * TTN_QKV_FWD_TWO_HEADS_FROM &&
+                      blocks < (int64_t)cus * (TTN_QKV_FWD_TWO_HEADS_BELOW)))
+        launch_qkv_fwd_heads<T, LANES, FULL, Rope, 2>(z, cus, q, k, mixed, wq, wk, rope, eps, stream);
+    else if constexpr (!Rope::kOn)
+        launch_qkv_fwd_heads<T, LANES, FULL, Rope, 1>(z, cus, q, k, mixed, wq, wk, rope, eps, stream);
 }
 
 template <typename T, int LANES, bool FULL, typename Rope>
@@ -384,9 +423,12 @@ int tt_qkv_rmsnorm_forward(void *q, void *k, const void *mixed, const void *weig
     if (z.units() == 0) return TT_NORM_OK;
     st = check_qkv_ptrs(who, {q, k, mixed, weight_q, weight_k});
     if (st != TT_NORM_OK) return st;
+    int known = TT_NORM_OK;
+    int cus = current_device_cus(&known);
+    if (known != TT_NORM_OK) cus = 256;  // chooses the split only; without a device the launch itself reports it
     const bool full = qkv_pieces(cols, dtype) == z.lanes;
     const RopeTable rope{cos, sin, rope_tokens};
-#define CALL(T, L, F, R, r) launch_qkv_fwd<T, L, F, R>(z, q, k, mixed, weight_q, weight_k, r, (float)eps, (hipStream_t)stream)
+#define CALL(T, L, F, R, r) launch_qkv_fwd<T, L, F, R>(z, cus, q, k, mixed, weight_q, weight_k, r, (float)eps, (hipStream_t)stream)
     TTN_QKV_DISPATCH(CALL);
 #undef CALL
     return check_launch("qkv forward launch");

@@ -119,3 +119,33 @@ def test_an_infinite_gradient_stays_in_its_column(capi, gpu_device, D, dtype):
     a, b = (capi.qkv_rmsnorm_backward(*g, mixed, w, w, EPS) for g in (grads, bad))
     assert torch.equal(a[1][others], b[1][others]) and not bool(torch.isfinite(b[1][20]))
     assert torch.equal(a[2], b[2])
+
+
+# Both sides of the forward's rules: one head / two heads per wavefront (four workgroups of one head per compute unit; whole
+# rows back to one from 32 on; odd heads, a single head), heads by pieces of 2048 tokens where tokens lie whole 4 KiB apart
+# (three pieces and a ragged last one, and too few), and the throttled grid with tables.
+SPLITS = [
+    (1, 681, 24, 128, 0, BF), (1, 685, 24, 128, 0, BF), (3, 913, 5, 64, 0, HF), (1, 5463, 24, 128, 0, BF), (1, 20000, 1, 128, 0, BF),
+    (1, 4099, 5, 80, 0, BF), (2, 9001, 7, 96, 0, F32), (1, 6143, 16, 128, 0, BF), (1, 6151, 16, 128, 0, BF), (2, 6149, 8, 128, 0, F32),
+    (1, 8201, 32, 64, 0, HF), (1, 6147, 16, 128, 6100, BF), (1, 6147, 16, 128, 6147, F32), (1, 3417, 24, 128, 3400, BF),
+]
+
+
+@pytest.mark.parametrize("B,S,H,D,rotated,dtype", SPLITS)
+def test_forward_splits_equal_one_norm_per_tensor(capi, gpu_device, B, S, H, D, rotated, dtype):
+    gen = torch.Generator(device=gpu_device).manual_seed(S + D)
+    mixed = torch.randn(B, S, H, 3 * D, device=gpu_device, generator=gen).to(dtype)
+    w = [(1 + 0.02 * torch.randn(D, device=gpu_device, generator=gen)).to(dtype) for _ in range(2)]
+    cos, sin = (t.to(gpu_device) for t in O.make_rope_tables(rotated, D, seed=5)) if rotated else (None, None)
+    n = B * H * S * D
+    buf = torch.full((2, 4096 + n + 4096), 7.0, dtype=dtype, device=gpu_device)
+    q, k = (b[4096:-4096].view(B, H, S, D) for b in buf)
+    p = capi._p
+    capi._check(capi.lib().tt_qkv_rmsnorm_forward(p(q), p(k), p(mixed), p(w[0]), p(w[1]), p(cos), p(sin), rotated, B, S, H, D, EPS,
+                                                  capi._dt(mixed), capi._stream(mixed)), "tt_qkv_rmsnorm_forward")
+    for t, out in enumerate((q, k)):
+        x = mixed[..., t * D:(t + 1) * D].transpose(1, 2)
+        want = (capi.rmsnorm_rope_forward_strided(x, w[t], cos, sin, EPS) if rotated else
+                capi.rmsnorm_forward_strided(x, w[t], EPS))[0]
+        assert torch.equal(out, want)
+    assert bool((buf[:, :4096] == 7.0).all()) and bool((buf[:, -4096:] == 7.0).all())
