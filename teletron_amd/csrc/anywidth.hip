@@ -45,6 +45,12 @@
 #ifndef TTN_ANY_BWD_STORE
 #define TTN_ANY_BWD_STORE 1
 #endif
+// Into a strided view the rows of neighbouring heads come from different wavefronts: a row that does not end with a 128-byte
+// line then shares one, which the L2 puts together only if it is not written through (39062 x 16 x 80 bf16 101.8 -> 89.7 us;
+// rows of whole lines the same either way, 48828 x 16 x 64 65.4 / 65.0).
+#ifndef TTN_ANY_STRIDED_BWD_STORE
+#define TTN_ANY_STRIDED_BWD_STORE 0
+#endif
 // AdaLN forward of two-byte rows whose grid of one row per wavefront is larger than what the chip holds at a time: rows
 // per wavefront, which share the modulation row (100000 x 1024 bf16 one row 79.5, two 75.3 us; 30000 x 768 23.2 / 21.6;
 // 12000 x 1024 12.2 / 11.1).  A grid that fits gets longer with a second row (64 x 64 x 1024 fp32 8.6 instead of 7.0 us,
@@ -307,7 +313,7 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_rmsnorm_bwd_kernel(
         keep_packed(gyp);
 
         // dx goes through its own strides: base = the wavefront's first row, the lane adds its row's distance
-        const RowOut<G, TTN_ANY_BWD_STORE, kBwdStore> wd(
+        const RowOut<G, (std::is_same<Map, DenseRows>::value ? TTN_ANY_BWD_STORE : TTN_ANY_STRIDED_BWD_STORE), kBwdStore> wd(
             dx + b.doff0, (uint32_t)((b.at.doff - b.doff0) * (int64_t)sizeof(T)) + l * 16, l, row_bytes);
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
