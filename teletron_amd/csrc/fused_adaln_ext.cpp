@@ -258,16 +258,25 @@ static bool ready_modulation(const torch::Tensor &x, const torch::Tensor &scale,
     return batch == 1 || (x.dim() >= 2 && x.size(0) == batch);
 }
 
-// out, mean, inv_variance
-static c10::optional<Tensors> adaln_forward(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift,
-                                            int64_t cols, double epsilon, bool seq_first) {
-    if (!ready_rows(x, cols) || !ready(scale, x) || !ready(shift, x) || shift.numel() != scale.numel() ||
-        !ready_modulation(x, scale, cols, seq_first))
-        return c10::nullopt;
+static bool adaln_ready(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift, int64_t cols,
+                        bool seq_first) {
+    return ready_rows(x, cols) && ready(scale, x) && ready(shift, x) && shift.numel() == scale.numel() &&
+           ready_modulation(x, scale, cols, seq_first);
+}
+
+// out, mean, inv_variance of ready operands
+static Tensors adaln_run(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift, int64_t cols,
+                         double epsilon, bool seq_first) {
     const int64_t rows = x.numel() / cols;
     torch::Tensor out = at::empty_like(x), mean = row_statistics(x, rows), inv_variance = row_statistics(x, rows);
     adaln_forward_stats_impl(out, x, scale, shift, rows, cols, epsilon, mean, inv_variance, seq_first);
-    return Tensors{out, mean, inv_variance};
+    return {out, mean, inv_variance};
+}
+
+static c10::optional<Tensors> adaln_forward(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift,
+                                            int64_t cols, double epsilon, bool seq_first) {
+    if (!adaln_ready(x, scale, shift, cols, seq_first)) return c10::nullopt;
+    return adaln_run(x, scale, shift, cols, epsilon, seq_first);
 }
 
 // dinp, dscale, dshift; dres is the gradient the input receives from its other consumer, or None
@@ -285,21 +294,29 @@ static c10::optional<Tensors> adaln_backward(const torch::Tensor &dout, const c1
     return Tensors{dinp, dscale, dshift};
 }
 
-// h2, out, mean, inv_variance
-static c10::optional<Tensors> gated_forward(const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
-                                            const torch::Tensor &scale, const torch::Tensor &shift, double epsilon) {
-    if (h.dim() < 1 || !ready_rows(h, h.size(-1)) || !ready(attn, h) || attn.sizes() != h.sizes()) return c10::nullopt;
-    const int64_t cols = h.size(-1);
+static bool gated_ready(const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
+                        const torch::Tensor &scale, const torch::Tensor &shift) {
+    if (h.dim() < 1 || !ready_rows(h, h.size(-1)) || !ready(attn, h) || attn.sizes() != h.sizes()) return false;
     for (auto *t : {&gate, &scale, &shift})
-        if (!ready(*t, h) || t->numel() != scale.numel()) return c10::nullopt;
+        if (!ready(*t, h) || t->numel() != scale.numel()) return false;
     // backward shapes the gradients after gate and scale, the rows it keeps: shift's is scale's
-    if (shift.sizes() != scale.sizes()) return c10::nullopt;
-    if (!ready_modulation(h, scale, cols, false)) return c10::nullopt;
-    const int64_t rows = h.numel() / cols;
+    return shift.sizes() == scale.sizes() && ready_modulation(h, scale, h.size(-1), false);
+}
+
+// h2, out, mean, inv_variance of ready operands
+static Tensors gated_run(const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
+                         const torch::Tensor &scale, const torch::Tensor &shift, double epsilon) {
+    const int64_t cols = h.size(-1), rows = h.numel() / cols;
     torch::Tensor h2 = at::empty_like(h), out = at::empty_like(h);
     torch::Tensor mean = row_statistics(h, rows), inv_variance = row_statistics(h, rows);
     torch_launch_gated_adaln_forward(h2, out, h, attn, gate, scale, shift, rows, cols, epsilon, mean, inv_variance);
-    return Tensors{h2, out, mean, inv_variance};
+    return {h2, out, mean, inv_variance};
+}
+
+static c10::optional<Tensors> gated_forward(const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
+                                            const torch::Tensor &scale, const torch::Tensor &shift, double epsilon) {
+    if (!gated_ready(h, attn, gate, scale, shift)) return c10::nullopt;
+    return gated_run(h, attn, gate, scale, shift, epsilon);
 }
 
 // dh, dattn, dgate, dscale, dshift; dh2 may be None
@@ -315,7 +332,89 @@ static c10::optional<Tensors> gated_backward(const torch::Tensor &dout, const c1
     return Tensors{dh, dattn, dgate, dscale, dshift};
 }
 
+// ---- call sites (see torch_glue.h): AdaLNModelFunction, AdaLNResidualFunction and GatedResidualAdaLNFunction ----
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+
+struct AdalnSite : Function<AdalnSite> {
+    static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &x, const torch::Tensor &scale,
+                                 const torch::Tensor &shift, int64_t cols, double epsilon, bool seq_first) {
+        Tensors done = adaln_run(x, scale, shift, cols, epsilon, seq_first);
+        ctx->save_for_backward({x, scale, done[1], done[2]});
+        ctx->saved_data["cols"] = cols;
+        ctx->saved_data["seq_first"] = seq_first;
+        return done[0];
+    }
+    static Tensors backward(AutogradContext *ctx, Tensors grads) {
+        const Tensors kept = ctx->get_saved_variables();
+        Tensors d = taken(adaln_backward(prepared(grads[0], kept[0]), c10::nullopt, kept[0], kept[1], kept[2], kept[3],
+                                    ctx->saved_data["cols"].toInt(), ctx->saved_data["seq_first"].toBool()), "adaln_backward");
+        return {d[0], d[1], d[2], {}, {}, {}};
+    }
+};
+
+struct AdalnResidualSite : Function<AdalnResidualSite> {
+    static Tensors forward(AutogradContext *ctx, const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift,
+                           double epsilon) {
+        Tensors done = adaln_run(x, scale, shift, x.size(-1), epsilon, false);
+        ctx->set_materialize_grads(false);
+        ctx->save_for_backward({x, scale, done[1], done[2]});
+        return {x, done[0]};
+    }
+    static Tensors backward(AutogradContext *ctx, Tensors grads) {
+        const Tensors kept = ctx->get_saved_variables();
+        if (!grads[1].defined()) return {grads[0], {}, {}, {}};  // only the stream was used: the function was an identity
+        Tensors d = taken(adaln_backward(prepared(grads[1], kept[0]), prepared(grads[0], kept[0]), kept[0], kept[1], kept[2], kept[3],
+                                    kept[0].size(-1), false), "adaln_backward");
+        return {d[0], d[1], d[2], {}};
+    }
+};
+
+struct GatedResidualSite : Function<GatedResidualSite> {
+    static Tensors forward(AutogradContext *ctx, const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
+                           const torch::Tensor &scale, const torch::Tensor &shift, double epsilon) {
+        Tensors done = gated_run(h, attn, gate, scale, shift, epsilon);
+        ctx->set_materialize_grads(false);  // an unused h2 costs no zero tensor and no read
+        ctx->save_for_backward({done[0], attn, gate, scale, done[2], done[3]});
+        return {done[0], done[1]};
+    }
+    static Tensors backward(AutogradContext *ctx, Tensors grads) {
+        const Tensors kept = ctx->get_saved_variables();
+        const torch::Tensor dout = grads[1].defined() ? prepared(grads[1], kept[0]) : at::zeros_like(kept[0]);
+        Tensors d = taken(gated_backward(dout, prepared(grads[0], kept[0]), kept[0], kept[1], kept[2], kept[3], kept[4], kept[5],
+                                    kept[0].size(-1)), "gated_backward");
+        return {d[0], d[1], d[2], d[3], d[4], {}};
+    }
+};
+
+static c10::optional<torch::Tensor> adaln_site(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift,
+                                               int64_t cols, double epsilon, bool seq_first) {
+    if (!ordinary_call({&x, &scale, &shift}) || !adaln_ready(x, scale, shift, cols, seq_first)) return c10::nullopt;
+    return AdalnSite::apply(x, scale, shift, cols, epsilon, seq_first);
+}
+
+using Pair = std::tuple<torch::Tensor, torch::Tensor>;
+
+static c10::optional<Pair> adaln_residual_site(const torch::Tensor &x, const torch::Tensor &scale, const torch::Tensor &shift,
+                                               double epsilon) {
+    if (!ordinary_call({&x, &scale, &shift}) || x.dim() < 1 || !adaln_ready(x, scale, shift, x.size(-1), false))
+        return c10::nullopt;
+    Tensors outs = AdalnResidualSite::apply(x, scale, shift, epsilon);
+    return Pair{outs[0], outs[1]};
+}
+
+static c10::optional<Pair> gated_residual_site(const torch::Tensor &h, const torch::Tensor &attn, const torch::Tensor &gate,
+                                               const torch::Tensor &scale, const torch::Tensor &shift, double epsilon) {
+    if (!ordinary_call({&h, &attn, &gate, &scale, &shift}) || !gated_ready(h, attn, gate, scale, shift)) return c10::nullopt;
+    Tensors outs = GatedResidualSite::apply(h, attn, gate, scale, shift, epsilon);
+    return Pair{outs[0], outs[1]};
+}
+
 PYBIND11_MODULE(fused_adaln, m) {
+    m.def("adaln_site", &adaln_site, "AdaLNModelFunction as a native autograd node; None unless every operand is ready");
+    m.def("adaln_residual_site", &adaln_residual_site, "AdaLNResidualFunction as a native autograd node; or None");
+    m.def("gated_residual_site", &gated_residual_site, "GatedResidualAdaLNFunction as a native autograd node; or None");
     m.def("adaln_forward", &adaln_forward, "AdaLN forward: out, mean, inv_variance; None unless every operand is ready");
     m.def("adaln_backward", &adaln_backward, "AdaLN backward: dinp, dscale, dshift; None unless every operand is ready");
     m.def("gated_forward", &gated_forward, "gated residual update + AdaLN: h2, out, mean, inv_variance; or None");

@@ -357,28 +357,40 @@ static c10::optional<Tensors> rms_backward(const torch::Tensor &dout, const torc
     return Tensors{dinp, dweight};
 }
 
-// query, key, value: value is the transposed view of its slice of mixed
-static c10::optional<Tensors> qkv_forward(const torch::Tensor &mixed, const torch::Tensor &weight_q,
-                                          const torch::Tensor &weight_k, double epsilon,
-                                          const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
-    if (mixed.dim() != 4 || mixed.size(3) % 3 != 0) return c10::nullopt;
+static bool qkv_ready(const torch::Tensor &mixed, const torch::Tensor &weight_q, const torch::Tensor &weight_k,
+                      const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    if (mixed.dim() != 4 || mixed.size(3) % 3 != 0) return false;
     const int64_t cols = mixed.size(3) / 3;
-    if (!ready_rows(mixed, cols) || !tt_qkv_rmsnorm_supported(cols, dtype_code(mixed, "mixed_qkv"))) return c10::nullopt;
-    if (!cos.has_value() && mixed.numel() / mixed.size(3) > INT32_MAX) return c10::nullopt;  // beyond the joint kernels' units
+    if (!ready_rows(mixed, cols) || !tt_qkv_rmsnorm_supported(cols, dtype_code(mixed, "mixed_qkv"))) return false;
+    if (!cos.has_value() && mixed.numel() / mixed.size(3) > INT32_MAX) return false;  // beyond the joint kernels' units
     for (auto *w : {&weight_q, &weight_k})
-        if (!ready(*w, mixed) || w->numel() != cols) return c10::nullopt;
-    if (cos.has_value() != sin.has_value()) return c10::nullopt;
+        if (!ready(*w, mixed) || w->numel() != cols) return false;
+    if (cos.has_value() != sin.has_value()) return false;
     if (cos.has_value()) {
         for (auto *t : {&*cos, &*sin})
             if (t->scalar_type() != at::kFloat || !ready(*t, *t) || t->device() != mixed.device() || t->dim() != 2 ||
                 t->size(1) != cols || cols != 128 || t->size(0) > mixed.size(1))
-                return c10::nullopt;
-        if (cos->sizes() != sin->sizes()) return c10::nullopt;
+                return false;
+        if (cos->sizes() != sin->sizes()) return false;
     }
+    return true;
+}
+
+// query, key, value of ready operands: value is the transposed view of its slice of mixed
+static Tensors qkv_run(const torch::Tensor &mixed, const torch::Tensor &weight_q, const torch::Tensor &weight_k, double epsilon,
+                       const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    const int64_t cols = mixed.size(3) / 3;
     const std::vector<int64_t> shape{mixed.size(0), mixed.size(2), mixed.size(1), cols};
     torch::Tensor query = at::empty(shape, mixed.options()), key = at::empty(shape, mixed.options());
     torch_launch_qkv_rms_forward(query, key, mixed, weight_q, weight_k, epsilon, cos, sin);
-    return Tensors{query, key, mixed.slice(3, 2 * cols, 3 * cols).transpose(1, 2)};
+    return {query, key, mixed.slice(3, 2 * cols, 3 * cols).transpose(1, 2)};
+}
+
+static c10::optional<Tensors> qkv_forward(const torch::Tensor &mixed, const torch::Tensor &weight_q,
+                                          const torch::Tensor &weight_k, double epsilon,
+                                          const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    if (!qkv_ready(mixed, weight_q, weight_k, cos, sin)) return c10::nullopt;
+    return qkv_run(mixed, weight_q, weight_k, epsilon, cos, sin);
 }
 
 // dmixed, dweight_q, dweight_k; a gradient may be None
@@ -393,7 +405,92 @@ static c10::optional<Tensors> qkv_backward(const c10::optional<torch::Tensor> &d
     return Tensors{dmixed, dwq, dwk};
 }
 
+// ---- call sites (see torch_glue.h): RMSNormModelFunction and QKVSplitNormFunction ----
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+
+// A view whose rows the strided kernels read in place: at most 4-D, last dimension contiguous, every other stride a
+// non-negative multiple of 16 bytes.
+static bool ready_view(const torch::Tensor &x, int64_t cols) {
+    const auto st = x.scalar_type();
+    if (!x.is_cuda() || (st != at::kBFloat16 && st != at::kHalf && st != at::kFloat)) return false;
+    if (x.dim() < 2 || x.dim() > 4 || x.size(-1) != cols || x.stride(-1) != 1 || x.is_contiguous()) return false;
+    const int64_t vec = 16 / x.element_size();
+    for (int64_t d = 0; d + 1 < x.dim(); ++d)
+        if (x.stride(d) < 0 || x.stride(d) % vec != 0) return false;
+    return (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 && tt_norm_supported(cols, dtype_code(x, "input"));
+}
+
+static bool ready_parameter(const torch::Tensor &w, const torch::Tensor &x, int64_t cols) {
+    return ready(w, w) && w.numel() == cols && w.scalar_type() == x.scalar_type() && w.device() == x.device();
+}
+
+struct RmsSite : Function<RmsSite> {
+    static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &x, const torch::Tensor &weight, int64_t cols,
+                                 double epsilon, bool strided) {
+        const int64_t rows = x.numel() / cols;
+        torch::Tensor out = at::empty(x.sizes(), x.options()), inv_variance = row_statistics(x, rows);
+        if (strided)
+            torch_launch_rms_forward_strided(out, x, weight, epsilon, inv_variance);
+        else
+            torch_launch_rms_forward(out, x, weight, rows, cols, epsilon, inv_variance);
+        ctx->save_for_backward({x, weight, inv_variance});
+        ctx->saved_data["cols"] = cols;
+        ctx->saved_data["strided"] = strided;
+        return out;
+    }
+    static Tensors backward(AutogradContext *ctx, Tensors grads) {
+        const Tensors kept = ctx->get_saved_variables();
+        Tensors d = taken(rms_backward(prepared(grads[0], kept[1]), kept[0], kept[1], kept[2], ctx->saved_data["cols"].toInt(),
+                                  ctx->saved_data["strided"].toBool()), "rms_backward");
+        return {d[0], d[1], {}, {}, {}};
+    }
+};
+
+struct QkvSite : Function<QkvSite> {
+    static Tensors forward(AutogradContext *ctx, const torch::Tensor &mixed, const torch::Tensor &weight_q,
+                           const torch::Tensor &weight_k, double epsilon, const c10::optional<torch::Tensor> &cos,
+                           const c10::optional<torch::Tensor> &sin) {
+        Tensors outs = qkv_run(mixed, weight_q, weight_k, epsilon, cos, sin);
+        ctx->set_materialize_grads(false);
+        Tensors keep{mixed, weight_q, weight_k};
+        if (cos.has_value()) keep.insert(keep.end(), {*cos, *sin});
+        ctx->save_for_backward(std::move(keep));
+        ctx->saved_data["epsilon"] = epsilon;
+        return outs;
+    }
+    static Tensors backward(AutogradContext *ctx, Tensors grads) {
+        const Tensors kept = ctx->get_saved_variables();
+        for (auto &g : grads) g = prepared(g, kept[0]);
+        c10::optional<torch::Tensor> cos, sin;
+        if (kept.size() > 3) cos = kept[3], sin = kept[4];
+        Tensors d = taken(qkv_backward(grads[0], grads[1], grads[2], kept[0], kept[1], kept[2], ctx->saved_data["epsilon"].toDouble(),
+                                  cos, sin), "qkv_backward");
+        return {d[0], d[1], d[2], {}, {}, {}};
+    }
+};
+
+static c10::optional<torch::Tensor> rms_site(const torch::Tensor &x, const torch::Tensor &weight, int64_t cols, double epsilon) {
+    if (!ordinary_call({&x, &weight}) || !ready_parameter(weight, x, cols)) return c10::nullopt;
+    const bool strided = ready_view(x, cols);
+    if (!strided && !ready_rows(x, cols)) return c10::nullopt;
+    return RmsSite::apply(x, weight, cols, epsilon, strided);
+}
+
+static c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> qkv_site(
+    const torch::Tensor &mixed, const torch::Tensor &weight_q, const torch::Tensor &weight_k, double epsilon,
+    const c10::optional<torch::Tensor> &cos, const c10::optional<torch::Tensor> &sin) {
+    if (!ordinary_call({&mixed, &weight_q, &weight_k}) || (cos.has_value() && sin.has_value() && !ordinary_call({&*cos, &*sin})) ||
+        !qkv_ready(mixed, weight_q, weight_k, cos, sin))
+        return c10::nullopt;
+    Tensors outs = QkvSite::apply(mixed, weight_q, weight_k, epsilon, cos, sin);
+    return std::make_tuple(outs[0], outs[1], outs[2]);
+}
+
 PYBIND11_MODULE(fused_rmsnorm, m) {
+    m.def("rms_site", &rms_site, "RMSNormModelFunction as a native autograd node; None unless every operand is ready");
+    m.def("qkv_site", &qkv_site, "QKVSplitNormFunction as a native autograd node; None unless every operand is ready");
     m.def("rms_forward", &rms_forward, "RMSNorm forward: out, inv_variance; None unless every operand is ready");
     m.def("rms_backward", &rms_backward, "RMSNorm backward: dinp, dweight; None unless the gradient is ready");
     m.def("qkv_forward", &qkv_forward, "query, key, value of a fused projection; None unless every operand is ready");

@@ -5,6 +5,8 @@
 #pragma once
 
 #include <torch/extension.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include "teletron_norm.h"
@@ -57,6 +59,42 @@ inline bool ready_rows(const at::Tensor &x, int64_t cols) {
     const auto st = x.scalar_type();
     if (st != at::kBFloat16 && st != at::kHalf && st != at::kFloat) return false;
     return ready(x, x) && cols > 0 && x.numel() % cols == 0 && tt_norm_supported(cols, dtype_code(x, "input"));
+}
+
+// ---- call sites ------------------------------------------------------------------------------
+// The functions a block calls, as autograd nodes of the host runtime: graph recording, forward, and a backward that runs on
+// the engine's thread without the interpreter, its lock or a Python frame.  A call of forward and backward at 256 tokens is
+// host work only (its kernels take 15 us): 77 us a pass with the Python functions, 65 with the nodes, of which the engine's
+// hand-over to its thread and back takes 36 (QK-norm 106 -> 78, strided RMSNorm 90 -> 67, RMSNorm 6001 x 5120 78 -> 60).
+// The nodes take operands that are ready and ordinary tensors; under a transform, a dispatch mode, tracing or a tangent they
+// return None, and the Python functions handle or refuse the call as they always have.  What is kept goes through
+// SavedVariable, so saved-tensor hooks and version checks apply.
+inline bool ordinary_call(std::initializer_list<const at::Tensor *> operands) {
+    using c10::DispatchKey;
+    const c10::DispatchKeySet modes({DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::FuncTorchDynamicLayerBackMode,
+                                     DispatchKey::FuncTorchVmapMode, DispatchKey::VmapMode, DispatchKey::Functionalize,
+                                     DispatchKey::Tracer, DispatchKey::Python, DispatchKey::PreDispatch});
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+        c10::impl::tls_local_dispatch_key_set().included_.has_any(modes))
+        return false;
+    const c10::DispatchKeySet wrapped({DispatchKey::Python, DispatchKey::FuncTorchBatched, DispatchKey::FuncTorchGradWrapper,
+                                       DispatchKey::Batched, DispatchKey::Functionalize, DispatchKey::Negative,
+                                       DispatchKey::Conjugate, DispatchKey::ZeroTensor});
+    for (const at::Tensor *t : operands)
+        if (!t->defined() || t->key_set().has_any(wrapped) || t->_fw_grad(0).defined()) return false;
+    return true;
+}
+
+// A gradient as the kernels take it: the saved tensor's dtype, contiguous, 16-byte aligned.
+inline at::Tensor prepared(const at::Tensor &g, const at::Tensor &like) {
+    if (!g.defined() || ready(g, like)) return g;
+    at::Tensor t = g.to(like.scalar_type()).contiguous();
+    return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) ? t.clone() : t;
+}
+
+inline std::vector<at::Tensor> taken(c10::optional<std::vector<at::Tensor>> done, const char *what) {
+    TORCH_CHECK(done.has_value(), what, ": a gradient the kernels cannot take (another device, or no ordinary tensor)");
+    return std::move(*done);
 }
 
 inline at::Tensor row_statistics(const at::Tensor &x, int64_t rows) { return at::empty({rows}, x.options().dtype(at::kFloat)); }

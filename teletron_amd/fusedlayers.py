@@ -113,6 +113,13 @@ def _aligned_contiguous(t: torch.Tensor) -> torch.Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
+def _native(site, *args):
+    """The call as an autograd node of the host runtime (torch_glue.h: forward, graph and backward without Python frames),
+    or None where it does not apply as it is -- operands that need preparation, transforms, modes, a compiler tracing
+    this frame -- and the autograd functions below take it."""
+    return None if torch.compiler.is_compiling() else site(*args)
+
+
 class FP32LayerNorm(nn.LayerNorm):
     """LayerNorm evaluated in fp32 and cast back (dit_fusedlayers.py:48-57)."""
 
@@ -201,6 +208,14 @@ class AdaLNModelFunction(Function):
         return (grad_input, *_like_modulation(ctx, grad_scale, grad_shift), None, None) + (None,) * ctx.n_extra
 
 
+def _adaln(x, scale, shift, eps, cols, *seq_first):
+    if fused_adaln is not None:
+        done = _native(fused_adaln.adaln_site, x, scale, shift, cols, float(eps), bool(seq_first))
+        if done is not None:
+            return done
+    return AdaLNModelFunction.apply(x, scale, shift, eps, cols, *seq_first)
+
+
 class AdaLNResidualFunction(Function):
     """(x_same, out) = apply(x, scale, shift, epsilon): out is AdaLNModelFunction's result and x_same is x
     itself, handed back as an output for the caller to continue the residual stream with
@@ -263,6 +278,10 @@ class AdaLNResidualFunction(Function):
 def modulated_layer_norm_keeping_stream(x, scale, shift, eps: float = 1e-6):
     """Returns (x, LayerNorm(x) * (1 + scale[:, None]) + shift[:, None]); use the returned x for the residual
     connection so that its gradient is added inside the norm's backward kernel."""
+    if fused_adaln is not None:
+        done = _native(fused_adaln.adaln_residual_site, x, scale, shift, float(eps))
+        if done is not None:
+            return done
     return AdaLNResidualFunction.apply(x, scale, shift, eps)
 
 
@@ -279,7 +298,7 @@ class AdaLNCustom(nn.Module):
         for name, t in (("input x", x), ("scale", scale), ("shift", shift)):
             if t.shape[-1] != cols:
                 raise ValueError(f"Last dim of {name} must be hidden_size {cols}, got {t.shape[-1]}")
-        return AdaLNModelFunction.apply(x, scale, shift, self.eps, cols)
+        return _adaln(x, scale, shift, self.eps, cols)
 
 
 def modulated_layer_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor, eps: float = 1e-6,
@@ -290,9 +309,7 @@ def modulated_layer_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tens
     un-fused after attention (`norm2` + modulate, dit_layerspec.py:158-167) and
     in the output head (AdaLNContinuous, dit_layerspec.py:55-78).  seq_first: x is [S, B, C]
     and the result is LayerNorm(x) * (1 + scale) + shift broadcast over S, in place."""
-    if seq_first:
-        return AdaLNModelFunction.apply(x, scale, shift, eps, x.shape[-1], True)
-    return AdaLNModelFunction.apply(x, scale, shift, eps, x.shape[-1])
+    return _adaln(x, scale, shift, eps, x.shape[-1], *((True,) if seq_first else ()))
 
 
 class GatedResidualAdaLNFunction(Function):
@@ -368,6 +385,10 @@ class GatedResidualAdaLNFunction(Function):
 
 def gated_residual_layer_norm(h, attn, gate, scale, shift, eps: float = 1e-6):
     """Returns (h + attn * gate[:, None], modulated LayerNorm of that sum) from one fused pass."""
+    if fused_adaln is not None:
+        done = _native(fused_adaln.gated_residual_site, h, attn, gate, scale, shift, float(eps))
+        if done is not None:
+            return done
     return GatedResidualAdaLNFunction.apply(h, attn, gate, scale, shift, eps)
 
 
@@ -579,6 +600,10 @@ class RMSNorm(nn.Module):
         if fused_kernels_requested() and cols_supported(self.hidden_size, x.dtype):
             if not (eager_fallback_enabled() and (fused_rmsnorm is None or not x.is_cuda
                                                   or self.weight.dtype != x.dtype)):
+                if fused_rmsnorm is not None:
+                    done = _native(fused_rmsnorm.rms_site, x, self.weight, self.hidden_size, float(self.eps))
+                    if done is not None:
+                        return done
                 return RMSNormModelFunction.apply(x, self.weight, self.eps, self.hidden_size)
         return self._norm(x.float()).type_as(x) * self.weight
 
@@ -717,10 +742,14 @@ def split_qkv_and_norm(mixed_qkv: torch.Tensor, q_norm: "RMSNorm", k_norm: "RMSN
     D = mixed_qkv.shape[-1] // 3
     fusable = (fused_kernels_requested() and mixed_qkv.dtype in _ELEM_BYTES and cols_supported(D, mixed_qkv.dtype)
                and q_norm.eps == k_norm.eps)
-    if fusable and rotary is None:
-        return QKVSplitNormFunction.apply(mixed_qkv, q_norm.weight, k_norm.weight, q_norm.eps)
-    if fusable and D == 128:
-        return QKVSplitNormFunction.apply(mixed_qkv, q_norm.weight, k_norm.weight, q_norm.eps, *rotary)
+    if fusable and (rotary is None or D == 128):
+        tables = () if rotary is None else tuple(rotary)
+        if fused_rmsnorm is not None and len(tables) in (0, 2):
+            done = _native(fused_rmsnorm.qkv_site, mixed_qkv, q_norm.weight, k_norm.weight, float(q_norm.eps),
+                           *(tables or (None, None)))
+            if done is not None:
+                return done
+        return QKVSplitNormFunction.apply(mixed_qkv, q_norm.weight, k_norm.weight, q_norm.eps, *tables)
     if fusable:   # the strided-norm fusion is kept; only the rotation runs as separate ops
         query, key, value = QKVSplitNormFunction.apply(mixed_qkv, q_norm.weight, k_norm.weight, q_norm.eps)
     else:
