@@ -525,9 +525,9 @@ __device__ __forceinline__ void wave_clock_mark(int, int) {}
 // loads of a row, `process(buf, mid)` consumes them and calls `mid()` once
 // between its two register passes.  grp advances by `stride` and is
 // wave-uniform, so every branch here is too.
-// `prepare()` runs once, behind the requests of the first row: what a kernel forms from its parameters (which it has
-// requested before) then costs that row no time of its own.  A wavefront without rows never calls it.
-//   NBUF = 1 : one row at a time, the next one requested when the current one is done.
+// `prepare()` runs once, with two buffers behind the requests of the first row: what a kernel forms from its parameters
+// (which it has requested before) then costs that row no time of its own.  A wavefront without rows never calls it.
+//   NBUF = 1 : plain loop (load, process, store; nothing else in flight).
 //   NBUF = 2, MID = false : the next row is requested before the current one is processed.
 //   NBUF = 2, MID = true  : the next row is requested half-way through the current one.
 template <int NBUF, bool MID, typename RowRegs, typename Fetch, typename Process, typename Prepare>
@@ -537,14 +537,11 @@ __device__ __forceinline__ void row_pipeline(int64_t grp, int64_t groups, int64_
     auto nothing = [] {};
     if (grp >= groups) return;
     if constexpr (NBUF == 1) {
-        RowRegs a;
-        fetch(a, grp);
         prepare();
-        for (;;) {
-            process(a, nothing);
-            grp += stride;
-            if (grp >= groups) return;
+        for (; grp < groups; grp += stride) {
+            RowRegs a;
             fetch(a, grp);
+            process(a, nothing);
         }
     } else {
         RowRegs buf0, buf1;
