@@ -64,6 +64,13 @@ constexpr int64_t kInterleave = 4096, kTileTokens = 2048;
 #ifndef TTN_QKV_BWD_BLOCKS_PER_CU
 #define TTN_QKV_BWD_BLOCKS_PER_CU 2
 #endif
+// From this many steps per wavefront on, a step's rows are requested only when the stores of the step before have left the
+// wavefront: its reads and writes then take turns at the memory, as in the dense backward kernels (24 heads, 29700 tokens
+// 265 -> 251 us, 50000 451 -> 416, with tables 266 -> 259; 48828 x 16 x 64 151 -> 142; 39062 x 16 x 80 185 -> 182).  Shorter walks
+// are latency and lose the overlap (5000 tokens 49.5 / 49.9, 3000 32.6 / 33.4; 8000 73.7 / 73.3).
+#ifndef TTN_QKV_BWD_DRAIN_FROM
+#define TTN_QKV_BWD_DRAIN_FROM 24
+#endif
 // Consecutive steps of a wavefront that are neighbouring heads: with tables the rows it has fetched then serve more than
 // one head (runs of one 271, two 260, three 261, six 267 us); without tables runs only spread the writes (two: 261).
 #ifndef TTN_QKV_BWD_RUN
@@ -170,7 +177,7 @@ __global__ __launch_bounds__(kRowThreads) void qkv_fwd_kernel(T *__restrict__ q,
 }
 
 // gq / gk / gv may be null (that output was not used): its slice of d mixed is zero, as is its dweight.
-template <typename T, int LANES, bool FULL, typename Rope>
+template <typename T, int LANES, bool FULL, typename Rope, bool DRAIN>
 __global__ __launch_bounds__(kRowThreads) void qkv_bwd_kernel(
     T *__restrict__ dmixed, float *__restrict__ partial, const T *__restrict__ gq, const T *__restrict__ gk,
     const T *__restrict__ gv, const T *__restrict__ mixed, const T *__restrict__ wq, const T *__restrict__ wk,
@@ -216,6 +223,7 @@ __global__ __launch_bounds__(kRowThreads) void qkv_bwd_kernel(
         const int64_t at = ((b * S + s0) * H + h) * 3 * C;
         const int64_t dense = ((b * H + h) * S + s0) * C;
         u32x4 g[3], x[2];
+        if constexpr (DRAIN) wait_memory_ops<0>();
         {
             const RowReader<kLoadNt> rgq(gq + dense, dense_lane), rgk(gk + dense, dense_lane), rgv(gv + dense, dense_lane);
             const RowReader<kLoadNt> rxq(mixed + at, mixed_lane), rxk(mixed + at + C, mixed_lane);
@@ -350,7 +358,9 @@ static void launch_qkv_bwd(const QkvSizes &z, int64_t blocks, void *dmixed, void
                            const void *gv, const void *mixed, const void *wq, const void *wk, const Rope &rope, float eps,
                            hipStream_t stream) {
     RowKernelProfile prof(stream);
-    qkv_bwd_kernel<T, LANES, FULL, Rope><<<dim3((unsigned)blocks), dim3(kRowThreads), 0, stream>>>(
+    const bool drain = z.units() >= blocks * kRowWaves * TTN_QKV_BWD_DRAIN_FROM;
+    const auto kernel = drain ? qkv_bwd_kernel<T, LANES, FULL, Rope, true> : qkv_bwd_kernel<T, LANES, FULL, Rope, false>;
+    kernel<<<dim3((unsigned)blocks), dim3(kRowThreads), 0, stream>>>(
         (T *)dmixed, (float *)ws, (const T *)gq, (const T *)gk, (const T *)gv, (const T *)mixed, (const T *)wq,
         (const T *)wk, rope, z.S, (uint32_t)z.H, (uint32_t)z.token_groups(), (uint32_t)z.units(), (int)z.cols, eps);
 }
