@@ -577,8 +577,13 @@ __global__ __launch_bounds__(kRowThreads) void anywidth_adaln_bwd_kernel(
         q.r = q.ok ? rstd[srow] : 0.0f;
         q.mu = q.ok ? mean[srow] : 0.0f;
     };
+    // As in adaln.hip, a row's first pass waits for the stores of the row before it, which pays where a third tensor is read
+    // (residual: 24414 x 2048 bf16 74.1 -> 71.5 us, 43402 x 1152 81.2 -> 78.6, 1953 x 2560 17.3 -> 15.9, 8 x 1025 x 1536 fp16
+    // 26.6 -> 26.0).  The plain form loses 1-2 % and the gated one, whose operands are then waited for too, up to 7 %.
+    constexpr bool kDrain = RES && LANES == kWaveSize && CHUNKS >= 2;
     auto process = [&](Row &q, auto &&between_passes) {
         keep_packed(tr);
+        if constexpr (kDrain) wait_memory_ops<0>();
         const float r = q.r, mu = q.mu;
         const float nmr = -(mu * r);  // xhat = x*r + nmr
         // pass 1: gx = rnd(g*t) kept packed; s1 = sum_c gx; s2 = sum_c gx * xhat

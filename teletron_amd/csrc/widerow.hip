@@ -722,6 +722,9 @@ __global__ __launch_bounds__(kRowThreads) void wide_adaln_bwd_kernel(T *__restri
         }
     };
 
+    // Residual form: a row is requested only when the stores of the row before have left (two samples of 6178 x 3072 fp32
+    // 115.4 -> 110.2 us, 12207 x 4096 bf16 77.5 -> 75.1), unless the walk is short (2000 x 3072 fp32 26.8 / 27.6).
+    const bool drain = RES && rows_per_sample >= 8 * (int64_t)blocks_per_sample;
     const int64_t stride = blocks_per_sample;
     int64_t rs = slot;
     if (rs < rows_per_sample) {
@@ -739,6 +742,7 @@ __global__ __launch_bounds__(kRowThreads) void wide_adaln_bwd_kernel(T *__restri
 #else
         for (; rs < rows_per_sample; rs += stride) {
             Row b0;
+            if (drain) wait_memory_ops<0>();
             fetch(b0, rs);
             process(b0, [] {});
         }
