@@ -1,0 +1,60 @@
+"""Persistent backward grids walk a row at a time; from some length of the walk on a row's requests wait for the stores of the
+row before it.  Rows do not depend on each other, so a long call must equal its halves, each of them below that length."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-6
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.fixture(scope="module")
+def capi(gpu_device):
+    from teletron_amd import capi as c
+    c.lib()
+    return c
+
+
+def _sums_agree(whole, parts, terms, dtype):
+    """Column sums of `terms` positive-variance terms of size about one: fp32 partial sums differ by their order (at most
+    terms * 2^-24 of the sum of magnitudes, which is below 2 * terms), and each result is rounded once to the element type."""
+    total = sum(p.float() for p in parts)
+    slack = 2.0 * terms * terms ** 0.5 * 2.0 ** -24
+    ulp = {BF: 2.0 ** -8, HF: 2.0 ** -11, F32: 2.0 ** -24}[dtype]
+    size = torch.stack([whole.float().abs(), *(p.float().abs() for p in parts)]).sum(0)
+    return bool(((whole.float() - total).abs() <= slack + ulp * size).all())
+
+
+# 24 steps of 2048 wavefronts begin at 49 152 groups of heads and tokens
+@pytest.mark.parametrize("B,S,H,D,rotated,dtype", [
+    (1, 8240, 24, 128, 0, BF), (1, 8241, 24, 128, 8200, BF), (2, 6001, 9, 80, 0, HF), (1, 6003, 16, 96, 0, F32), (1, 12000, 34, 64, 0, BF),
+    (1, 4103, 24, 128, 4103, F32)])
+def test_joint_backward_equals_its_halves(capi, gpu_device, B, S, H, D, rotated, dtype):
+    gen = torch.Generator(device=gpu_device).manual_seed(S + D)
+    rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=gen).to(dtype)
+    mixed, w, grads = rnd(B, S, H, 3 * D), [rnd(D) for _ in range(2)], [rnd(B, H, S, D) for _ in range(3)]
+    cos, sin = (torch.randn(rotated, D, device=gpu_device, generator=gen) for _ in range(2)) if rotated else (None, None)
+    whole = capi.qkv_rmsnorm_backward(*grads, mixed, *w, EPS, cos, sin)
+    half = S // 2 // 8 * 8
+    parts = []
+    for cut in (slice(0, half), slice(half, S)):
+        t = (None, None) if not rotated else tuple(a[cut].contiguous() for a in (cos, sin))
+        parts.append(capi.qkv_rmsnorm_backward(*(g[:, :, cut].contiguous() for g in grads), mixed[:, cut].contiguous(), *w, EPS, *t))
+    assert torch.equal(whole[0], torch.cat([p[0] for p in parts], 1))
+    for i in (1, 2):
+        assert _sums_agree(whole[i], [p[i] for p in parts], B * S * H, dtype)
+    again = capi.qkv_rmsnorm_backward(*grads, mixed, *w, EPS, cos, sin)
+    assert all(torch.equal(a, b) for a, b in zip(whole, again))
+
+
+@pytest.mark.parametrize("batch,rows,cols,dtype", [
+    (1, 4099, 4096, BF), (2, 2051, 3072, F32), (1, 4095, 5128, HF), (1, 1031, 1152, BF), (3, 700, 2048, BF), (1, 2049, 1536, F32),
+    (1, 2050, 3072, BF)])
+def test_residual_backward_equals_the_plain_one_plus_the_other_gradient(capi, gpu_device, batch, rows, cols, dtype):
+    gen = torch.Generator(device=gpu_device).manual_seed(rows + cols)
+    rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=gen).to(dtype)
+    x, g, other, scale, shift = rnd(batch, rows, cols), rnd(batch, rows, cols), rnd(batch, rows, cols), rnd(batch, cols), rnd(batch, cols)
+    _, mean, rstd = capi.adaln_forward(x, scale, shift, EPS)
+    dx, dscale, dshift = capi.adaln_backward(g, x, scale, mean, rstd)
+    got = capi.adaln_backward_residual(g, other, x, scale, mean, rstd)
+    assert torch.equal(got[0], dx + other) and torch.equal(got[1], dscale) and torch.equal(got[2], dshift)
