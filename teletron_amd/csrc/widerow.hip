@@ -61,6 +61,8 @@
 // requested when the one before it is done (the two workgroups of a compute unit overlap each other instead:
 // 347 / 372 us against 380 / 385 us for RMSNorm / AdaLN backward at 89 100 x 4096 two-byte columns, and one
 // workgroup per compute unit without the request ahead is far slower, 504 / 560 us).
+// The backward kernels form what they need of the parameters behind the first row's requests (RMSNorm 500 x 4096 bf16 13.2 ->
+// 12.6 us, 2000 x 4096 18.4 -> 17.8, 6001 x 5120 41.3 -> 40.7; AdaLN 500 x 4096 18.3 -> 17.9; long walks the same).
 #ifndef TTN_WIDE_BWD_PREFETCH
 #define TTN_WIDE_BWD_PREFETCH 0
 #endif
@@ -294,9 +296,14 @@ __global__ __launch_bounds__(kRowThreads) void wide_rmsnorm_bwd_kernel(T *__rest
     const uint32_t one_hi = opaque_const(kOneHi<std::conditional_t<kHasDot2<T>, T, bf16_t>>);
 
     RowParam<T, CH> wp;
+    u32x4 wr[CH];
 #pragma unroll
     for (int k = 0; k < CH; ++k)
-        wp.set(k, m.in[k] ? load16(reinterpret_cast<const u32x4 *>(w + slice) + k * kWaveSize + lane) : u32x4{0, 0, 0, 0});
+        wr[k] = m.in[k] ? load16(reinterpret_cast<const u32x4 *>(w + slice) + k * kWaveSize + lane) : u32x4{0, 0, 0, 0};
+    auto prepare = [&] {
+#pragma unroll
+        for (int k = 0; k < CH; ++k) wp.set(k, wr[k]);
+    };
     float acc[1][CH][VEC];
 #pragma unroll
     for (int k = 0; k < CH; ++k)
@@ -361,6 +368,7 @@ __global__ __launch_bounds__(kRowThreads) void wide_rmsnorm_bwd_kernel(T *__rest
 #if TTN_WIDE_BWD_PREFETCH
         Row b0, b1;
         fetch(b0, row);
+        prepare();
         for (;;) {
             process(b0, row, [&] { fetch(b1, row + stride); });
             row += stride;
@@ -370,7 +378,13 @@ __global__ __launch_bounds__(kRowThreads) void wide_rmsnorm_bwd_kernel(T *__rest
             if (row >= rows) break;
         }
 #else
-        for (; row < rows; row += stride) {
+        {
+            Row b0;
+            fetch(b0, row);
+            prepare();
+            process(b0, row, [] {});
+        }
+        for (row += stride; row < rows; row += stride) {
             Row b0;
             fetch(b0, row);
             process(b0, row, [] {});
@@ -598,15 +612,20 @@ __global__ __launch_bounds__(kRowThreads) void wide_adaln_bwd_kernel(T *__restri
     const uint32_t one_hi = opaque_const(kOneHi<std::conditional_t<kHasDot2<T>, T, bf16_t>>);
 
     RowParam<T, CH> tp;  // t = rnd(1 + scale[sample])
+    u32x4 sr[CH];
 #pragma unroll
-    for (int k = 0; k < CH; ++k) {
-        float v[VEC];
-        E::unpack(m.in[k] ? load16(reinterpret_cast<const u32x4 *>(scale + smp * C + slice) + k * kWaveSize + lane)
-                          : u32x4{0, 0, 0, 0}, v);
+    for (int k = 0; k < CH; ++k)
+        sr[k] = m.in[k] ? load16(reinterpret_cast<const u32x4 *>(scale + smp * C + slice) + k * kWaveSize + lane) : u32x4{0, 0, 0, 0};
+    auto prepare = [&] {
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
-        tp.set(k, E::pack(v));
-    }
+        for (int k = 0; k < CH; ++k) {
+            float v[VEC];
+            E::unpack(sr[k], v);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) v[j] = 1.0f + v[j];
+            tp.set(k, E::pack(v));
+        }
+    };
     [[maybe_unused]] u32x4 qr[GATED ? CH : 1];  // gate[sample], packed
     if constexpr (GATED) {
 #pragma unroll
@@ -731,6 +750,7 @@ __global__ __launch_bounds__(kRowThreads) void wide_adaln_bwd_kernel(T *__restri
 #if TTN_WIDE_BWD_PREFETCH
         Row b0, b1;
         fetch(b0, rs);
+        prepare();
         for (;;) {
             process(b0, [&] { fetch(b1, rs + stride); });
             rs += stride;
@@ -740,7 +760,13 @@ __global__ __launch_bounds__(kRowThreads) void wide_adaln_bwd_kernel(T *__restri
             if (rs >= rows_per_sample) break;
         }
 #else
-        for (; rs < rows_per_sample; rs += stride) {
+        {
+            Row b0;
+            fetch(b0, rs);
+            prepare();
+            process(b0, [] {});
+        }
+        for (rs += stride; rs < rows_per_sample; rs += stride) {
             Row b0;
             if (drain) wait_memory_ops<0>();
             fetch(b0, rs);
