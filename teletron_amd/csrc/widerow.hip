@@ -10,7 +10,7 @@
 // addition at all).
 //
 // Grids (measured at 4096, 5120 and 8192 two-byte columns, 730 MB per tensor): RMSNorm forward one-shot (one
-// row per workgroup); AdaLN forward in short-lived workgroups of four rows each, which amortise the set-up of
+// row per workgroup); AdaLN forward in short-lived workgroups of a few rows each, which amortise the set-up of
 // the modulation row (kept as fp32 values) and still retire and get replaced as the grid drains; both request
 // the next row before the current row's output pass.  Backward persistent, two workgroups per compute unit that
 // overlap each other (no request ahead inside a wavefront), write-through stores.  The gated residual and residual forms
@@ -34,12 +34,12 @@
 #define TTN_WIDE_BWD_BLOCKS_PER_CU 2
 #endif
 // Forward grids: rows per workgroup (1 = one-shot grid, N = short-lived workgroups of N rows each, 0 = persistent
-// grid of TTN_WIDE_FWD_BLOCKS_PER_CU resident workgroups per compute unit).
+// grid of TTN_WIDE_FWD_BLOCKS_PER_CU resident workgroups per compute unit).  AdaLN's number follows the call (wide_adaln_fwd_rows).
 #ifndef TTN_WIDE_RMS_FWD_ROWS_PER_BLOCK
 #define TTN_WIDE_RMS_FWD_ROWS_PER_BLOCK 1
 #endif
 #ifndef TTN_WIDE_ADALN_FWD_ROWS_PER_BLOCK
-#define TTN_WIDE_ADALN_FWD_ROWS_PER_BLOCK 4
+#define TTN_WIDE_ADALN_FWD_ROWS_PER_BLOCK wide_adaln_fwd_rows(batch * rows_per_sample, cus, !GATED && dtype != TT_NORM_F32)
 #endif
 // Stores: 1 = write-through at device scope (RowWriter<1>), 0 = plain streaming store.
 #ifndef TTN_WIDE_FWD_STORE
@@ -886,6 +886,16 @@ int widerow_rmsnorm_backward(void *dx, void *dw, const void *g, const void *x, c
     return launch_colreduce(dw, nullptr, nullptr, (const float *)ws, 1, p.blocks_per_sample, cols, cols, dtype, stream);
 }
 
+// AdaLN forward: rows per workgroup.  Setting up the modulation row costs about a row, so a long grid takes four rows of the
+// plain two-byte form at a time (3000 x 4096 bf16 12.5 us, 13.5 with two) and two of the forms that
+// move twice the bytes per column (gated 60 000 x 4096 bf16 345 us with four, 329 with two; 50 000 x 2048 fp32 142 / 139).
+// A grid that would leave compute units idle takes fewer: one row up to four workgroups per compute unit (100 x 4096 6.7 ->
+// 3.9 us, 1000 x 4096 7.8 -> 6.5, gated 700 x 4096 10.1 -> 7.9), two up to ten (1300 x 4096 9.1 -> 7.9, 2500 x 4096 12.0 -> 10.9).
+static int wide_adaln_fwd_rows(int64_t rows, int cus, bool plain_two_byte) {
+    if (rows <= 4 * (int64_t)cus) return 1;
+    return plain_two_byte && rows > 10 * (int64_t)cus ? 4 : 2;
+}
+
 struct WideExtra {  // operands of the gated / residual forms (null otherwise)
     void *h2_or_da;    // forward: h2 out; backward: da out
     const void *e;     // backward: the gradient arriving at h2 / at the input from its other use
@@ -900,6 +910,8 @@ static int wide_adaln_forward_t(void *out, float *mean, float *rstd, const void 
     if (rows_per_sample == 0) return TT_NORM_OK;
     RowPlan p;
     int st = TT_NORM_OK;
+    [[maybe_unused]] const int cus = current_device_cus(&st);
+    if (st != TT_NORM_OK) return st;
     const SampleLayout lay = seq_first ? SampleLayout{1, batch} : SampleLayout{rows_per_sample, 1};
     const int ch = wide_chunks(cols, dtype), ppw = wide_pieces_per_wave(cols, dtype);
     {

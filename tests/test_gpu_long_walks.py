@@ -58,3 +58,28 @@ def test_residual_backward_equals_the_plain_one_plus_the_other_gradient(capi, gp
     dx, dscale, dshift = capi.adaln_backward(g, x, scale, mean, rstd)
     got = capi.adaln_backward_residual(g, other, x, scale, mean, rstd)
     assert torch.equal(got[0], dx + other) and torch.equal(got[1], dscale) and torch.equal(got[2], dshift)
+
+
+# wide rows: one, two and four rows per workgroup of the forward, each side of the lines (four and ten workgroups of one row per
+# compute unit), rows that do not fill the last workgroup
+@pytest.mark.parametrize("batch,rows,cols,dtype", [
+    (1, 1, 4096, BF), (1, 1024, 4096, BF), (1, 1027, 4096, HF), (3, 853, 5128, BF), (1, 2563, 4096, BF), (2, 1283, 5120, BF),
+    (1, 1023, 2048, F32), (5, 207, 3072, F32), (1, 2575, 2048, F32)])
+def test_wide_forward_does_not_depend_on_its_grid(capi, gpu_device, batch, rows, cols, dtype):
+    gen = torch.Generator(device=gpu_device).manual_seed(rows + cols)
+    rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=gen).to(dtype)
+    x, attn, gate, scale, shift = rnd(batch, rows, cols), rnd(batch, rows, cols), rnd(batch, cols), rnd(batch, cols), rnd(batch, cols)
+
+    def one_sample(b, cut):
+        return (capi.adaln_forward(x[b:b + 1, cut].contiguous(), scale[b:b + 1].contiguous(), shift[b:b + 1].contiguous(), EPS),
+                capi.gated_residual_adaln_forward(x[b:b + 1, cut].contiguous(), attn[b:b + 1, cut].contiguous(), gate[b:b + 1].contiguous(),
+                                                  scale[b:b + 1].contiguous(), shift[b:b + 1].contiguous(), EPS))
+
+    plain, gated = capi.adaln_forward(x, scale, shift, EPS), capi.gated_residual_adaln_forward(x, attn, gate, scale, shift, EPS)
+    for b in range(batch):
+        for start in range(0, rows, 400):
+            cut = slice(start, min(start + 400, rows))
+            a, g = one_sample(b, cut)
+            for whole, part in zip((*plain, *gated), (*a, *g)):
+                assert torch.equal(whole.view(batch, rows, -1)[b, cut], part.view(cut.stop - cut.start, -1))
+    assert torch.isfinite(plain[0].float()).all()
