@@ -42,14 +42,15 @@
 // With its row requested before the parameters are staged, a two-byte workgroup streams best four to a compute unit
 // while the grid is short (16 KiB on top of its 24 KiB: 14 850 rows 34.0 us against 34.3 with six and 34.5 with three,
 // 4000 rows 10.0 / 10.1 / 11.9) and three once it refills every compute unit many times (24 KiB: 118 800 rows 240.5 us
-// against 244.6 with four and 250.7 with six; 80 000 rows 165 either way).  The gated form runs unthrottled, five by its
-// registers and LDS (118 800 rows 489 us, 493 with three; 4000 rows 20.9 / 22.2).  4-byte rows carry twice the bytes per
+// against 244.6 with four and 250.7 with six; 80 000 rows 165 either way).  The gated form runs unthrottled, by its registers and
+// LDS, on short grids (4000 rows 20.9 us, 22.2 with 12 KiB more; 60 000 rows 244.7 / 248.2).  On long ones it takes the
+// 12 KiB: between backward launches 118 800 rows take 482 us, 490 without (on its own 492 / 488).  4-byte rows carry twice the bytes per
 // wavefront: 40 KiB on top of the staged modulation rows leaves two workgroups per compute unit (59 400 rows 243 us, 260
 // with three); gated, 16 KiB leave three (8192 rows 70.2 us, 72.9 with two).
 #ifndef TTN_ADALN_FWD_DYN_LDS
 #define TTN_ADALN_FWD_DYN_LDS                                                                        \
     (C < 1024           ? 0                                                                          \
-     : GATED            ? (sizeof(T) == 4 ? 16384 : 0)                                               \
+     : GATED            ? (sizeof(T) == 4 ? 16384 : p.blocks < 64 * (int64_t)cus ? 0 : 12288)         \
      : sizeof(T) == 4   ? 40960                                                                      \
      : p.blocks < 64 * (int64_t)cus ? 16384                                                          \
                         : 24576)
