@@ -337,6 +337,17 @@ static c10::optional<Tensors> gated_backward(const torch::Tensor &dout, const c1
 using torch::autograd::AutogradContext;
 using torch::autograd::Function;
 
+// adaln_backward returns both modulation gradients in scale's shape; a shift that came in another shape of as many
+// elements gets its gradient in its own.
+static void keep_shift_shape(AutogradContext *ctx, const torch::Tensor &scale, const torch::Tensor &shift) {
+    if (shift.sizes() != scale.sizes()) ctx->saved_data["shift_shape"] = shift.sizes().vec();
+}
+
+static torch::Tensor in_shift_shape(AutogradContext *ctx, const torch::Tensor &dshift) {
+    const auto kept = ctx->saved_data.find("shift_shape");
+    return kept == ctx->saved_data.end() ? dshift : dshift.view(kept->second.toIntVector());
+}
+
 struct AdalnSite : Function<AdalnSite> {
     static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &x, const torch::Tensor &scale,
                                  const torch::Tensor &shift, int64_t cols, double epsilon, bool seq_first) {
@@ -344,13 +355,14 @@ struct AdalnSite : Function<AdalnSite> {
         ctx->save_for_backward({x, scale, done[1], done[2]});
         ctx->saved_data["cols"] = cols;
         ctx->saved_data["seq_first"] = seq_first;
+        keep_shift_shape(ctx, scale, shift);
         return done[0];
     }
     static Tensors backward(AutogradContext *ctx, Tensors grads) {
         const Tensors kept = ctx->get_saved_variables();
         Tensors d = taken(adaln_backward(prepared(grads[0], kept[0]), c10::nullopt, kept[0], kept[1], kept[2], kept[3],
                                     ctx->saved_data["cols"].toInt(), ctx->saved_data["seq_first"].toBool()), "adaln_backward");
-        return {d[0], d[1], d[2], {}, {}, {}};
+        return {d[0], d[1], in_shift_shape(ctx, d[2]), {}, {}, {}};
     }
 };
 
@@ -360,6 +372,7 @@ struct AdalnResidualSite : Function<AdalnResidualSite> {
         Tensors done = adaln_run(x, scale, shift, x.size(-1), epsilon, false);
         ctx->set_materialize_grads(false);
         ctx->save_for_backward({x, scale, done[1], done[2]});
+        keep_shift_shape(ctx, scale, shift);
         return {x, done[0]};
     }
     static Tensors backward(AutogradContext *ctx, Tensors grads) {
@@ -367,7 +380,7 @@ struct AdalnResidualSite : Function<AdalnResidualSite> {
         if (!grads[1].defined()) return {grads[0], {}, {}, {}};  // only the stream was used: the function was an identity
         Tensors d = taken(adaln_backward(prepared(grads[1], kept[0]), prepared(grads[0], kept[0]), kept[0], kept[1], kept[2], kept[3],
                                     kept[0].size(-1), false), "adaln_backward");
-        return {d[0], d[1], d[2], {}};
+        return {d[0], d[1], in_shift_shape(ctx, d[2]), {}};
     }
 };
 

@@ -130,11 +130,11 @@ class FP32LayerNorm(nn.LayerNorm):
 
 
 def _like_modulation(ctx, *grads):
-    """Gradients of modulation rows in the shape and dtype the caller passed; ctx.mod_shape is None where the rows
-    were used as they came."""
-    if ctx.mod_shape is None:
+    """Gradients of scale and shift in the shapes and dtypes the caller passed; ctx.mod_meta is None where the rows
+    were used as they came, both in one shape."""
+    if ctx.mod_meta is None:
         return grads
-    return tuple(g.reshape(ctx.mod_shape).to(ctx.mod_dtype) for g in grads)
+    return tuple(g.reshape(shape).to(dtype) for g, (shape, dtype) in zip(grads, ctx.mod_meta))
 
 
 class AdaLNModelFunction(Function):
@@ -157,7 +157,8 @@ class AdaLNModelFunction(Function):
         if done is not None:   # every operand was ready as it is; anything else is prepared, or refused, below
             out, mean, invvar = done
             ctx.save_for_backward(x, scale, mean, invvar)
-            ctx.rows, ctx.cols, ctx.seq_first, ctx.mod_shape, ctx.mod_dtype = invvar.shape[0], cols, seq_first, None, None
+            ctx.rows, ctx.cols, ctx.seq_first = invvar.shape[0], cols, seq_first
+            ctx.mod_meta = None if scale.shape == shift.shape else [(t.shape, t.dtype) for t in (scale, shift)]
             return out
         _require_gpu(x, "AdaLNModelFunction")
         x = _aligned_contiguous(x)
@@ -186,7 +187,7 @@ class AdaLNModelFunction(Function):
         launch(out, x, scale_c, shift_c, rows, cols, float(epsilon), mean, invvar)
         ctx.save_for_backward(x, scale_c, mean, invvar)
         ctx.rows, ctx.cols, ctx.seq_first = rows, cols, seq_first
-        ctx.mod_shape, ctx.mod_dtype = scale.shape, scale.dtype
+        ctx.mod_meta = [(t.shape, t.dtype) for t in (scale, shift)]
         return out
 
     @staticmethod
@@ -231,7 +232,8 @@ class AdaLNResidualFunction(Function):
         if done is not None:
             out, mean, invvar = done
             ctx.save_for_backward(x, scale, mean, invvar)
-            ctx.rows, ctx.cols, ctx.mod_shape, ctx.mod_dtype = invvar.shape[0], x.shape[-1], None, None
+            ctx.rows, ctx.cols = invvar.shape[0], x.shape[-1]
+            ctx.mod_meta = None if scale.shape == shift.shape else [(t.shape, t.dtype) for t in (scale, shift)]
             return x, out
         _require_gpu(x, "AdaLNResidualFunction")
         cols = x.shape[-1]
@@ -251,7 +253,7 @@ class AdaLNResidualFunction(Function):
         ext.torch_launch_adaln_forward_stats(out, x_c, scale_c, shift_c, rows, cols, float(epsilon), mean, invvar)
         ctx.save_for_backward(x_c, scale_c, mean, invvar)
         ctx.rows, ctx.cols = rows, cols
-        ctx.mod_shape, ctx.mod_dtype = scale.shape, scale.dtype
+        ctx.mod_meta = [(t.shape, t.dtype) for t in (scale, shift)]
         return x, out
 
     @staticmethod

@@ -171,6 +171,32 @@ def test_transforms_and_tangents_do_what_the_python_function_does(FL, gpu_device
         assert _same(a[1], b[1]) if a[0] == "ran" else a[1] == b[1], (a, b)
 
 
+@pytest.mark.parametrize("kind,scale,shift", [
+    (kind, *shapes) for kind in ("adaln", "stream") for shapes in (
+        ((2, 1, 3072), (2, 3072)), ((2, 3072), (2, 1, 3072)), ((3072,), (1, 3072)), ((1, 3072), (3072,)), ((1, 1, 3072), (3072,)))
+] + [("seq_first", (2, 1, 1536), (2, 1536)), ("seq_first", (2, 1536), (2, 1, 1536))])
+@pytest.mark.parametrize("how", ["ready", "gradient to prepare", "rows to prepare", "other dtypes"])
+def test_scale_and_shift_of_unlike_shapes(FL, gpu_device, kind, scale, shift, how):
+    """Each gets its gradient in its own shape and dtype, with the values that equal shapes get."""
+    args, grads, site, function = _case(FL, kind, torch.bfloat16, gpu_device)
+    if scale[0] != 2:   # one modulation row
+        args, grads = [a[:1].contiguous() for a in args], [g[:1].contiguous() for g in grads]
+    want = _both(function, args, grads)[1]
+    shaped = [args[0], args[1].reshape(scale), args[2].reshape(shift)]
+    if how == "gradient to prepare":
+        grads = [g.transpose(-1, -2).contiguous().transpose(-1, -2) for g in grads]
+    if how == "rows to prepare":
+        shaped[0] = torch.empty(args[0].numel() + 1, dtype=args[0].dtype, device=gpu_device)[1:].view(args[0].shape).copy_(args[0])
+    if how == "other dtypes":
+        shaped[1] = shaped[1].float()
+    for call in (site, function):
+        leaves = [t.detach().requires_grad_(True) for t in shaped]
+        outs = _tuple(call(*leaves))
+        got = [o.detach() for o in outs] + list(torch.autograd.grad(outs, leaves, grads))
+        assert [(g.shape, g.dtype) for g in got[-2:]] == [(t.shape, t.dtype) for t in shaped[1:]]
+        assert all(torch.equal(g.reshape(w.shape).to(w.dtype), w) for g, w in zip(got, want))
+
+
 def test_another_stream_and_several_threads(FL, gpu_device):
     args, grads, site, function = _case(FL, "gated", torch.bfloat16, gpu_device)
     want = _both(function, args, grads)[1]
