@@ -35,6 +35,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd import Function
+from torch.overrides import has_torch_function_variadic
 
 log = logging.getLogger(__name__)
 log.addHandler(logging.NullHandler())
@@ -53,6 +54,7 @@ TUNED_COLS = (128, 3072)  # the reference's two shapes (the tuned kernels)
 _ELEM_BYTES = {torch.bfloat16: 2, torch.float16: 2, torch.float32: 4}
 _MAX_PIECES = 1024  # 16-byte pieces per row the kernels are built for
 _MAX_JOINT_HEAD_BYTES = 1024  # a head's row the joint q / k / v kernels take: 64 16-byte pieces
+_PLAIN = frozenset((torch.Tensor, nn.Parameter, int, float, bool, type(None)))  # what a native node takes for itself
 _MAX_JOINT_ROWS = 2 ** 31 - 1  # rows of q (or k) whose groups their 32-bit unit numbers are sure to hold
 
 
@@ -115,9 +117,13 @@ def _aligned_contiguous(t: torch.Tensor) -> torch.Tensor:
 
 def _native(site, *args):
     """The call as an autograd node of the host runtime (torch_glue.h: forward, graph and backward without Python frames),
-    or None where it does not apply as it is -- operands that need preparation, transforms, modes, a compiler tracing
-    this frame -- and the autograd functions below take it."""
-    return None if torch.compiler.is_compiling() else site(*args)
+    or None where it does not apply as it is -- operands that need preparation, transforms, dispatch modes, a compiler
+    tracing this frame -- and the autograd functions below take it.  So they do with a tensor subclass: an input handed
+    back as an output keeps its class there, a node's view of it is a plain tensor.  A function mode alone changes
+    nothing (has_torch_function_variadic is true for it too, hence the second look)."""
+    if torch.compiler.is_compiling() or (has_torch_function_variadic(*args) and not _PLAIN.issuperset(map(type, args))):
+        return None
+    return site(*args)
 
 
 class FP32LayerNorm(nn.LayerNorm):

@@ -171,6 +171,26 @@ def test_transforms_and_tangents_do_what_the_python_function_does(FL, gpu_device
         assert _same(a[1], b[1]) if a[0] == "ran" else a[1] == b[1], (a, b)
 
 
+class _Tagged(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_subclasses_keep_what_the_python_function_gives_them(FL, gpu_device, kind):
+    """The stream handed back is the caller's class, not a plain view of it."""
+    args, grads, site, function = _case(FL, kind, torch.bfloat16, gpu_device)
+
+    def run(call):
+        leaves = _leaves(args)
+        leaves[0] = leaves[0].detach().as_subclass(_Tagged).requires_grad_(True)
+        outs = _tuple(call(*leaves))
+        return [type(o) for o in outs], [o.detach() for o in outs] + list(torch.autograd.grad(outs, leaves, grads))
+
+    (a, got), (b, want) = run(site), run(function)
+    assert a == b and _same(got, want)
+    assert kind != "stream" or a[0] is _Tagged
+
+
 @pytest.mark.parametrize("kind,scale,shift", [
     (kind, *shapes) for kind in ("adaln", "stream") for shapes in (
         ((2, 1, 3072), (2, 3072)), ((2, 3072), (2, 1, 3072)), ((3072,), (1, 3072)), ((1, 3072), (3072,)), ((1, 1, 3072), (3072,)))

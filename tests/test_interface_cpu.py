@@ -266,3 +266,28 @@ def test_eager_fallback_switch_restores_the_reference_gating(monkeypatch):
     monkeypatch.setenv("TELETRON_AMD_FALLBACK", "")
     with pytest.raises(ValueError, match="unsupported cols 66"):
         FL.FusedAdaLayerNormZero(66, fused_kernels=True, linear_parallel=False)
+
+
+def test_native_nodes_are_offered_plain_tensors_only(monkeypatch):
+    """Plain tensors and parameters, function mode or not; a subclass and a compiler's frame are left to the Python functions."""
+    from torch.overrides import TorchFunctionMode
+
+    from teletron_amd import fusedlayers as FL
+
+    class Tagged(torch.Tensor):
+        pass
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    site = lambda *args: len(args)
+    x, w = torch.zeros(2, 8), torch.nn.Parameter(torch.ones(8))
+    assert FL._native(site, x, w, 8, 1e-6, False, None) == 6
+    assert FL._native(site, x.as_subclass(Tagged), w, 8, 1e-6) is None
+    assert FL._native(site, x, w, w.detach().as_subclass(Tagged)) is None
+    with Mode():
+        assert FL._native(site, x, w, 8, 1e-6, False, None) == 6
+        assert FL._native(site, x.as_subclass(Tagged), w) is None
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert FL._native(site, x, w, 8, 1e-6) is None
