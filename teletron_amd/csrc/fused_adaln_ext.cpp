@@ -362,7 +362,7 @@ struct AdalnSite : Function<AdalnSite> {
         const Tensors kept = ctx->get_saved_variables();
         Tensors d = taken(adaln_backward(prepared(grads[0], kept[0]), c10::nullopt, kept[0], kept[1], kept[2], kept[3],
                                     ctx->saved_data["cols"].toInt(), ctx->saved_data["seq_first"].toBool()), "adaln_backward");
-        return {d[0], d[1], in_shift_shape(ctx, d[2]), {}, {}, {}};
+        return first_order({d[0], d[1], in_shift_shape(ctx, d[2]), {}, {}, {}}, kept, grads);
     }
 };
 
@@ -380,7 +380,7 @@ struct AdalnResidualSite : Function<AdalnResidualSite> {
         if (!grads[1].defined()) return {grads[0], {}, {}, {}};  // only the stream was used: the function was an identity
         Tensors d = taken(adaln_backward(prepared(grads[1], kept[0]), prepared(grads[0], kept[0]), kept[0], kept[1], kept[2], kept[3],
                                     kept[0].size(-1), false), "adaln_backward");
-        return {d[0], d[1], in_shift_shape(ctx, d[2]), {}};
+        return first_order({d[0], d[1], in_shift_shape(ctx, d[2]), {}}, kept, grads);
     }
 };
 
@@ -397,7 +397,7 @@ struct GatedResidualSite : Function<GatedResidualSite> {
         const torch::Tensor dout = grads[1].defined() ? prepared(grads[1], kept[0]) : at::zeros_like(kept[0]);
         Tensors d = taken(gated_backward(dout, prepared(grads[0], kept[0]), kept[0], kept[1], kept[2], kept[3], kept[4], kept[5],
                                     kept[0].size(-1)), "gated_backward");
-        return {d[0], d[1], d[2], d[3], d[4], {}};
+        return first_order({d[0], d[1], d[2], d[3], d[4], {}}, kept, grads);
     }
 };
 

@@ -444,7 +444,7 @@ struct RmsSite : Function<RmsSite> {
         const Tensors kept = ctx->get_saved_variables();
         Tensors d = taken(rms_backward(prepared(grads[0], kept[1]), kept[0], kept[1], kept[2], ctx->saved_data["cols"].toInt(),
                                   ctx->saved_data["strided"].toBool()), "rms_backward");
-        return {d[0], d[1], {}, {}, {}};
+        return first_order({d[0], d[1], {}, {}, {}}, kept, grads);
     }
 };
 
@@ -467,7 +467,7 @@ struct QkvSite : Function<QkvSite> {
         if (kept.size() > 3) cos = kept[3], sin = kept[4];
         Tensors d = taken(qkv_backward(grads[0], grads[1], grads[2], kept[0], kept[1], kept[2], ctx->saved_data["epsilon"].toDouble(),
                                   cos, sin), "qkv_backward");
-        return {d[0], d[1], d[2], {}, {}, {}};
+        return first_order({d[0], d[1], d[2], {}, {}, {}}, kept, grads);
     }
 };
 

@@ -85,6 +85,31 @@ inline bool ordinary_call(std::initializer_list<const at::Tensor *> operands) {
     return true;
 }
 
+// Under create_graph the engine runs a node's backward with grad mode on and takes gradients that carry no graph for
+// constants: a second derivative would lose their part without a word.  They leave with a graph that refuses instead.
+constexpr const char *kFirstOrderOnly =
+    "the fused norms have no second derivative: a gradient of theirs taken with create_graph=True cannot be differentiated again";
+
+struct FirstOrderOnly : torch::autograd::Function<FirstOrderOnly> {
+    static at::Tensor forward(torch::autograd::AutogradContext *, const at::Tensor &grad, at::TensorList) {
+        return grad.tensor_data();
+    }
+    static std::vector<at::Tensor> backward(torch::autograd::AutogradContext *, std::vector<at::Tensor>) {
+        TORCH_CHECK(false, kFirstOrderOnly);
+    }
+};
+
+// kept, incoming: what the gradients were computed from, so that asking for a derivative by any of it meets the refusal.
+inline std::vector<at::Tensor> first_order(std::vector<at::Tensor> grads, const std::vector<at::Tensor> &kept,
+                                           const std::vector<at::Tensor> &incoming) {
+    if (!at::GradMode::is_enabled()) return grads;
+    std::vector<at::Tensor> from = kept;
+    from.insert(from.end(), incoming.begin(), incoming.end());
+    for (at::Tensor &g : grads)
+        if (g.defined()) g = FirstOrderOnly::apply(g.detach().requires_grad_(true), at::TensorList(from));
+    return grads;
+}
+
 // A gradient as the kernels take it: the saved tensor's dtype, contiguous, 16-byte aligned.
 inline at::Tensor prepared(const at::Tensor &g, const at::Tensor &like) {
     if (!g.defined() || ready(g, like)) return g;

@@ -27,6 +27,7 @@ What differs from the reference, on purpose:
 """
 from __future__ import annotations
 
+import functools
 import logging
 import os
 from typing import Optional, Tuple
@@ -126,6 +127,32 @@ def _native(site, *args):
     return site(*args)
 
 
+class _FirstOrderOnly(Function):
+    @staticmethod
+    def forward(ctx, grad, *computed_from):
+        return grad.data
+
+    @staticmethod
+    def backward(ctx, grad):
+        raise RuntimeError("the fused norms have no second derivative: a gradient of theirs taken with create_graph=True "
+                           "cannot be differentiated again")
+
+
+def _first_order(backward):
+    """A backward whose gradients refuse a second differentiation.  Under create_graph autograd takes gradients that carry
+    no graph for constants, and a second derivative would lose their part without a word.  A gradient handed on as it
+    came stays differentiable."""
+    @functools.wraps(backward)
+    def guarded(ctx, *grads):
+        result = backward(ctx, *grads)
+        if not torch.is_grad_enabled():
+            return result
+        computed_from = (*ctx.saved_tensors, *grads)   # asking for a derivative by any of it meets the refusal
+        return tuple(r if r is None or any(r is g for g in grads) else
+                     _FirstOrderOnly.apply(r.detach().requires_grad_(True), *computed_from) for r in result)
+    return guarded
+
+
 class FP32LayerNorm(nn.LayerNorm):
     """LayerNorm evaluated in fp32 and cast back (dit_fusedlayers.py:48-57)."""
 
@@ -197,6 +224,7 @@ class AdaLNModelFunction(Function):
         return out
 
     @staticmethod
+    @_first_order
     def backward(ctx, grad_output):
         x, scale_c, mean, invvar = ctx.saved_tensors
         done = fused_adaln.adaln_backward(grad_output, None, x, scale_c, mean, invvar, ctx.cols, ctx.seq_first)
@@ -263,6 +291,7 @@ class AdaLNResidualFunction(Function):
         return x, out
 
     @staticmethod
+    @_first_order
     def backward(ctx, grad_x_same, grad_out):
         x, scale_c, mean, invvar = ctx.saved_tensors
         if grad_out is None:   # only the stream was used: the Function was an identity
@@ -369,6 +398,7 @@ class GatedResidualAdaLNFunction(Function):
         return h2, out
 
     @staticmethod
+    @_first_order
     def backward(ctx, grad_h2, grad_out):
         h2, attn_c, gate_c, scale_c, mean, invvar = ctx.saved_tensors
         if grad_out is None:
@@ -570,6 +600,7 @@ class RMSNormModelFunction(Function):
         return out
 
     @staticmethod
+    @_first_order
     def backward(ctx, grad_output):
         x, w, invvar = ctx.saved_tensors
         done = fused_rmsnorm.rms_backward(grad_output, x, w, invvar, ctx.cols, ctx.strided)
@@ -692,6 +723,7 @@ class QKVSplitNormFunction(Function):
         return outs[0], outs[1], v_out
 
     @staticmethod
+    @_first_order
     def backward(ctx, grad_q, grad_k, grad_v):
         if ctx.joint:
             mixed, wq, wk, *tables = ctx.saved_tensors

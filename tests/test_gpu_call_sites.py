@@ -217,6 +217,35 @@ def test_scale_and_shift_of_unlike_shapes(FL, gpu_device, kind, scale, shift, ho
         assert all(torch.equal(g.reshape(w.shape).to(w.dtype), w) for g, w in zip(got, want))
 
 
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_second_derivative_is_refused(FL, gpu_device, kind):
+    """Under create_graph the gradients are the same; a loss that mixes them with other terms is not differentiated without
+    them in silence."""
+    args, grads, site, function = _case(FL, kind, torch.bfloat16, gpu_device)
+    want = _both(function, args, grads)[1]
+    for call in (site, function):
+        leaves = _leaves(args)
+        outs = _tuple(call(*leaves))
+        got = torch.autograd.grad(outs, leaves, grads, create_graph=True)
+        assert _same([g.detach() for g in got], want[len(outs):]) and all(g.requires_grad for g in got)
+        assert [g.stride() for g in got] == [g.stride() for g in want[len(outs):]]
+        for g in got:
+            with pytest.raises(RuntimeError, match="no second derivative"):
+                torch.autograd.grad(g.float().sum() + leaves[0].float().pow(2).sum(), leaves[0], retain_graph=True)
+        # operands that were copied first have no path to the copy; backward() refuses all the same
+        leaves = _leaves(args)
+        rows = torch.empty(args[0].numel() + 1, dtype=args[0].dtype, device=gpu_device)[1:].view(args[0].shape).copy_(leaves[0])
+        got = torch.autograd.grad(_tuple(call(rows, *leaves[1:])), leaves, grads, create_graph=True)
+        with pytest.raises(RuntimeError, match="no second derivative"):
+            (got[0].float().sum() + leaves[0].float().pow(2).sum()).backward()
+        if kind == "stream":   # the stream alone is an identity, differentiable as often as one likes
+            leaves = _leaves(args)
+            out = call(*leaves)[0]
+            first, = torch.autograd.grad(out.float().pow(3).sum(), leaves[0], create_graph=True)
+            second, = torch.autograd.grad(first.float().sum(), leaves[0])
+            torch.testing.assert_close(second.float(), 6 * args[0].float(), rtol=2.0 ** -6, atol=0)
+
+
 def test_another_stream_and_several_threads(FL, gpu_device):
     args, grads, site, function = _case(FL, "gated", torch.bfloat16, gpu_device)
     want = _both(function, args, grads)[1]
