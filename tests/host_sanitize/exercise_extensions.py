@@ -58,7 +58,11 @@ def main(directory):
         assert rms.qkv_forward(torch.zeros(1, 2, 3, 384, dtype=bf), v, w, 1e-6, v, v) is None
         assert ada.adaln_forward(v, s, s, 3072, 1e-6, False) is None and ada.adaln_forward(h, v, v, 0, 1e-6, True) is None
         assert ada.gated_forward(v, h, s, s, s, 1e-6) is None and ada.gated_forward(h, h, v, v, v, 1e-6) is None
-        n += 8
+        assert rms.rms_site(v, w, 128, 1e-6) is None and rms.qkv_site(v, w, w, 1e-6, None, None) is None
+        assert rms.qkv_site(torch.zeros(1, 2, 3, 384, dtype=bf), v, w, 1e-6, v, v) is None
+        assert ada.adaln_site(v, s, s, 3072, 1e-6, False) is None and ada.adaln_site(h, v, v, 0, 1e-6, True) is None
+        assert ada.adaln_residual_site(v, s, s, 1e-6) is None and ada.gated_residual_site(v, h, s, s, s, 1e-6) is None
+        n += 15
     assert rms.supported(128, x) and rms.supported(3072, torch.zeros(1)) and not rms.supported(3071, x)
     assert not rms.supported(128, torch.zeros(1, dtype=torch.int32))
     print(f"sanitised extensions ok: {n} refused calls")

@@ -5,6 +5,7 @@ import threading
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 from torch.utils.checkpoint import checkpoint
 
 pytestmark = pytest.mark.gpu
@@ -128,7 +129,16 @@ def test_hooks_repeats_and_checkpoints(FL, gpu_device, kind):
     packed = []
     with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.to(gpu_device)):
         got = _both(site, args, grads)[1]
-    assert packed and (_same(got, want) if kind not in ("view", "view3") else _same(got[:2], want[:2]))
+    if kind in ("view", "view3"):
+        # the view comes back dense, its rows in another order: each sum of n terms is off by at most n 2^-24 of their
+        # magnitudes (|xhat| <= sqrt(80)), and is rounded to bf16 once
+        per_column = grads[0].float().abs().sum(tuple(range(grads[0].dim() - 1)))
+        slack = 2 * (grads[0].numel() // 80) * 2.0 ** -24 * per_column * 80 ** 0.5
+        apart = (got[2].float() - want[2].float()).abs()
+        assert bool((apart <= slack + 2.0 ** -7 * want[2].float().abs()).all())
+        got, want = got[:2], want[:2] + want[3:]
+    assert packed and len(got) == len(want) and _same(got, want)
+    want = _both(function, args, grads)[1]
     leaves = _leaves(args)
     outs = _tuple(site(*leaves))
     first = torch.autograd.grad(outs, leaves, grads, retain_graph=True)
@@ -165,7 +175,23 @@ def test_transforms_and_tangents_do_what_the_python_function_does(FL, gpu_device
         except Exception as exc:
             return type(exc).__name__, str(exc)[:60]
 
-    for run in (lambda c: torch.func.vmap(c)(args[0].unsqueeze(0)), lambda c: torch.func.vjp(c, args[0])[0], tangent):
+    def batched(call):
+        leaf = args[0].clone().requires_grad_(True)
+        outs = _tuple(call(leaf))
+        return torch.autograd.grad(outs, leaf, [torch.stack([g, g]) for g in grads], is_grads_batched=True)
+
+    fixed = [torch.nn.Parameter(a.clone(), requires_grad=False) if a.dim() == 1 else a.clone() for a in args[1:]]
+
+    def traced(call):   # operands that need a gradient cannot become constants of a trace
+        rest[:] = fixed
+        return torch.jit.trace(lambda t: call(t), (args[0],), check_trace=False)(args[0])
+
+    def recorded(call):
+        rest[:] = fixed
+        return make_fx(lambda t: call(t))(args[0])(args[0])
+
+    for run in (lambda c: torch.func.vmap(c)(args[0].unsqueeze(0)), lambda c: torch.func.vjp(c, args[0])[0], tangent, batched,
+                traced, recorded):
         a, b = outcome(run, site), outcome(run, function)
         assert a[0] == b[0], (a, b)
         assert _same(a[1], b[1]) if a[0] == "ran" else a[1] == b[1], (a, b)
