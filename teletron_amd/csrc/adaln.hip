@@ -41,11 +41,11 @@
 // one-shot workgroups a compute unit holds at once; the kernel does not touch it.
 // With its row requested before the parameters are staged, a two-byte workgroup streams best four to a compute unit
 // while the grid is short (16 KiB on top of its 24 KiB: 14 850 rows 34.0 us against 34.3 with six and 34.5 with three,
-// 4000 rows 10.0 / 10.1 / 11.9) and three once it refills every compute unit many times (24 KiB: 118 800 rows 240.5 us
-// against 244.6 with four and 250.7 with six; 80 000 rows 165 either way).  The gated form runs unthrottled, by its registers and
-// LDS, on short grids (4000 rows 20.9 us, 22.2 with 12 KiB more; 60 000 rows 244.7 / 248.2).  On long ones it takes the
-// 12 KiB: between backward launches 118 800 rows take 482 us, 490 without (on its own 492 / 488).  4-byte rows carry twice the bytes per
-// wavefront: 40 KiB on top of the staged modulation rows leaves two workgroups per compute unit (59 400 rows 243 us, 260
+// 4000 rows 10.0 / 10.1 / 11.9) and three once it refills every compute unit many times (24 KiB: 118 800 rows 241 us
+// against 246 with four and 251 with six, launched on its own; 80 000 rows 165 with either).  The gated form runs unthrottled, by
+// its registers and LDS, on short grids (4000 rows 20.6 us, 22.1 with 12 KiB more; 60 000 rows 246 either way).  On long ones it takes
+// the 12 KiB: between backward launches 118 800 rows take 482 us, 490 without (on its own 499 / 492).  4-byte rows carry twice the
+// bytes per wavefront: 40 KiB on top of the staged modulation rows leaves two workgroups per compute unit (59 400 rows 243 us, 260
 // with three); gated, 16 KiB leave three (8192 rows 70.2 us, 72.9 with two).
 #ifndef TTN_ADALN_FWD_DYN_LDS
 #define TTN_ADALN_FWD_DYN_LDS                                                                        \
@@ -126,7 +126,8 @@ __global__ __launch_bounds__(kRowThreads) TTN_MIN_WAVES_PER_SIMD(sizeof(T) == 2 
     __shared__ u32x4 lds_t[kPlanes][kPieces], lds_h[kPlanes][kPieces], lds_g[GATED ? kPieces : 1];
     // The modulation row is requested first and the wavefront's row right behind it, before the staging waits for the
     // former: a workgroup of the one-shot grid then spends one memory latency less (4000 x 3072 bf16 11.1 -> 10.7 us, 29 700 64.9 -> 63.4,
-    // 118 800 245 -> 241; gated fp32 8192 rows 74.4 -> 70.2, bf16 4000 rows 22.0 -> 20.9; 1500 rows 6.4 -> 6.5).
+    // 118 800 242 -> 240 launched on its own, 235-236 inside a step either way; gated fp32 8192 rows 74.8 -> 70.1, bf16 4000 rows
+    // 22.1 -> 20.6; 1500 rows 6.3 -> 6.5).
     constexpr int kShare = (kPieces + kRowThreads - 1) / kRowThreads;  // pieces of a parameter row per thread
     u32x4 ps[kShare], ph[kShare];
     [[maybe_unused]] u32x4 pg[GATED ? kShare : 1];

@@ -890,7 +890,8 @@ int widerow_rmsnorm_backward(void *dx, void *dw, const void *g, const void *x, c
 // plain two-byte form at a time (3000 x 4096 bf16 12.5 us, 13.5 with two) and two of the forms that
 // move twice the bytes per column (gated 60 000 x 4096 bf16 345 us with four, 329 with two; 50 000 x 2048 fp32 142 / 139).
 // A grid that would leave compute units idle takes fewer: one row up to four workgroups per compute unit (100 x 4096 6.7 ->
-// 3.9 us, 1000 x 4096 7.8 -> 6.5, gated 700 x 4096 10.1 -> 7.9), two up to ten (1300 x 4096 9.1 -> 7.9, 2500 x 4096 12.0 -> 10.9).
+// 3.9 us, 1000 x 4096 7.8 -> 6.5, gated 700 x 4096 10.1 -> 7.9), two up to ten (1300 x 4096 9.1 -> 8.0, 2500 x 4096 12.2 -> 10.9).
+// Where four rows make just one full wave of workgroups, two lose: 4000 x 2048 fp32 14.8 -> 15.1.
 static int wide_adaln_fwd_rows(int64_t rows, int cus, bool plain_two_byte) {
     if (rows <= 4 * (int64_t)cus) return 1;
     return plain_two_byte && rows > 10 * (int64_t)cus ? 4 : 2;
