@@ -104,7 +104,8 @@ inline std::vector<at::Tensor> first_order(std::vector<at::Tensor> grads, const 
                                            const std::vector<at::Tensor> &incoming) {
     if (!at::GradMode::is_enabled()) return grads;
     std::vector<at::Tensor> from = kept;
-    from.insert(from.end(), incoming.begin(), incoming.end());
+    for (const at::Tensor &g : incoming)
+        if (g.defined()) from.push_back(g);
     for (at::Tensor &g : grads)
         if (g.defined()) g = FirstOrderOnly::apply(g.detach().requires_grad_(true), at::TensorList(from));
     return grads;

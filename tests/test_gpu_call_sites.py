@@ -258,6 +258,14 @@ def test_a_second_derivative_is_refused(FL, gpu_device, kind):
         for g in got:
             with pytest.raises(RuntimeError, match="no second derivative"):
                 torch.autograd.grad(g.float().sum() + leaves[0].float().pow(2).sum(), leaves[0], retain_graph=True)
+        for i in range(len(grads) if len(grads) > 1 else 0):   # one output used, the others' gradients missing
+            if kind == "stream" and i == 0:
+                continue
+            leaves = _leaves(args)
+            some = torch.autograd.grad(_tuple(call(*leaves))[i], leaves, grads[i], create_graph=True, allow_unused=True)
+            assert _same([g if g is None else g.detach() for g in some], _both(function, args, grads, [i])[1][len(outs):])
+            with pytest.raises(RuntimeError, match="no second derivative"):
+                torch.autograd.grad(some[0].float().sum() + leaves[0].float().pow(2).sum(), leaves[0])
         # operands that were copied first have no path to the copy; backward() refuses all the same
         leaves = _leaves(args)
         rows = torch.empty(args[0].numel() + 1, dtype=args[0].dtype, device=gpu_device)[1:].view(args[0].shape).copy_(leaves[0])
